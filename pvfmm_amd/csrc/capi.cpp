@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <string>
@@ -56,6 +57,17 @@ struct FmmHandle {
   Operators O;
   int precision = 0;
   std::mutex bc_mutex;  // the boundary operators are built on first use, by any tree set up with this handle
+  // the operators on each device that a tree was set up on with this handle (precision `precision`)
+  std::mutex ops_mutex;
+  std::map<int, std::shared_ptr<DeviceOpsBase>> ops;
+  std::shared_ptr<DeviceOpsBase> device_ops() {
+    int dev = 0;
+    HIP_CHECK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lock(ops_mutex);
+    std::shared_ptr<DeviceOpsBase>& o = ops[dev];
+    if (!o) o = make_device_ops(O, precision);
+    return o;
+  }
 };
 
 struct DeviceArray {
@@ -111,7 +123,8 @@ void setup_tree(TreeHandle* t, FmmHandle* f, int n_vec_max) {
     std::lock_guard<std::mutex> lock(f->bc_mutex);
     build_bc_operator(f->O, t->T.bndry);
   }
-  t->plan = make_plan(t->T, f->O, t->src.data(), t->trg.data(), f->precision, n_vec_max, t->stream);
+  t->plan = make_plan(t->T, f->O, t->src.data(), t->trg.data(), f->precision, n_vec_max, t->stream,
+                      f->device_ops());
 }
 
 void eval_device(TreeHandle* t, const double* d_den, double* d_out, int n_vec, double den_scale, double out_scale) {
@@ -352,6 +365,7 @@ void context_eval(Context* c, const Real* src_pos, const Real* sl_den, const Rea
                             c->box_size > 0 ? kPXYZ : kFreeSpace));
     if (c->fmm->precision != c->precision) {
       // the pseudo-inverse truncation depends on the evaluation precision
+      c->fmm->ops.clear();  // made from the operators replaced here
       build_operators_cached(c->fmm->O, c->kernel, c->m, 0.0, c->precision, std::getenv("PVFMM_DIR"));
       c->fmm->precision = c->precision;
     }
@@ -651,6 +665,13 @@ int64_t pvfmm_amd_fmm_operator(void* fmm, int which, double* out) {
       return -1;
     if (out) std::copy(f->O.bc[which - 6].begin(), f->O.bc[which - 6].end(), out);
     return n;
+  }
+  if (which == 6) {  // the M2L blocks, computed on first request
+    if (guarded([&] {
+          std::lock_guard<std::mutex> lock(f->bc_mutex);
+          ensure_v1(f->O);
+        }) != 0)
+      return -1;
   }
   const Operators& O = f->O;
   const std::vector<double>* v = nullptr;

@@ -10,6 +10,7 @@
 #include <string>
 #include <unordered_map>
 
+#include "device_ops.hpp"
 #include "kernels.hpp"
 
 namespace pvfmm_amd {
@@ -29,63 +30,6 @@ const char* phase_name(int p) {
 }
 
 namespace {
-
-template <typename T>
-struct DBuf {
-  T* p = nullptr;
-  int64_t n = 0;
-  DBuf() = default;
-  DBuf(const DBuf&) = delete;
-  DBuf& operator=(const DBuf&) = delete;
-  ~DBuf() { if (p) (void)hipFree(p); }
-  void alloc(int64_t count, int64_t* total) {
-    if (p) { (void)hipFree(p); p = nullptr; }
-    n = count;
-    if (count > 0) {
-      HIP_CHECK(hipMalloc(&p, sizeof(T) * count));
-      if (total) *total += sizeof(T) * count;
-    }
-  }
-  void upload(const std::vector<T>& v, int64_t* total) {
-    alloc((int64_t)v.size(), total);
-    if (!v.empty()) HIP_CHECK(hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
-  }
-};
-
-// U2U and D2D through the rank of the check-to-equivalent factors.  The composite translations
-// are u2u = T uc2ue1 (T: 8 K0 x r, uc2ue1: r x K0 with orthonormal rows) and d2d = dc2de0 B
-// (dc2de0: K1 x r with orthogonal columns of norms 1/s_j, B: r x 8 K1), so T = u2u uc2ue1^T and
-// B = diag(s^2) dc2de0^T d2d (include/fmm_pts.txx:582-643 forms the same products).  Applied as
-// two GEMMs they cost 9 K r instead of 8 K^2 multiply-adds per row; the results are returned in
-// the padded layouts of the plan (r -> rp columns of T, rows of B, zero-filled).
-static std::vector<double> u2u_rank_factor(const Operators& O, int rp) {
-  const int K0 = O.K0(), r = O.rank_u;
-  std::vector<double> T((size_t)8 * K0 * rp, 0.0);
-  #pragma omp parallel for schedule(static)
-  for (int i = 0; i < 8 * K0; i++)
-    for (int j = 0; j < r; j++) {
-      double acc = 0;
-      for (int k = 0; k < K0; k++) acc += O.u2u[(size_t)i * K0 + k] * O.uc2ue1[(size_t)j * K0 + k];
-      T[(size_t)i * rp + j] = acc;
-    }
-  return T;
-}
-static std::vector<double> d2d_rank_factor(const Operators& O, int rp) {
-  const int K1 = O.K1(), r = O.rank_d;
-  std::vector<double> B((size_t)rp * 8 * K1, 0.0);
-  #pragma omp parallel for schedule(static)
-  for (int j = 0; j < r; j++) {
-    double n2 = 0;
-    for (int i = 0; i < K1; i++) n2 += O.dc2de0[(size_t)i * r + j] * O.dc2de0[(size_t)i * r + j];
-    double* b = &B[(size_t)j * 8 * K1];
-    for (int i = 0; i < K1; i++) {
-      const double c = O.dc2de0[(size_t)i * r + j] / n2;
-      const double* d = &O.d2d[(size_t)i * 8 * K1];
-      for (int n = 0; n < 8 * K1; n++) b[n] += c * d[n];
-    }
-  }
-  return B;
-}
 
 // LDS pool slots of the V-list tiles' staged partners for the bf16 kernel (FP32 scalar
 // kernels), which keeps one pool of `pool` staged entries across the run of tiles a block
@@ -188,8 +132,9 @@ static void assign_pool_slots(int n_off, int pool, int n_s, const std::vector<in
 template <typename Real>
 class DevicePlan final : public DevicePlanBase {
  public:
-  DevicePlan(const Octree& T, const Operators& O, const double* src_xyz, const double* trg_xyz, int n_vec, hipStream_t s)
-      : O_(O), st_(s) {
+  DevicePlan(const Octree& T, const Operators& O, std::shared_ptr<DeviceOps<Real>> ops, const double* src_xyz,
+             const double* trg_xyz, int n_vec, hipStream_t s)
+      : O_(O), ops_(std::move(ops)), st_(s) {
     n_vec_max = std::max(1, n_vec);
     build(T, src_xyz, trg_xyz);
   }
@@ -251,13 +196,14 @@ class DevicePlan final : public DevicePlanBase {
  private:
   using K = DeviceKernels<Real>;
   const Operators& O_;
+  std::shared_ptr<DeviceOps<Real>> ops_;  // the operators on the device, shared with other trees
   hipStream_t st_;
   int64_t n_src_ = 0, n_trg_ = 0;
   int k0_ = 1, k1_ = 1, e0_ = 1, e1_ = 1, K0_ = 0, K1_ = 0, ns_ = 0, m_ = 0, M_dim_ = 0;
   int n_nodes_ = 0, max_depth_ = 0;
   int bndry_ = 0;     // boundary type of the tree (0 free space, 1-3 periodic)
+  const Real* bc_ = nullptr;  // periodic boundary operator (K0_ x K1_)
   bool vol_ = false;  // PXYZ with a kernel carrying the analytic volume potential
-  DBuf<Real> bc_;     // periodic boundary operator (K0_ x K1_)
   DBuf<double> txa_;  // target coordinates in sorted order (SoA), for the volume-potential correction
 
   // tree arrays (periodic trees append virtual image nodes: a source node's point range and size
@@ -271,28 +217,21 @@ class DevicePlan final : public DevicePlanBase {
   DBuf<double> tval_;
   // expansions: eq_ = [up (n_nodes x K0) | L2T equivalent rows (n_l2t x K0)]
   DBuf<Real> eq_, dn_, chk_;
-  // operators
-  DBuf<Real> uc2ue0_, uc2ue1_, dc2de0_, dc2de1_, u2u_, d2d_, V_, unit_surf_, ctmp_;
-  // U2U / D2D through the check-to-equivalent rank (u2u_rank_factor, d2d_rank_factor) when
-  // 9 r < 8 K, at levels of at least kFactorRows parents (a smaller level costs less as one
-  // GEMM than as two launches): u2ur_ 8 K0 x ru_, d2dr_ rd_ x 8 K1; lvl_seq_ = 0, 1, ... (rows
-  // of ctmp_)
+  DBuf<Real> ctmp_;
+  // U2U / D2D through the check-to-equivalent rank (DeviceOps::u2ur, d2dr) at levels of at least
+  // kFactorRows parents (a smaller level costs less as one GEMM than as two launches);
+  // lvl_seq_ = 0, 1, ... (rows of ctmp_)
   static constexpr int kFactorRows = 256;
-  bool u2u_fact_ = false, d2d_fact_ = false;
-  DBuf<Real> u2ur_, d2dr_;
   DBuf<int32_t> lvl_seq_;
-  DBuf<uint16_t> Vb_;  // transfer blocks as bf16 parts (FP32 scalar kernels, 16-vector passes)
-  // the fp16 form of the FP32 scalar Hadamard: transfer parts, 1 / tau_f, the spectrum bound of
-  // each slot of X (or, in the adjoint, of Y) and the scale of each run of tiles
-  DBuf<uint16_t> Vh_;
-  DBuf<float> vtinv_, vbound_, vrscale_;
+  // the fp16 Hadamard kernels (FP32): the spectrum bound of each slot of X (or, in the adjoint,
+  // of Y) and the scale of each run of tiles
+  DBuf<float> vbound_, vrscale_;
   bool split_ = false;
   DBuf<Real> gemm_work_;  // split-K partial tiles of the small coarse-level GEMMs
   int64_t gemm_work_elems_ = 0;
   int nvb_ = 1;  // density vectors per evaluation pass (buffers hold this many)
   int64_t eq_vs_ = 0, dn_vs_ = 0, chk_vs_ = 0, ctmp_vs_ = 0;  // per-vector strides  // room for 4 K-split partials of the largest GEMM output, at most 2^25
   int ru_ = 0, rd_ = 0;
-  DBuf<int32_t> lattice_, lattice_inv_;
   // S2M
   DBuf<int32_t> s2m_node_, s2m_ptr_, s2m_items_, s2m_orow_;
   DBuf<Real> s2m_alpha_;
@@ -326,8 +265,8 @@ class DevicePlan final : public DevicePlanBase {
   // operands of the fp16 Hadamard with run scales in `rs` (kept until the launch returns)
   HadamardParts hp_;
   const HadamardParts& hparts(DBuf<float>& rs) {
-    hp_.Vh = Vh_.p;
-    hp_.tinv = vtinv_.p;
+    hp_.Vh = ops_->Vh.p;
+    hp_.tinv = ops_->vtinv.p;
     hp_.bound = vbound_.p;
     hp_.run_scale = rs.p;
     hp_.run_scale_cap = (int)rs.n;
@@ -466,10 +405,10 @@ class DevicePlan final : public DevicePlanBase {
   }
 
   void build(const Octree& T, const double* src_xyz, const double* trg_xyz) {
-    int64_t total = 0;
+    int64_t total = ops_->bytes();
     const KernelInfo& ki = O_.ker;
     k0_ = ki.k0; k1_ = ki.k1; e0_ = ki.e0; e1_ = ki.e1;
-    ns_ = O_.ns; m_ = O_.m; K0_ = O_.K0(); K1_ = O_.K1(); M_dim_ = O_.M_dim;
+    ns_ = O_.ns; m_ = O_.m; K0_ = O_.K0(); K1_ = O_.K1(); M_dim_ = ops_->grid.M;
     n_src_ = T.src.n; n_trg_ = T.trg.n;
     n_nodes_ = T.n_nodes();
     max_depth_ = T.max_depth;
@@ -554,189 +493,9 @@ class DevicePlan final : public DevicePlanBase {
     sden_.alloc((int64_t)k0_ * n_src_ * nvb_, &total);
     tval_.alloc((int64_t)k1_ * n_trg_ * nvb_, &total);
 
-    // ---- operators in the working precision
-    auto conv = [](const std::vector<double>& v) { return std::vector<Real>(v.begin(), v.end()); };
-    // check -> equivalent factors with the rank padded to a multiple of 16 (zero columns of
-    // the first factor, zero rows of the second), so the GEMM operands stay 4-vector aligned
-    ru_ = (O_.rank_u + 15) / 16 * 16;
-    rd_ = (O_.rank_d + 15) / 16 * 16;
-    auto pad_cols = [&](const std::vector<double>& m, int rows, int r, int rp) {
-      std::vector<Real> out((size_t)rows * rp, Real(0));
-      for (int i = 0; i < rows; i++)
-        for (int j = 0; j < r; j++) out[(size_t)i * rp + j] = (Real)m[(size_t)i * r + j];
-      return out;
-    };
-    auto pad_rows = [&](const std::vector<double>& m, int r, int cols, int rp) {
-      std::vector<Real> out((size_t)rp * cols, Real(0));
-      for (int i = 0; i < r; i++)
-        for (int j = 0; j < cols; j++) out[(size_t)i * cols + j] = (Real)m[(size_t)i * cols + j];
-      return out;
-    };
-    uc2ue0_.upload(pad_cols(O_.uc2ue0, K1_, O_.rank_u, ru_), &total);
-    uc2ue1_.upload(pad_rows(O_.uc2ue1, O_.rank_u, K0_, ru_), &total);
-    dc2de0_.upload(pad_cols(O_.dc2de0, K1_, O_.rank_d, rd_), &total);
-    dc2de1_.upload(pad_rows(O_.dc2de1, O_.rank_d, K0_, rd_), &total);
-    u2u_fact_ = 9 * ru_ < 8 * K0_;
-    d2d_fact_ = 9 * rd_ < 8 * K1_;
-    if (u2u_fact_) u2ur_.upload(conv(u2u_rank_factor(O_, ru_)), &total);
-    if (d2d_fact_) d2dr_.upload(conv(d2d_rank_factor(O_, rd_)), &total);
-    u2u_.upload(conv(O_.u2u), &total);
-    d2d_.upload(conv(O_.d2d), &total);
-    {
-      // Transfer blocks in real form for y = x B with x, y interleaved (re, im):
-      //   B[2s][2t] = Re M[t][s], B[2s+1][2t] = -Im M[t][s], B[2s][2t+1] = Im M[t][s],
-      //   B[2s+1][2t+1] = Re M[t][s],
-      // stored per MFMA lane: [R][f][kb][nb][lane][q] = B[16kb + 4(lane/16) + q][16nb + lane%16].
-      // Spectrum rows are component-major (the DFTs write and read them so): row position k of
-      // an input spectrum holds component k / 16 of child (k % 16) / 2, which is complex source
-      // index s_of(k) of M (child-major: s = child * E0 + component), and output position n is
-      // complex target index t_of(n).
-      const int E0 = e0_, E1 = e1_, NS = 8 * E0, NR = 8 * E1;
-      auto s_of = [E0](int k) { return ((k & 15) >> 1) * E0 + (k >> 4); };
-      auto t_of = [E1](int n) { return ((n & 15) >> 1) * E1 + (n >> 4); };
-      // the FP32 kernels use the fp16 (and, scalar, bf16) parts below instead
-      const bool bf16_parts = std::is_same<Real, float>::value && E0 == 1 && E1 == 1;
-      const bool stokes_parts = std::is_same<Real, float>::value && E0 == 3 && E1 == 3;
-      const bool real_form = !bf16_parts && !stokes_parts;
-      std::vector<Real> Vp(real_form ? (size_t)27 * M_dim_ * E0 * E1 * 256 : 0, (Real)0);
-      #pragma omp parallel for schedule(static)
-      for (int64_t rf = 0; rf < (real_form ? (int64_t)27 * M_dim_ : 0); rf++) {
-        const std::complex<double>* Mb = &O_.v1[(size_t)rf * NR * NS];  // [t][s]
-        for (int kb = 0; kb < E0; kb++)
-          for (int nb = 0; nb < E1; nb++)
-            for (int l = 0; l < 64; l++)
-              for (int q = 0; q < 4; q++) {
-                const int k = 16 * kb + 4 * (l >> 4) + q, n = 16 * nb + (l & 15);
-                const std::complex<double> v = Mb[(size_t)t_of(n) * NS + s_of(k)];
-                double val = ((k & 1) == 0) ? ((n & 1) == 0 ? v.real() : v.imag()) : ((n & 1) == 0 ? -v.imag() : v.real());
-                Vp[((((size_t)rf * E0 + kb) * E1 + nb) * 64 + l) * 4 + q] = (Real)val;
-              }
-      }
-      V_.upload(Vp, &total);
-      if (bf16_parts) {
-        // the same blocks as three bf16 parts for the matrix-core kernel, offsets taken in
-        // pairs in the order of v1_offsets: [pair j][part p][f][lane][i] = part p of
-        // B_{2j + lane/32}[8 ((lane/16) % 2) + i][lane % 16]; each part rounds the remainder of
-        // the FP64 value to nearest
-        auto bf16_rn = [](float x) {
-          uint32_t u;
-          std::memcpy(&u, &x, 4);
-          u += 0x7FFFu + ((u >> 16) & 1u);
-          return (uint16_t)(u >> 16);
-        };
-        auto bf16_val = [](uint16_t h) {
-          const uint32_t u = (uint32_t)h << 16;
-          float x;
-          std::memcpy(&x, &u, 4);
-          return (double)x;
-        };
-        const int n_pair = (int)O_.v1_offsets.size() / 2;
-        std::vector<uint16_t> Vb((size_t)n_pair * 3 * M_dim_ * 64 * 8);
-        #pragma omp parallel for schedule(static)
-        for (int64_t jf = 0; jf < (int64_t)n_pair * M_dim_; jf++) {
-          const int j = (int)(jf / M_dim_), f = (int)(jf % M_dim_);
-          for (int l = 0; l < 64; l++) {
-            const int R = O_.v1_offsets[2 * j + (l >> 5)];
-            const std::complex<double>* Mb = &O_.v1[((size_t)R * M_dim_ + f) * NR * NS];
-            for (int i = 0; i < 8; i++) {
-              const int k = 8 * ((l >> 4) & 1) + i, n = l & 15;
-              const std::complex<double> v = Mb[(size_t)(n >> 1) * NS + (k >> 1)];
-              double r = ((k & 1) == 0) ? ((n & 1) == 0 ? v.real() : v.imag()) : ((n & 1) == 0 ? -v.imag() : v.real());
-              for (int p = 0; p < 3; p++) {
-                const uint16_t h = bf16_rn((float)r);
-                Vb[((((size_t)j * 3 + p) * M_dim_ + f) * 64 + l) * 8 + i] = h;
-                r -= bf16_val(h);
-              }
-            }
-          }
-        }
-        Vb_.upload(Vb, &total);
-        // two fp16 parts of tau_f B for k_hadamard_split: tau_f = 2^(14 - e) with every entry
-        // of frequency f's blocks below 2^e (so below 2^14 after scaling); part 0 rounds tau_f t
-        // to nearest, part 1 the remainder
-        std::vector<uint16_t> Vh((size_t)n_pair * 2 * M_dim_ * 64 * 8);
-        std::vector<float> tinv(M_dim_);
-        auto entry = [&](int j, int f, int l, int i) {
-          const int R = O_.v1_offsets[2 * j + (l >> 5)];
-          const std::complex<double> v = O_.v1[((size_t)R * M_dim_ + f) * NR * NS + (size_t)((l & 15) >> 1) * NS +
-                                               ((8 * ((l >> 4) & 1) + i) >> 1)];
-          const int k = 8 * ((l >> 4) & 1) + i, n = l & 15;
-          return ((k & 1) == 0) ? ((n & 1) == 0 ? v.real() : v.imag()) : ((n & 1) == 0 ? -v.imag() : v.real());
-        };
-        #pragma omp parallel for schedule(static)
-        for (int f = 0; f < M_dim_; f++) {
-          double mx = 0;
-          for (int j = 0; j < n_pair; j++)
-            for (int l = 0; l < 64; l++)
-              for (int i = 0; i < 8; i++) mx = std::max(mx, std::fabs(entry(j, f, l, i)));
-          int e = 0;
-          if (mx > 0) (void)std::frexp(mx, &e);
-          const double tau = mx > 0 ? std::ldexp(1.0, std::min(100, std::max(-100, 14 - e))) : 1.0;
-          tinv[f] = (float)(1.0 / tau);
-          for (int j = 0; j < n_pair; j++)
-            for (int l = 0; l < 64; l++)
-              for (int i = 0; i < 8; i++) {
-                const double x = entry(j, f, l, i) * tau;
-                const _Float16 h0 = (_Float16)x, h1 = (_Float16)(x - (double)h0);
-                std::memcpy(&Vh[((((size_t)j * 2 + 0) * M_dim_ + f) * 64 + l) * 8 + i], &h0, 2);
-                std::memcpy(&Vh[((((size_t)j * 2 + 1) * M_dim_ + f) * 64 + l) * 8 + i], &h1, 2);
-              }
-        }
-        Vh_.upload(Vh, &total);
-        vtinv_.upload(tinv, &total);
-        split_ = true;
-      }
-      if (stokes_parts) {
-        // two fp16 parts of tau_f B for k_hadamard_split3, offsets in pairs (2j, 2j+1) of
-        // v1_offsets: [f][pair j][chunk c][tile nb][part p][lane][i] = part p of
-        // B_{2j + a}[8 b + i][16 nb + lane % 16], q = 4c + lane / 16, a = q / 6, b = q % 6;
-        // tau_f = 2^(14 - e) with every entry of frequency f's blocks below 2^e
-        const int n_pair = (int)O_.v1_offsets.size() / 2;
-        const size_t per_f = (size_t)n_pair * 3 * 3 * 2 * 64 * 8;
-        std::vector<uint16_t> Vh((size_t)M_dim_ * per_f);
-        std::vector<float> tinv(M_dim_);
-        auto entry = [&](int R, int f, int k, int n) {
-          const std::complex<double> v = O_.v1[((size_t)R * M_dim_ + f) * NR * NS + (size_t)t_of(n) * NS + s_of(k)];
-          return ((k & 1) == 0) ? ((n & 1) == 0 ? v.real() : v.imag()) : ((n & 1) == 0 ? -v.imag() : v.real());
-        };
-        #pragma omp parallel for schedule(static)
-        for (int f = 0; f < M_dim_; f++) {
-          double mx = 0;
-          for (int o = 0; o < 2 * n_pair; o++)
-            for (int k = 0; k < 2 * NS; k++)
-              for (int n = 0; n < 2 * NR; n++) mx = std::max(mx, std::fabs(entry(O_.v1_offsets[o], f, k, n)));
-          int e = 0;
-          if (mx > 0) (void)std::frexp(mx, &e);
-          const double tau = mx > 0 ? std::ldexp(1.0, std::min(100, std::max(-100, 14 - e))) : 1.0;
-          tinv[f] = (float)(1.0 / tau);
-          uint16_t* out = &Vh[(size_t)f * per_f];
-          for (int j = 0; j < n_pair; j++)
-            for (int c = 0; c < 3; c++)
-              for (int nb = 0; nb < 3; nb++)
-                for (int l = 0; l < 64; l++) {
-                  const int q = 4 * c + (l >> 4), a = q / 6, b = q % 6, R = O_.v1_offsets[2 * j + a];
-                  for (int i = 0; i < 8; i++) {
-                    const double x = entry(R, f, 8 * b + i, 16 * nb + (l & 15)) * tau;
-                    const _Float16 h0 = (_Float16)x, h1 = (_Float16)(x - (double)h0);
-                    const size_t at = (((((size_t)j * 3 + c) * 3 + nb) * 2) * 64 + l) * 8 + i;
-                    std::memcpy(&out[at], &h0, 2);
-                    std::memcpy(&out[at + 64 * 8], &h1, 2);
-                  }
-                }
-        }
-        Vh_.upload(Vh, &total);
-        vtinv_.upload(tinv, &total);
-        split_ = true;
-      }
-    }
-    unit_surf_.upload(conv(O_.unit_surf), &total);
-    lattice_.upload(O_.lattice, &total);
-    {
-      std::vector<int32_t> inv((size_t)m_ * m_ * m_, -1);
-      for (int p = 0; p < ns_; p++)
-        inv[((size_t)O_.lattice[3 * p + 2] * m_ + O_.lattice[3 * p + 1]) * m_ + O_.lattice[3 * p]] = p;
-      lattice_inv_.upload(inv, &total);
-    }
+    ru_ = ops_->ru;
+    rd_ = ops_->rd;
+    split_ = ops_->split;
 
     const double ts = ki.trg_scal + ki.src_scal;
     // ---- S2M rows: leaves holding sources (Source2UpSetup, include/fmm_pts.txx:2287-2290)
@@ -945,9 +704,7 @@ class DevicePlan final : public DevicePlanBase {
     far_rad_.upload(far_rad, &total);
     u_ptr_.upload(u_ptr, &total); u_items_.upload(u_items, &total);
     if (bndry_ != kFreeSpace) {  // FMM_Pts::PeriodicBC and PostProcessing (include/fmm_pts.txx:2641-2657,5740-5774)
-      const std::vector<double>& bc = O_.bc[bndry_];
-      if (bc.size() != (size_t)K0_ * K1_) throw Error(kErrInternal, "periodic tree without its boundary operator");
-      bc_.upload(conv(bc), &total);
+      bc_ = ops_->bc(bndry_, false);
       vol_ = bndry_ == kPXYZ && ki.id != 1;
       if (vol_) {
         std::vector<double> xa(3 * (size_t)n_trg_);
@@ -994,13 +751,13 @@ class DevicePlan final : public DevicePlanBase {
   int64_t device_bytes_ = 0;
 
   struct AdjointPlan {
-    DBuf<Real> uc2ue0T, uc2ue1T, dc2de0T, dc2de1T, u2uT, d2dT, u2urT, d2drT;
+    const typename DeviceOps<Real>::Transposed* op = nullptr;  // the transposed operators
     // node table of the transposed lists: the forward one plus images of target-side nodes (a
     // forward item at shift s becomes, transposed, its target seen from the source at -s)
     DBuf<double> center;
     DBuf<float> nsz;
     DBuf<int32_t> sb, se, tb, te;
-    DBuf<Real> bcT;        // periodic boundary operator transposed (K1_ x K0_)
+    const Real* bcT = nullptr;  // periodic boundary operator transposed (K1_ x K0_)
     DBuf<double> volpart;  // per-block partial sums of the volume-potential correction's transpose
     DBuf<Real> tden;     // adjoint input gathered into target order (k1 x n_trg per vector)
     DBuf<double> sval;   // adjoint output accumulated in source order (k0 x n_src per vector)
@@ -1022,13 +779,6 @@ class DevicePlan final : public DevicePlanBase {
     int n_vt = 0;
   };
   std::unique_ptr<AdjointPlan> adj_;
-
-  static std::vector<Real> transposed(const std::vector<Real>& a, int rows, int cols) {
-    std::vector<Real> t((size_t)rows * cols);
-    for (int i = 0; i < rows; i++)
-      for (int j = 0; j < cols; j++) t[(size_t)j * rows + i] = a[(size_t)i * cols + j];
-    return t;
-  }
 
   // CSR of the transposed relation: for rows r with items it, the rows of item -> list of r
   // Groups (key, value, payload) triples by key (stable): the rows out_row (keys in increasing
@@ -1059,28 +809,7 @@ class DevicePlan final : public DevicePlanBase {
     auto a = std::make_unique<AdjointPlan>();
     int64_t total = 0;
     const int N = n_nodes_;
-    // transposed operators, in the padded layouts of the forward ones
-    auto conv = [](const std::vector<double>& v) { return std::vector<Real>(v.begin(), v.end()); };
-    auto pad_cols = [&](const std::vector<double>& m, int rows, int r, int rp) {
-      std::vector<Real> out((size_t)rows * rp, Real(0));
-      for (int i = 0; i < rows; i++)
-        for (int j = 0; j < r; j++) out[(size_t)i * rp + j] = (Real)m[(size_t)i * r + j];
-      return out;
-    };
-    auto pad_rows = [&](const std::vector<double>& m, int r, int cols, int rp) {
-      std::vector<Real> out((size_t)rp * cols, Real(0));
-      for (int i = 0; i < r; i++)
-        for (int j = 0; j < cols; j++) out[(size_t)i * cols + j] = (Real)m[(size_t)i * cols + j];
-      return out;
-    };
-    a->uc2ue0T.upload(transposed(pad_cols(O_.uc2ue0, K1_, O_.rank_u, ru_), K1_, ru_), &total);  // ru x K1
-    a->uc2ue1T.upload(transposed(pad_rows(O_.uc2ue1, O_.rank_u, K0_, ru_), ru_, K0_), &total);  // K0 x ru
-    a->dc2de0T.upload(transposed(pad_cols(O_.dc2de0, K1_, O_.rank_d, rd_), K1_, rd_), &total);  // rd x K1
-    a->dc2de1T.upload(transposed(pad_rows(O_.dc2de1, O_.rank_d, K0_, rd_), rd_, K0_), &total);  // K0 x rd
-    if (u2u_fact_) a->u2urT.upload(transposed(conv(u2u_rank_factor(O_, ru_)), 8 * K0_, ru_), &total);  // ru x 8K0
-    if (d2d_fact_) a->d2drT.upload(transposed(conv(d2d_rank_factor(O_, rd_)), rd_, 8 * K1_), &total);  // 8K1 x rd
-    a->u2uT.upload(transposed(conv(O_.u2u), 8 * K0_, K0_), &total);                                     // K0 x 8K0
-    a->d2dT.upload(transposed(conv(O_.d2d), K1_, 8 * K1_), &total);                                     // 8K1 x K1
+    a->op = &ops_->transposed();
     a->tden.alloc((int64_t)k1_ * n_trg_ * nvb_, &total);
     a->sval.alloc((int64_t)k0_ * n_src_ * nvb_, &total);
     // the adjoint's node table and the transposition of a list with images: a forward item v of
@@ -1207,7 +936,7 @@ class DevicePlan final : public DevicePlanBase {
     a->sb.upload(asb, &total); a->se.upload(ase, &total);
     a->tb.upload(atb, &total); a->te.upload(ate, &total);
     if (bndry_ != kFreeSpace) {
-      a->bcT.upload(transposed(conv(O_.bc[bndry_]), K0_, K1_), &total);
+      a->bcT = ops_->bc(bndry_, true);
       if (vol_) a->volpart.alloc((int64_t)K::vol_adjoint_blocks() * 3 * nvb_, &total);
     }
     device_bytes_ += total;
@@ -1233,67 +962,67 @@ class DevicePlan final : public DevicePlanBase {
                   a.center.p, sx64_.p, n_src_, tx64_.p, a.tden.p, n_trg_, a.sval.p, true, nv, g_vs, o_vs);
     // (L2T P2P)^T: target points -> their leaf's downward equivalent surface (RAD1)
     K::p2p_surface(st_, ek, n_tleaf_, t_leaf_.p, a.iota.p, t_leaf_.p, a.tb.p, a.te.p, a.center.p, a.nsz.p, kRad1,
-                   unit_surf_.p, ns_, tx_.p, a.tden.p, n_trg_, eq_.p, l2t_rc_.p, K0_, true, nv, g_vs, eq_vs_);
+                   ops_->unit_surf.p, ns_, tx_.p, a.tden.p, n_trg_, eq_.p, l2t_rc_.p, K0_, true, nv, g_vs, eq_vs_);
     // (W list M2T)^T: target points -> upward equivalent surfaces (RAD0) of their W sources
     K::p2p_surface(st_, ek, a.n_w, a.w_node.p, a.w_ptr.p, a.w_items.p, a.tb.p, a.te.p, a.center.p, a.nsz.p, kRad0,
-                   unit_surf_.p, ns_, tx_.p, a.tden.p, n_trg_, eq_.p, a.w_node.p, K0_, true, nv, g_vs, eq_vs_);
+                   ops_->unit_surf.p, ns_, tx_.p, a.tden.p, n_trg_, eq_.p, a.w_node.p, K0_, true, nv, g_vs, eq_vs_);
     // D2T GEMMs^T: equivalent -> check potential of each target leaf
-    K::gemm_rows(st_, n_l2t_, rd_, K0_, eq_.p, l2t_rc_.p, K0_, a.dc2de1T.p, ctmp_.p, l2t_seq_.p, rd_, nullptr, false,
+    K::gemm_rows(st_, n_l2t_, rd_, K0_, eq_.p, l2t_rc_.p, K0_, a.op->dc2de1.p, ctmp_.p, l2t_seq_.p, rd_, nullptr, false,
                  gemm_work_.p, gemm_work_elems_, sp, nv, eq_vs_, ctmp_vs_);
-    K::gemm_rows(st_, n_l2t_, K1_, rd_, ctmp_.p, l2t_seq_.p, rd_, a.dc2de0T.p, dn_.p, l2t_ra_.p, K1_, l2t_alpha_.p, true,
+    K::gemm_rows(st_, n_l2t_, K1_, rd_, ctmp_.p, l2t_seq_.p, rd_, a.op->dc2de0.p, dn_.p, l2t_ra_.p, K1_, l2t_alpha_.p, true,
                  gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, dn_vs_);
     // D2D^T, bottom-up: parent += [8 children] x [D2D_0 .. D2D_7]^T
     for (int l = max_depth_; l >= 1; l--) {
       const LevelRows& L = *l2l_[l - 1];
-      if (d2d_fact_ && L.n >= kFactorRows) {
-        K::gemm_rows(st_, L.n, rd_, 8 * K1_, dn_.p, L.rc.p, K1_, a.d2drT.p, ctmp_.p, lvl_seq_.p, rd_, nullptr, false,
+      if (ops_->d2d_fact && L.n >= kFactorRows) {
+        K::gemm_rows(st_, L.n, rd_, 8 * K1_, dn_.p, L.rc.p, K1_, a.op->d2dr.p, ctmp_.p, lvl_seq_.p, rd_, nullptr, false,
                      gemm_work_.p, gemm_work_elems_, sp, nv, dn_vs_, ctmp_vs_);
-        K::gemm_rows(st_, L.n, K1_, rd_, ctmp_.p, lvl_seq_.p, rd_, a.dc2de0T.p, dn_.p, L.ra.p, K1_, nullptr, true,
+        K::gemm_rows(st_, L.n, K1_, rd_, ctmp_.p, lvl_seq_.p, rd_, a.op->dc2de0.p, dn_.p, L.ra.p, K1_, nullptr, true,
                      gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, dn_vs_);
       } else {
-        K::gemm_rows(st_, L.n, K1_, 8 * K1_, dn_.p, L.rc.p, K1_, a.d2dT.p, dn_.p, L.ra.p, K1_, nullptr, true, gemm_work_.p,
+        K::gemm_rows(st_, L.n, K1_, 8 * K1_, dn_.p, L.rc.p, K1_, a.op->d2d.p, dn_.p, L.ra.p, K1_, nullptr, true, gemm_work_.p,
                      gemm_work_elems_, sp, nv, dn_vs_, dn_vs_);
       }
     }
     // (periodic boundary)^T: root equivalent density += root check potential x BC^T
     if (bndry_ != kFreeSpace)
-      K::gemm_rows(st_, 1, K0_, K1_, dn_.p, lvl_seq_.p, K1_, a.bcT.p, eq_.p, lvl_seq_.p, K0_, nullptr, true, gemm_work_.p,
+      K::gemm_rows(st_, 1, K0_, K1_, dn_.p, lvl_seq_.p, K1_, a.bcT, eq_.p, lvl_seq_.p, K0_, nullptr, true, gemm_work_.p,
                    gemm_work_elems_, sp, nv, dn_vs_, eq_vs_);
     // V list^T: the M2L of offset -R from the target parents' children to the source parents'
     // (the spectra buffers swap roles: Y_ holds the new sources, X_ the new targets)
     for (int v = 0; v < nv; v++) {
-      K::fft_up(st_, n_vtrg_, v_trg_fc_.p, dn_.p + v * dn_vs_, K1_, e1_, m_, lattice_.p, lattice_inv_.p, a.fft_scal.p, Y_.p,
+      K::fft_up(st_, n_vtrg_, v_trg_fc_.p, dn_.p + v * dn_vs_, K1_, e1_, m_, ops_->lattice.p, ops_->lattice_inv.p, a.fft_scal.p, Y_.p,
                 1, 0, split_ ? vbound_.p : nullptr);
       K::hadamard_tiled(st_, a.vt.n, M_dim_, e0_, e1_, n_off_, a.vt.t0.p, a.vt.u0.p, a.vt.usrc.p, a.vt.d0.p, a.vt.dent.p,
-                        a.vt.uidx.p, a.vt.gmask.p, v_offsets_.p, V_.p, Y_.p, X_.p, tuning.hadamard_tpb,
+                        a.vt.uidx.p, a.vt.gmask.p, v_offsets_.p, ops_->V.p, Y_.p, X_.p, tuning.hadamard_tpb,
                         split_ ? &hparts(a.vrscale) : nullptr);
-      K::ifft_down(st_, a.n_vt, a.v_fc.p, X_.p, eq_.p + v * eq_vs_, K0_, e0_, m_, lattice_.p, lattice_inv_.p, ns_,
+      K::ifft_down(st_, a.n_vt, a.v_fc.p, X_.p, eq_.p + v * eq_vs_, K0_, e0_, m_, ops_->lattice.p, ops_->lattice_inv.p, ns_,
                    a.ifft_scal.p);
     }
     // (X list S2L)^T: downward check surfaces (RAD0) -> source points
     K::far_points(st_, ek, a.n_x, a.x_leaf.p, a.x_ptr.p, a.x_node.p, a.x_den.p, a.x_rad.p, a.sb.p, a.se.p,
-                  a.center.p, a.nsz.p, unit_surf_.p, ns_, sx_.p, n_src_, dn_.p, a.sval.p, true, nv, dn_vs_, o_vs);
+                  a.center.p, a.nsz.p, ops_->unit_surf.p, ns_, sx_.p, n_src_, dn_.p, a.sval.p, true, nv, dn_vs_, o_vs);
     // U2U^T, top-down: [8 children] += parent x [U2U_0 .. U2U_7]^T
     for (int l = 0; l <= max_depth_ - 1; l++) {
       const LevelRows& L = *m2m_[l];
-      if (u2u_fact_ && L.n >= kFactorRows) {
-        K::gemm_rows(st_, L.n, ru_, K0_, eq_.p, L.rc.p, K0_, a.uc2ue1T.p, ctmp_.p, lvl_seq_.p, ru_, nullptr, false,
+      if (ops_->u2u_fact && L.n >= kFactorRows) {
+        K::gemm_rows(st_, L.n, ru_, K0_, eq_.p, L.rc.p, K0_, a.op->uc2ue1.p, ctmp_.p, lvl_seq_.p, ru_, nullptr, false,
                      gemm_work_.p, gemm_work_elems_, sp, nv, eq_vs_, ctmp_vs_);
-        K::gemm_rows(st_, L.n, 8 * K0_, ru_, ctmp_.p, lvl_seq_.p, ru_, a.u2urT.p, eq_.p, L.ra.p, K0_, nullptr, true,
+        K::gemm_rows(st_, L.n, 8 * K0_, ru_, ctmp_.p, lvl_seq_.p, ru_, a.op->u2ur.p, eq_.p, L.ra.p, K0_, nullptr, true,
                      gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, eq_vs_);
       } else {
-        K::gemm_rows(st_, L.n, 8 * K0_, K0_, eq_.p, L.rc.p, K0_, a.u2uT.p, eq_.p, L.ra.p, K0_, nullptr, true, gemm_work_.p,
+        K::gemm_rows(st_, L.n, 8 * K0_, K0_, eq_.p, L.rc.p, K0_, a.op->u2u.p, eq_.p, L.ra.p, K0_, nullptr, true, gemm_work_.p,
                      gemm_work_elems_, sp, nv, eq_vs_, eq_vs_);
       }
     }
     // S2U GEMMs^T: upward equivalent -> check potential of each source leaf
-    K::gemm_rows(st_, n_s2m_, ru_, K0_, eq_.p, s2m_node_.p, K0_, a.uc2ue1T.p, ctmp_.p, s2m_orow_.p, ru_, nullptr, false,
+    K::gemm_rows(st_, n_s2m_, ru_, K0_, eq_.p, s2m_node_.p, K0_, a.op->uc2ue1.p, ctmp_.p, s2m_orow_.p, ru_, nullptr, false,
                  gemm_work_.p, gemm_work_elems_, sp, nv, eq_vs_, ctmp_vs_);
-    K::gemm_rows(st_, n_s2m_, K1_, ru_, ctmp_.p, s2m_orow_.p, ru_, a.uc2ue0T.p, chk_.p, s2m_orow_.p, K1_, s2m_alpha_.p, false,
+    K::gemm_rows(st_, n_s2m_, K1_, ru_, ctmp_.p, s2m_orow_.p, ru_, a.op->uc2ue0.p, chk_.p, s2m_orow_.p, K1_, s2m_alpha_.p, false,
                  gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, chk_vs_);
     // (S2U P2P)^T: upward check surface (RAD1) -> the leaf's source points
     K::far_points(st_, ek, n_s2m_, s2m_node_.p, a.iota.p, s2m_node_.p, a.s2u_den.p, a.s2u_rad.p, a.sb.p, a.se.p,
-                  a.center.p, a.nsz.p, unit_surf_.p, ns_, sx_.p, n_src_, chk_.p, a.sval.p, true, nv, chk_vs_, o_vs);
+                  a.center.p, a.nsz.p, ops_->unit_surf.p, ns_, sx_.p, n_src_, chk_.p, a.sval.p, true, nv, chk_vs_, o_vs);
     // gather^T: back to the input order of the sources (times the density scale)
     K::scatter_output(st_, n_src_, k0_, a.sval.p, src_perm_.p, den_scale, d_out, nv, o_vs);
   }
@@ -1323,34 +1052,34 @@ class DevicePlan final : public DevicePlanBase {
     mark(1);
     // S2U: sources -> upward check surface (RAD1), then check -> equivalent
     K::p2p_surface(st_, ek, n_s2m_, s2m_node_.p, s2m_ptr_.p, s2m_items_.p, src_begin_.p, src_end_.p, center_.p, node_size_.p,
-                   kRad1, unit_surf_.p, ns_, sx_.p, sden_.p, n_src_, chk_.p, s2m_orow_.p, K1_, false, nv, den_vs, chk_vs_);
+                   kRad1, ops_->unit_surf.p, ns_, sx_.p, sden_.p, n_src_, chk_.p, s2m_orow_.p, K1_, false, nv, den_vs, chk_vs_);
     mark(2);
-    K::gemm_rows(st_, n_s2m_, ru_, K1_, chk_.p, s2m_orow_.p, K1_, uc2ue0_.p, ctmp_.p, s2m_orow_.p, ru_, s2m_alpha_.p, false,
+    K::gemm_rows(st_, n_s2m_, ru_, K1_, chk_.p, s2m_orow_.p, K1_, ops_->uc2ue0.p, ctmp_.p, s2m_orow_.p, ru_, s2m_alpha_.p, false,
                  gemm_work_.p, gemm_work_elems_, sp, nv, chk_vs_, ctmp_vs_);
-    K::gemm_rows(st_, n_s2m_, K0_, ru_, ctmp_.p, s2m_orow_.p, ru_, uc2ue1_.p, eq_.p, s2m_node_.p, K0_, nullptr, false,
+    K::gemm_rows(st_, n_s2m_, K0_, ru_, ctmp_.p, s2m_orow_.p, ru_, ops_->uc2ue1.p, eq_.p, s2m_node_.p, K0_, nullptr, false,
                  gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, eq_vs_);
     mark(3);
     // U2U, bottom-up: parent row = [8 children] x stacked U2U
     for (int l = max_depth_ - 1; l >= 0; l--) {
       const LevelRows& L = *m2m_[l];
-      if (u2u_fact_ && L.n >= kFactorRows) {  // [8 children] -> rank coordinates -> parent
-        K::gemm_rows(st_, L.n, ru_, 8 * K0_, eq_.p, L.ra.p, K0_, u2ur_.p, ctmp_.p, lvl_seq_.p, ru_, nullptr, false,
+      if (ops_->u2u_fact && L.n >= kFactorRows) {  // [8 children] -> rank coordinates -> parent
+        K::gemm_rows(st_, L.n, ru_, 8 * K0_, eq_.p, L.ra.p, K0_, ops_->u2ur.p, ctmp_.p, lvl_seq_.p, ru_, nullptr, false,
                      gemm_work_.p, gemm_work_elems_, sp, nv, eq_vs_, ctmp_vs_);
-        K::gemm_rows(st_, L.n, K0_, ru_, ctmp_.p, lvl_seq_.p, ru_, uc2ue1_.p, eq_.p, L.rc.p, K0_, nullptr, false,
+        K::gemm_rows(st_, L.n, K0_, ru_, ctmp_.p, lvl_seq_.p, ru_, ops_->uc2ue1.p, eq_.p, L.rc.p, K0_, nullptr, false,
                      gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, eq_vs_);
       } else {
-        K::gemm_rows(st_, L.n, K0_, 8 * K0_, eq_.p, L.ra.p, K0_, u2u_.p, eq_.p, L.rc.p, K0_, nullptr, false, gemm_work_.p,
+        K::gemm_rows(st_, L.n, K0_, 8 * K0_, eq_.p, L.ra.p, K0_, ops_->u2u.p, eq_.p, L.rc.p, K0_, nullptr, false, gemm_work_.p,
                      gemm_work_elems_, sp, nv, eq_vs_, eq_vs_);
       }
     }
     // periodic images beyond the root's colleagues: root check potential += root equivalent x BC
     if (bndry_ != kFreeSpace)
-      K::gemm_rows(st_, 1, K1_, K0_, eq_.p, lvl_seq_.p, K0_, bc_.p, dn_.p, lvl_seq_.p, K1_, nullptr, true, gemm_work_.p,
+      K::gemm_rows(st_, 1, K1_, K0_, eq_.p, lvl_seq_.p, K0_, bc_, dn_.p, lvl_seq_.p, K1_, nullptr, true, gemm_work_.p,
                    gemm_work_elems_, sp, nv, eq_vs_, dn_vs_);
     mark(4);
     // X list: source points -> downward check surface (RAD0)
     K::p2p_surface(st_, ek, n_x_, x_node_.p, x_ptr_.p, x_items_.p, src_begin_.p, src_end_.p, center_.p, node_size_.p, kRad0,
-                   unit_surf_.p, ns_, sx_.p, sden_.p, n_src_, dn_.p, x_orow_.p, K1_, true, nv, den_vs, dn_vs_);
+                   ops_->unit_surf.p, ns_, sx_.p, sden_.p, n_src_, dn_.p, x_orow_.p, K1_, true, nv, den_vs, dn_vs_);
     mark(5);
     // V list: groups of 16 vectors through the 16-vector Hadamard, or one vector at a time
     // through the spectra buffers (with several passes the three sub-phases are timed per
@@ -1363,22 +1092,22 @@ class DevicePlan final : public DevicePlanBase {
       const int v0 = grouped ? 16 * g : g, gn = grouped ? std::min(16, nv - v0) : 1;
       if (sub) HIP_CHECK(hipEventRecord(vev_[4 * g], st_));
       for (int v = v0; v < v0 + gn; v++)
-        K::fft_up(st_, n_vsrc_, v_src_fc_.p, eq_.p + v * eq_vs_, K0_, e0_, m_, lattice_.p, lattice_inv_.p, v_src_scal_.p,
+        K::fft_up(st_, n_vsrc_, v_src_fc_.p, eq_.p + v * eq_vs_, K0_, e0_, m_, ops_->lattice.p, ops_->lattice_inv.p, v_src_scal_.p,
                   grouped ? Xv_.p : X_.p, grouped ? 16 : 1, grouped ? v - v0 : 0,
                   split_ && !grouped ? vbound_.p : nullptr);
       if (sub) HIP_CHECK(hipEventRecord(vev_[4 * g + 1], st_));
       if (n_pass == 1) mark(6);
       if (grouped)
-        K::hadamard_vec16(st_, n_vtrg_, M_dim_, v_partner_.p, Vb_.p, Xv_.p, Yv_.p, tuning.hadamard_vec_tpw);
+        K::hadamard_vec16(st_, n_vtrg_, M_dim_, v_partner_.p, ops_->vb(), Xv_.p, Yv_.p, tuning.hadamard_vec_tpw);
       else
         K::hadamard_tiled(st_, vt_.n, M_dim_, e0_, e1_, n_off_, vt_.t0.p, vt_.u0.p, vt_.usrc.p, vt_.d0.p, vt_.dent.p,
-                          vt_.uidx.p, vt_.gmask.p, v_offsets_.p, V_.p, X_.p, Y_.p, tuning.hadamard_tpb,
+                          vt_.uidx.p, vt_.gmask.p, v_offsets_.p, ops_->V.p, X_.p, Y_.p, tuning.hadamard_tpb,
                           split_ ? &hparts(vrscale_) : nullptr);
       if (sub) HIP_CHECK(hipEventRecord(vev_[4 * g + 2], st_));
       if (n_pass == 1) mark(7);
       for (int v = v0; v < v0 + gn; v++)
-        K::ifft_down(st_, n_vtrg_, v_trg_fc_.p, grouped ? Yv_.p : Y_.p, dn_.p + v * dn_vs_, K1_, e1_, m_, lattice_.p,
-                     lattice_inv_.p, ns_, v_trg_scal_.p, grouped ? 16 : 1, grouped ? v - v0 : 0);
+        K::ifft_down(st_, n_vtrg_, v_trg_fc_.p, grouped ? Yv_.p : Y_.p, dn_.p + v * dn_vs_, K1_, e1_, m_, ops_->lattice.p,
+                     ops_->lattice_inv.p, ns_, v_trg_scal_.p, grouped ? 16 : 1, grouped ? v - v0 : 0);
       if (sub) HIP_CHECK(hipEventRecord(vev_[4 * g + 3], st_));
     }
     if (n_pass > 1) {
@@ -1389,26 +1118,26 @@ class DevicePlan final : public DevicePlanBase {
     // D2D, top-down: 8 children rows += parent x [D2D_0 .. D2D_7]
     for (int l = 1; l <= max_depth_; l++) {
       const LevelRows& L = *l2l_[l - 1];
-      if (d2d_fact_ && L.n >= kFactorRows) {  // parent check -> rank coordinates -> [8 children]
-        K::gemm_rows(st_, L.n, rd_, K1_, dn_.p, L.ra.p, K1_, dc2de0_.p, ctmp_.p, lvl_seq_.p, rd_, nullptr, false,
+      if (ops_->d2d_fact && L.n >= kFactorRows) {  // parent check -> rank coordinates -> [8 children]
+        K::gemm_rows(st_, L.n, rd_, K1_, dn_.p, L.ra.p, K1_, ops_->dc2de0.p, ctmp_.p, lvl_seq_.p, rd_, nullptr, false,
                      gemm_work_.p, gemm_work_elems_, sp, nv, dn_vs_, ctmp_vs_);
-        K::gemm_rows(st_, L.n, 8 * K1_, rd_, ctmp_.p, lvl_seq_.p, rd_, d2dr_.p, dn_.p, L.rc.p, K1_, nullptr, true,
+        K::gemm_rows(st_, L.n, 8 * K1_, rd_, ctmp_.p, lvl_seq_.p, rd_, ops_->d2dr.p, dn_.p, L.rc.p, K1_, nullptr, true,
                      gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, dn_vs_);
       } else {
-        K::gemm_rows(st_, L.n, 8 * K1_, K1_, dn_.p, L.ra.p, K1_, d2d_.p, dn_.p, L.rc.p, K1_, nullptr, true, gemm_work_.p,
+        K::gemm_rows(st_, L.n, 8 * K1_, K1_, dn_.p, L.ra.p, K1_, ops_->d2d.p, dn_.p, L.rc.p, K1_, nullptr, true, gemm_work_.p,
                      gemm_work_elems_, sp, nv, dn_vs_, dn_vs_);
       }
     }
     mark(9);
     // D2T: check -> equivalent
-    K::gemm_rows(st_, n_l2t_, rd_, K1_, dn_.p, l2t_ra_.p, K1_, dc2de0_.p, ctmp_.p, l2t_seq_.p, rd_, l2t_alpha_.p, false,
+    K::gemm_rows(st_, n_l2t_, rd_, K1_, dn_.p, l2t_ra_.p, K1_, ops_->dc2de0.p, ctmp_.p, l2t_seq_.p, rd_, l2t_alpha_.p, false,
                  gemm_work_.p, gemm_work_elems_, sp, nv, dn_vs_, ctmp_vs_);
-    K::gemm_rows(st_, n_l2t_, K0_, rd_, ctmp_.p, l2t_seq_.p, rd_, dc2de1_.p, eq_.p, l2t_rc_.p, K0_, nullptr, false,
+    K::gemm_rows(st_, n_l2t_, K0_, rd_, ctmp_.p, l2t_seq_.p, rd_, ops_->dc2de1.p, eq_.p, l2t_rc_.p, K0_, nullptr, false,
                  gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, eq_vs_);
     mark(10);
     // equivalent surfaces -> targets (own downward equivalent + W list)
     K::far_points(st_, pk, n_tleaf_, t_leaf_.p, far_ptr_.p, far_node_.p, far_den_.p, far_rad_.p, trg_begin_.p, trg_end_.p,
-                  center_.p, node_size_.p, unit_surf_.p, ns_, tx_.p, n_trg_, eq_.p, tval_.p, false, nv, eq_vs_, val_vs);
+                  center_.p, node_size_.p, ops_->unit_surf.p, ns_, tx_.p, n_trg_, eq_.p, tval_.p, false, nv, eq_vs_, val_vs);
     mark(11);
     // U list: near-field P2P
     K::p2p_points(st_, pk, n_tleaf_, t_leaf_.p, u_ptr_.p, u_items_.p, trg_begin_.p, trg_end_.p, src_begin_.p, src_end_.p,
@@ -1442,9 +1171,20 @@ class DevicePlan final : public DevicePlanBase {
 }  // namespace
 
 std::unique_ptr<DevicePlanBase> make_plan(const Octree& T, const Operators& O, const double* src_xyz, const double* trg_xyz,
-                                          int precision, int n_vec_max, hipStream_t stream) {
-  if (precision == 0) return std::make_unique<DevicePlan<double>>(T, O, src_xyz, trg_xyz, n_vec_max, stream);
-  if (precision == 1) return std::make_unique<DevicePlan<float>>(T, O, src_xyz, trg_xyz, n_vec_max, stream);
+                                          int precision, int n_vec_max, hipStream_t stream,
+                                          std::shared_ptr<DeviceOpsBase> ops) {
+  if (precision == 0)
+    return std::make_unique<DevicePlan<double>>(T, O, std::static_pointer_cast<DeviceOps<double>>(ops), src_xyz, trg_xyz,
+                                                n_vec_max, stream);
+  if (precision == 1)
+    return std::make_unique<DevicePlan<float>>(T, O, std::static_pointer_cast<DeviceOps<float>>(ops), src_xyz, trg_xyz,
+                                               n_vec_max, stream);
+  throw Error(kErrInvalidArgument, "precision must be 0 (fp64) or 1 (mixed fp32)");
+}
+
+std::shared_ptr<DeviceOpsBase> make_device_ops(const Operators& O, int precision) {
+  if (precision == 0) return std::make_shared<DeviceOps<double>>(O);
+  if (precision == 1) return std::make_shared<DeviceOps<float>>(O);
   throw Error(kErrInvalidArgument, "precision must be 0 (fp64) or 1 (mixed fp32)");
 }
 

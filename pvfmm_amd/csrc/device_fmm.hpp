@@ -79,8 +79,17 @@ class DevicePlanBase {
   bool timing_ = false;
 };
 
-// precision: 0 = FP64 throughout, 1 = FP32 bulk with FP64 operators precompute and FP64 merge
+// An operator set on the current device (device_ops.hpp), shared by the plans made with it.
+class DeviceOpsBase {
+ public:
+  virtual ~DeviceOpsBase() = default;
+  virtual int64_t bytes() const = 0;
+};
+
+// precision: 0 = FP64 throughout, 1 = FP32 bulk with FP64 operators precompute and FP64 merge.
+// The operators must outlive what is made from them.
+std::shared_ptr<DeviceOpsBase> make_device_ops(const Operators& O, int precision);
 std::unique_ptr<DevicePlanBase> make_plan(const Octree& T, const Operators& O, const double* src_xyz, const double* trg_xyz,
-                                          int precision, int n_vec_max, hipStream_t stream);
+                                          int precision, int n_vec_max, hipStream_t stream, std::shared_ptr<DeviceOpsBase> ops);
 
 }  // namespace pvfmm_amd

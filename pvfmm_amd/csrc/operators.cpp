@@ -439,7 +439,10 @@ void build_operators(Operators& O, int kernel_id, int m, double cutoff_rel, int 
   O.on_device = device_precompute_enabled();
   compute_factors(O);
   compute_translations(O);
-  compute_v1(O);
+}
+
+void ensure_v1(Operators& O) {
+  if (O.v1.empty()) compute_v1(O);
 }
 
 // ----------------------------------------------------------------------------- periodic boundary
@@ -942,8 +945,6 @@ void build_operators_cached(Operators& O, int kernel_id, int m, double cutoff_re
     O.v1.assign((size_t)27 * M_dim * bw * bh, 0.0);
     for (int R = 0; R < 27; R++)
       if (R != 13) std::memcpy(&O.v1[(size_t)R * M_dim * bw * bh], mats[kV1T][R].v.data(), sizeof(double) * mats[kV1T][R].v.size());
-  } else {
-    compute_v1(O);
   }
   // boundary operators, one per BoundaryType (FreeSpace stored as zeros, include/fmm_pts.txx:
   // 288-300): read where present; a new file gets all of them, as the reference computes them
@@ -954,6 +955,7 @@ void build_operators_cached(Operators& O, int kernel_id, int m, double cutoff_re
     for (int b = 1; b <= 3; b++) O.bc[b] = mats[kBCT][b].v;
   O.from_cache = have_f && have_t && have_v;
   if (exists) return;  // an existing file is never replaced (PrecompMat::Save2File with replace = false)
+  ensure_v1(O);
   build_bc_operators(O, (1 << kPX) | (1 << kPXY) | (1 << kPXYZ));
   std::vector<Mat> bcm{Mat{K0, K1, std::vector<double>((size_t)K0 * K1, 0.0)}};
   for (int b = 1; b <= 3; b++) bcm.push_back(Mat{K0, K1, O.bc[b]});

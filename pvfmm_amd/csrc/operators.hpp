@@ -32,7 +32,9 @@ struct Operators {
   std::vector<double> u2u;     // 8 stacked: (8*ns*e0) x (ns*e0), child c rows [c*ns*e0, (c+1)*ns*e0)
   std::vector<double> d2d;     // (ns*e1) x (8*ns*e1), child c columns [c*ns*e1, (c+1)*ns*e1)
   // M2L transfer blocks: [R 27][f M_dim][t*e1+j][s*e0+i] complex, R = (dx+1)+3(dy+1)+9(dz+1)
-  // (R = 13 unused), 1/n1^3 included; zero blocks for adjacent child pairs.
+  // (R = 13 unused), 1/n1^3 included; zero blocks for adjacent child pairs.  The stored and
+  // exported form: computed on request (ensure_v1) or read from a precompute file; evaluations
+  // build their own blocks on the device (transfer.hpp).
   std::vector<std::complex<double>> v1;
   std::vector<int32_t> v1_offsets;  // the 26 offsets R in use
 
@@ -51,6 +53,7 @@ struct Operators {
 // cutoff_rel <= 0 selects the reference's rule 4*eps*max_S with eps of `precision`
 // (0: FP64, 1: FP32 as the reference's float build).
 void build_operators(Operators& O, int kernel_id, int m, double cutoff_rel = 0.0, int precision = 0);
+void ensure_v1(Operators& O);  // computes O.v1 unless it is there
 
 // The same through a precompute file in directory `dir` (no file I/O when dir is null or empty,
 // or for a custom cutoff): Precomp_<ker_name>_m<m>[_mixed].data in the container format of the
