@@ -138,7 +138,7 @@ def roofline(ph: dict, st: dict, m: int, real_bytes: int):
     target-stationary model's bytes (each pair re-reading its partner's spectrum), which the
     kernel avoids by staging each tile's partners in LDS once; `traffic` is the measured HBM
     bytes per launch.  U-list P2P: 16 flop per pair for laplace_grad, VALU-bound."""
-    n1 = 2 * m
+    n1 = 2 * m - 1
     M_dim = n1 * n1 * (n1 // 2 + 1)
     dom = max(ph, key=ph.get)
     t = ph[dom] * 1e-3

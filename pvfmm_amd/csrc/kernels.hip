@@ -7,7 +7,7 @@
 //    mixed-precision path), the splits of a target in a fixed order.
 //  * Row-gathered GEMM for S2M/L2T (check -> equivalent), M2M and L2L (8 children stored
 //    contiguously so a parent row is one 8*K row of the child block), on MFMA.
-//  * V list: pruned separable DFT of the m^3 surface lattice embedded in the (2m)^3 grid,
+//  * V list: pruned separable DFT of the m^3 surface lattice embedded in the (2m-1)^3 grid,
 //    one x-frequency slice at a time in LDS; a tiled frequency-domain Hadamard sum over the 26
 //    parent offsets on the matrix cores (FP32 scalar kernels on the bf16 cores with exact
 //    three-way operand splits); the inverse DFT evaluates only the check-surface points.
@@ -926,7 +926,7 @@ __global__ __launch_bounds__(512) void k_fft_up(const int32_t* __restrict__ firs
                                                 Real* __restrict__ X, int vg, int vi) {
   extern __shared__ unsigned char smem_raw[];
   Real* sm = reinterpret_cast<Real*>(smem_raw);
-  const int n1 = 2 * m, nh = m + 1, M_dim = n1 * n1 * nh, ns = 6 * (m - 1) * (m - 1) + 2;
+  const int n1 = 2 * m - 1, nh = m, M_dim = n1 * n1 * nh, ns = 6 * (m - 1) * (m - 1) + 2;
   const int m2 = m * m, m3 = m2 * m, mn = m * n1;
   Real* cube = sm;                 // CB * m^3
   Real* twr = cube + CB * m3;      // n1
@@ -1005,7 +1005,7 @@ __global__ __launch_bounds__(512) void k_ifft_down(const int32_t* __restrict__ f
                                                    int vg, int vi) {
   extern __shared__ unsigned char smem_raw[];
   Real* sm = reinterpret_cast<Real*>(smem_raw);
-  const int n1 = 2 * m, nh = m + 1, M_dim = n1 * n1 * nh;
+  const int n1 = 2 * m - 1, nh = m, M_dim = n1 * n1 * nh;
   const int nn = n1 * n1, nm = n1 * m, m2 = m * m;
   Real* twr = sm;                  // n1
   Real* twi = twr + n1;
@@ -1061,7 +1061,7 @@ __global__ __launch_bounds__(512) void k_ifft_down(const int32_t* __restrict__ f
       s2i[o] = ai;
     }
     __syncthreads();
-    const Real wk = (kx == 0 || 2 * kx == n1) ? Real(1) : Real(2);
+    const Real wk = kx == 0 ? Real(1) : Real(2);
 #pragma unroll
     for (int q = 0; q < MAXQ; q++) {
       const int o = tid + q * nt;
@@ -1138,24 +1138,19 @@ __device__ __forceinline__ void sfor_(F& f) {
 template <int N, typename F>
 __device__ __forceinline__ void sfor(F f) { sfor_<0, N>(f); }
 
-// s += g * w^{SIGN K}, w = exp(2 pi i / N), K compile-time: twiddles +-1 and +-i become adds,
-// real or imaginary twiddles one FMA per part.
-template <int N, int K, int SIGN, typename Real>
-__device__ __forceinline__ void cmac_tw(Real gr, Real gi, Real& sr, Real& si) {
-  constexpr double c = ct_cs(K, N, false), s = SIGN * ct_cs(K, N, true);
-  if constexpr (s == 0.0) {
-    if constexpr (c == 1.0) { sr += gr; si += gi; }
-    else if constexpr (c == -1.0) { sr -= gr; si -= gi; }
-    else { sr = fma(gr, (Real)c, sr); si = fma(gi, (Real)c, si); }
-  } else if constexpr (c == 0.0) {
-    if constexpr (s == 1.0) { sr -= gi; si += gr; }
-    else if constexpr (s == -1.0) { sr += gi; si -= gr; }
-    else { sr = fma(-gi, (Real)s, sr); si = fma(gr, (Real)s, si); }
+// Cosine and sine sums of a complex value g: c += g cos(2 pi K / N), s += g sin(2 pi K / N), K
+// compile-time (K = 0 adds to the cosine sum only).
+template <int N, int K, typename Real>
+__device__ __forceinline__ void cs_tw(Real gr, Real gi, Real& cr, Real& ci, Real& sr, Real& si) {
+  if constexpr (K == 0) {
+    cr += gr;
+    ci += gi;
   } else {
-    sr = fma(gr, (Real)c, sr);
-    sr = fma(-gi, (Real)s, sr);
-    si = fma(gr, (Real)s, si);
-    si = fma(gi, (Real)c, si);
+    constexpr double c = ct_cs(K, N, false), s = ct_cs(K, N, true);
+    cr = fma(gr, (Real)c, cr);
+    ci = fma(gi, (Real)c, ci);
+    sr = fma(gr, (Real)s, sr);
+    si = fma(gi, (Real)s, si);
   }
 }
 
@@ -1222,7 +1217,7 @@ __global__ __launch_bounds__(256) void k_run_scale(int n_tiles, int tpb, const i
 // blocks share one CU's 160 KiB.
 template <typename Real, int M>
 struct DftShape {
-  static constexpr int N1 = 2 * M, NH = M + 1, MD = N1 * N1 * NH, M2 = M * M;
+  static constexpr int N1 = 2 * M - 1, NH = M, MD = N1 * N1 * NH, M2 = M * M;
   static constexpr int CG = (8 * M2 <= 512) ? 8 : (4 * M2 <= 512) ? 4 : (2 * M2 <= 512) ? 2 : 1;
   static constexpr int NT = M2 * CG;
   static constexpr int LPT = 8 / CG;
@@ -1234,22 +1229,32 @@ struct DftShape {
   }
   static constexpr int KC_UP = kc_for(8 * M2 * 2 * (int)sizeof(Real));       // s1[c][kx][z][y]
   static constexpr int KC_DN = kc_for(8 * N1 * M * 2 * (int)sizeof(Real));   // s1[c][kx][ky][z]
+  // Waves per SIMD the forward transform is compiled for: at 4 its FP64 form for m >= 10 spills
+  // (m = 10: 138 registers at 4, none at 2; 1.22, 0.95 and 0.82 ms at 4, 3 and 2 on the 1M
+  // adaptive tree), the others fit
+  static constexpr int WAVES_UP = sizeof(Real) == 8 && M >= 10 ? 2 : 4;
   // FP64 recomputes the y stage per half (ky, ky+m) instead of holding both in registers
   static constexpr bool SPLIT_H = sizeof(Real) == 8;
 };
 
+// The grid of the V-list transforms is N = 2m - 1 points per axis, the least that keeps the
+// convolution of the m-point lattices free of wrap-around (displacements -(m-1) .. m-1), so a
+// spectrum has m N^2 values, 18% (m = 10) to 28% (m = 6) fewer than on the usual 2m grid, in
+// every V-list kernel (2M adaptive, m = 10, FP32: Hadamard 3.78 -> 2.84 ms, inverse DFT 1.57 ->
+// 1.37, forward 1.10 -> 1.00; 1M FP64: 5.65 -> 4.61, 1.53 -> 1.42, 0.95 -> 0.82).
+//
 // Forward DFT of the 8 children of one source parent, component i (grid n_slots * e0).
-// x stage (real -> complex, kx < m+1) on thread-owned lattice lines into LDS; then one task
-// per (c, kx, ky < m) runs the y stage for ky and ky+m (w^{-(ky+m)y} = (-1)^y w^{-ky y}) and the
-// z stage of both (X[kz] = E + O, X[kz+m] = E - O over even/odd z), writing the spectra as
-// X[slot][f][8i+c] complex (component-major, so each component's block writes its own 64-byte
-// segment of a row), f = kx + (m+1)(ky + 2m kz).
+// x stage (real -> complex, kx < m) on thread-owned lattice lines into LDS; then one task per
+// (c, kx, ky < m) runs the y stage for ky and N - ky from one pair of cosine and sine sums and
+// the z stage of both the same way, writing the spectra as X[slot][f][8i+c] complex
+// (component-major, so each component's block writes its own 64-byte segment of a row),
+// f = kx + m(ky + N kz).
 // NTS: non-temporal stores of X, which is read back only by the Hadamard, long after its lines
 // would have left the caches (1.20 -> 1.04 ms for the 2M adaptive workload).  Only where each
 // block writes whole lines: with several components (or vectors in one group) the blocks of one
 // parent interleave their stores within a line, which must merge in L2 first.
 template <typename Real, int M, bool NTS>
-__global__ __launch_bounds__((DftShape<Real, M>::NT), 4) void k_fft_up_m(const int32_t* __restrict__ first_child,
+__global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_UP)) void k_fft_up_m(const int32_t* __restrict__ first_child,
                                                                          const Real* __restrict__ up, int K0, int e0,
                                                                          const int32_t* __restrict__ lat_inv,
                                                                          const Real* __restrict__ scal, Real* __restrict__ X,
@@ -1323,76 +1328,80 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), 4) void k_fft_up_m(const i
       const int c = T % 8, kl = (T / 8) % kn, ky = T / (8 * kn), kx = k0 + kl;
       const Real* pr = &s1r[c * CST + kl * M2];
       const Real* pi = &s1i[c * CST + kl * M2];
-      // z stage of one y-stage output column g (z < m) for frequency row kyy
+      auto store = [&](int64_t f, Real re, Real im) __attribute__((always_inline)) {
+        // an opaque copy of the base keeps the 64-bit store addresses from being hoisted
+        // out of the unrolled loop (they would not fit in registers for FP64)
+        Real* xb = Xs;
+        asm volatile("" : "+s"(xb));
+        Real* d = xb + (f * vg * 8 * e0 + c) * 2;
+        if constexpr (NTS) {
+          __builtin_nontemporal_store(re, &d[0]);
+          __builtin_nontemporal_store(im, &d[1]);
+        } else {
+          d[0] = re;
+          d[1] = im;
+        }
+      };
+      // z stage of one y-stage output column g (z < m) for frequency row kyy: kz and N - kz from
+      // the cosine and sine sums C, S of the column, X[kz] = C - i S, X[N - kz] = C + i S
       auto zstage = [&](const Real* gr, const Real* gi, int kyy) __attribute__((always_inline)) {
         sfor<M>([&](auto ikz) __attribute__((always_inline)) {
           constexpr int kz = decltype(ikz)::value;
-          Real er = 0, ei = 0, orr = 0, oi = 0;
-          sfor<M>([&](auto izz) __attribute__((always_inline)) {
-            constexpr int zz = decltype(izz)::value;
-            if constexpr (zz % 2 == 0)
-              cmac_tw<N1, (kz * zz) % N1, -1>(gr[zz], gi[zz], er, ei);
-            else
-              cmac_tw<N1, (kz * zz) % N1, -1>(gr[zz], gi[zz], orr, oi);
+          Real cr = gr[0], ci = gi[0], sr = 0, si = 0;
+          sfor<M - 1>([&](auto iz1) __attribute__((always_inline)) {
+            constexpr int zz = decltype(iz1)::value + 1;
+            cs_tw<N1, (kz * zz) % N1>(gr[zz], gi[zz], cr, ci, sr, si);
           });
-          const int64_t f0 = kx + (int64_t)NH * (kyy + N1 * kz), f1 = kx + (int64_t)NH * (kyy + N1 * (kz + M));
-          // an opaque copy of the base keeps the 64-bit store addresses from being hoisted
-          // out of the unrolled loop (they would not fit in registers for FP64)
-          Real* xb = Xs;
-          asm volatile("" : "+s"(xb));
-          Real* d0 = xb + (f0 * vg * 8 * e0 + c) * 2;
-          Real* d1 = xb + (f1 * vg * 8 * e0 + c) * 2;
-          if constexpr (NTS) {
-            __builtin_nontemporal_store(er + orr, &d0[0]);
-            __builtin_nontemporal_store(ei + oi, &d0[1]);
-            __builtin_nontemporal_store(er - orr, &d1[0]);
-            __builtin_nontemporal_store(ei - oi, &d1[1]);
-          } else {
-            d0[0] = er + orr; d0[1] = ei + oi;
-            d1[0] = er - orr; d1[1] = ei - oi;
-          }
+          store(kx + (int64_t)NH * (kyy + N1 * kz), cr + si, ci - sr);
+          if constexpr (kz > 0) store(kx + (int64_t)NH * (kyy + N1 * (N1 - kz)), cr - si, ci + sr);
         });
       };
-      // y stage: column zz of ky (E + O) and of ky + m (E - O)
-      auto ystage = [&](int zz, Real& er, Real& ei, Real& orr, Real& oi) __attribute__((always_inline)) {
-        er = ei = orr = oi = 0;
+      // y stage: cosine and sine sums of column zz; rows ky (C - i S) and N - ky (C + i S)
+      auto ystage = [&](int zz, Real& cr, Real& ci, Real& sr, Real& si) __attribute__((always_inline)) {
+        cr = pr[zz * M];
+        ci = pi[zz * M];
+        sr = si = 0;
 #pragma unroll
-        for (int yy = 0, e = 0; yy < M; yy++) {
-          const Real dr = pr[zz * M + yy], di = pi[zz * M + yy];
-          const Real wc = twc[e], ws = -tws[e];
-          const Real tr = dr * wc - di * ws, ti = dr * ws + di * wc;
-          if (yy % 2 == 0) { er += tr; ei += ti; } else { orr += tr; oi += ti; }
+        for (int yy = 1, e = 0; yy < M; yy++) {
           e += ky;
           if (e >= N1) e -= N1;
+          const Real dr = pr[zz * M + yy], di = pi[zz * M + yy];
+          const Real wc = twc[e], ws = tws[e];
+          cr = fma(dr, wc, cr);
+          ci = fma(di, wc, ci);
+          sr = fma(dr, ws, sr);
+          si = fma(di, ws, si);
         }
       };
       if constexpr (S::SPLIT_H) {
         Real gr[M], gi[M];
 #pragma unroll
         for (int zz = 0; zz < M; zz++) {
-          Real er, ei, orr, oi;
-          ystage(zz, er, ei, orr, oi);
-          gr[zz] = er + orr; gi[zz] = ei + oi;
+          Real cr, ci, sr, si;
+          ystage(zz, cr, ci, sr, si);
+          gr[zz] = cr + si; gi[zz] = ci - sr;
         }
         zstage(gr, gi, ky);
+        if (ky > 0) {
 #pragma unroll
-        for (int zz = 0; zz < M; zz++) {
-          Real er, ei, orr, oi;
-          ystage(zz, er, ei, orr, oi);
-          gr[zz] = er - orr; gi[zz] = ei - oi;
+          for (int zz = 0; zz < M; zz++) {
+            Real cr, ci, sr, si;
+            ystage(zz, cr, ci, sr, si);
+            gr[zz] = cr - si; gi[zz] = ci + sr;
+          }
+          zstage(gr, gi, N1 - ky);
         }
-        zstage(gr, gi, ky + M);
       } else {
         Real ar[M], ai[M], br[M], bi[M];
 #pragma unroll
         for (int zz = 0; zz < M; zz++) {
-          Real er, ei, orr, oi;
-          ystage(zz, er, ei, orr, oi);
-          ar[zz] = er + orr; ai[zz] = ei + oi;
-          br[zz] = er - orr; bi[zz] = ei - oi;
+          Real cr, ci, sr, si;
+          ystage(zz, cr, ci, sr, si);
+          ar[zz] = cr + si; ai[zz] = ci - sr;
+          br[zz] = cr - si; bi[zz] = ci + sr;
         }
         zstage(ar, ai, ky);
-        zstage(br, bi, ky + M);
+        if (ky > 0) zstage(br, bi, N1 - ky);
       }
     }
     __syncthreads();
@@ -1402,8 +1411,8 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), 4) void k_fft_up_m(const i
 // Inverse DFT of the 8 children of one target parent, component j (grid n_slots * e1),
 // evaluated at the check-surface lattice points only; Y rows are component-major
 // (Y[slot][f][8j+c] complex), so a component's 8 children are one 64-byte segment.  z stage
-// per (c, kx, ky) task straight from Y (output z < m needs P = Y[a] + Y[a+m] for even z, Q = Y[a] - Y[a+m] for odd z) into
-// LDS; then each thread runs the y stage
+// per (c, kx, ky) task straight from Y (the sums and differences over kz and N - kz) into LDS;
+// then each thread runs the y stage
 // of its own lines (c, y, z) and accumulates the c2r x sum in registers; the lattice values
 // are added into dn at the end.
 // FP64: one block per CU, so that the compiler keeps the y/z stage in registers instead of
@@ -1430,7 +1439,6 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
   const int t = threadIdx.x, yz = t % M2, cg = t / M2, y = yz % M, z = yz / M;
   if (t < N1) { twc[t] = (Real)TW.c[t]; tws[t] = (Real)TW.s[t]; }
   __syncthreads();
-  const Real sgn = (y & 1) ? Real(-1) : Real(1);
   Real acc[LPT][M];
 #pragma unroll
   for (int q = 0; q < LPT; q++)
@@ -1442,11 +1450,17 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
     const int ntask = 8 * N1 * kn;
     for (int T = t; T < ntask; T += NT) {  // z stage
       const int c = T % 8, ky = (T / 8) % N1, kl = T / (8 * N1), kx = k0 + kl;
+      // sums and differences over kz and N - kz: out[z] = Y[0] + sum of P cos + i Q sin
       Real pr_[M], pi_[M], qr_[M], qi_[M];
+      {
+        const Real* s0 = Ys + ((kx + (int64_t)NH * ky) * vg * 8 * e1 + c) * 2;
+        pr_[0] = s0[0];
+        pi_[0] = s0[1];
+      }
 #pragma unroll
-      for (int a = 0; a < M; a++) {
+      for (int a = 1; a < M; a++) {
         const Real* s0 = Ys + ((kx + (int64_t)NH * (ky + N1 * a)) * vg * 8 * e1 + c) * 2;
-        const Real* s1 = Ys + ((kx + (int64_t)NH * (ky + N1 * (a + M))) * vg * 8 * e1 + c) * 2;
+        const Real* s1 = Ys + ((kx + (int64_t)NH * (ky + N1 * (N1 - a))) * vg * 8 * e1 + c) * 2;
         const Real ur = s0[0], ui = s0[1], vr = s1[0], vi = s1[1];
         pr_[a] = ur + vr; pi_[a] = ui + vi;
         qr_[a] = ur - vr; qi_[a] = ui - vi;
@@ -1455,13 +1469,16 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
       Real* di = &s1i[c * CST + kl * PL + ky * M];
       sfor<M>([&](auto izz) __attribute__((always_inline)) {
         constexpr int zz = decltype(izz)::value;
-        Real sr = 0, si = 0;
-        sfor<M>([&](auto ia) __attribute__((always_inline)) {
-          constexpr int a = decltype(ia)::value;
-          if constexpr (zz % 2 == 0)
-            cmac_tw<N1, (a * zz) % N1, 1>(pr_[a], pi_[a], sr, si);
-          else
-            cmac_tw<N1, (a * zz) % N1, 1>(qr_[a], qi_[a], sr, si);
+        Real sr = pr_[0], si = pi_[0];
+        sfor<M - 1>([&](auto ia) __attribute__((always_inline)) {
+          constexpr int a = decltype(ia)::value + 1;
+          constexpr double wc = ct_cs((a * zz) % N1, N1, false), ws = ct_cs((a * zz) % N1, N1, true);
+          sr = fma(pr_[a], (Real)wc, sr);
+          si = fma(pi_[a], (Real)wc, si);
+          if constexpr (zz > 0) {
+            sr = fma(qi_[a], (Real)-ws, sr);
+            si = fma(qr_[a], (Real)ws, si);
+          }
         });
         dr[zz] = sr;
         di[zz] = si;
@@ -1470,23 +1487,22 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
     __syncthreads();
     for (int kl = 0; kl < kn; kl++) {  // y stage and c2r x sum of the owned lines
       const int kx = k0 + kl;
-      const Real wk = (kx == 0 || 2 * kx == N1) ? Real(1) : Real(2);
+      const Real wk = kx == 0 ? Real(1) : Real(2);
       Real sr[LPT], si[LPT];
 #pragma unroll
       for (int q = 0; q < LPT; q++) {
         const int c = cg + CG * q;
         const Real* pr = &s1r[c * CST + kl * PL + z];
         const Real* pi = &s1i[c * CST + kl * PL + z];
-        Real ar = 0, ai = 0;
+        Real ar = pr[0], ai = pi[0];
 #pragma unroll
-        for (int a = 0, e = 0; a < M; a++) {
-          const Real gr = pr[a * M] + sgn * pr[(a + M) * M];
-          const Real gi = pi[a * M] + sgn * pi[(a + M) * M];
-          const Real wc = twc[e], ws = tws[e];
-          ar += gr * wc - gi * ws;
-          ai += gr * ws + gi * wc;
+        for (int a = 1, e = 0; a < M; a++) {
           e += y;
           if (e >= N1) e -= N1;
+          const Real wc = twc[e], ws = tws[e];
+          const Real ur = pr[a * M], ui = pi[a * M], vr = pr[(N1 - a) * M], vi = pi[(N1 - a) * M];
+          ar += (ur + vr) * wc - (ui - vi) * ws;
+          ai += (ui + vi) * wc + (ur - vr) * ws;
         }
         sr[q] = wk * ar;
         si[q] = wk * ai;
@@ -2484,7 +2500,7 @@ void DeviceKernels<Real>::fft_up(hipStream_t s, int n_slots, const int32_t* firs
     default: break;
   }
 #undef PVFMM_FFT_UP_M
-  const int n1 = 2 * m;
+  const int n1 = 2 * m - 1;
   const size_t per_child = sizeof(Real) * (m * m * m + 2 * m * m + 2 * m * n1), fixed = sizeof(Real) * 2 * n1;
   const int cb = fft_children_per_block<Real>(per_child, fixed);
   const size_t lds = fixed + cb * per_child;
@@ -2605,7 +2621,7 @@ void DeviceKernels<Real>::ifft_down(hipStream_t s, int n_slots, const int32_t* f
     default: break;
   }
 #undef PVFMM_IFFT_DN_M
-  const int n1 = 2 * m;
+  const int n1 = 2 * m - 1;
   const size_t per_child = sizeof(Real) * (2 * n1 * n1 + 2 * n1 * m + 2 * m * m), fixed = sizeof(Real) * 2 * n1;
   const int cb = fft_children_per_block<Real>(per_child, fixed);
   if (cb * ns > 24 * 512) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);  // register accumulators

@@ -16,8 +16,8 @@ namespace pvfmm_amd {
 
 VGrid v_grid(int m) {
   VGrid g;
-  g.n = 2 * m;
-  g.nh = m + 1;
+  g.n = 2 * m - 1;
+  g.nh = m;
   g.M = g.n * g.n * g.nh;
   return g;
 }
