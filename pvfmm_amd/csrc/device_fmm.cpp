@@ -178,11 +178,7 @@ class DevicePlan final : public DevicePlanBase {
     };
     try {
       if (sizeof(Real) == 4 && e0_ == 1 && vt_.n > 0) {
-        // with 8 or more vectors: the 16-vector kernel (targets per wave) or, for 0, one vector
-        // at a time through the tiled kernel, compared over the whole V list (their spectra
-        // layouts differ)
-        if (vec16_ && n_vec >= 8) pick(tuning.hadamard_vec_tpw, {0, 4, 8, 16, 32}, {kPhFFT, kPhHadamard, kPhIFFT});
-        if (!use_vec16(n_vec)) pick(tuning.hadamard_tpb, {4, 8, 16, 32, 64}, {kPhHadamard});
+        pick(tuning.hadamard_tpb, {4, 8, 16, 32, 64}, {kPhHadamard});
       }
       pick(tuning.gemm_split_blocks, {0, 256, 512, 1024, 2048}, {kPhS2UGemm, kPhU2U, kPhD2D, kPhD2TGemm});
     } catch (...) {
@@ -222,6 +218,7 @@ class DevicePlan final : public DevicePlanBase {
   // kFactorRows parents (a smaller level costs less as one GEMM than as two launches);
   // lvl_seq_ = 0, 1, ... (rows of ctmp_)
   static constexpr int kFactorRows = 256;
+  static constexpr int kVListSlots = 4096;
   DBuf<int32_t> lvl_seq_;
   // the fp16 Hadamard kernels (FP32): the spectrum bound of each slot of X (or, in the adjoint,
   // of Y) and the scale of each run of tiles
@@ -243,13 +240,11 @@ class DevicePlan final : public DevicePlanBase {
   DBuf<int32_t> x_node_, x_ptr_, x_items_, x_orow_;
   int n_x_ = 0;
   // V list
-  DBuf<int32_t> v_src_fc_, v_trg_fc_, v_partner_, v_offsets_;
+  DBuf<int32_t> v_src_fc_, v_trg_fc_, v_offsets_;
   DBuf<Real> v_src_scal_, v_trg_scal_, X_, Y_;
-  // spectra of a group of 16 density vectors for the 16-vector Hadamard (FP32 scalar kernels,
-  // plans set up for 8 or more vectors): [slot][f][vector 16][16 reals]
-  DBuf<Real> Xv_, Yv_;
-  bool vec16_ = false;
-  bool use_vec16(int nv) const { return vec16_ && nv >= 8 && tuning.hadamard_vec_tpw > 0; }
+  // density vectors of one V-list pass: the spectra buffers hold that many, with these strides
+  int vlist_nv_ = 1;
+  int64_t x_vs_ = 0, y_vs_ = 0, bound_vs_ = 0;
   int n_vsrc_ = 0, n_vtrg_ = 0, n_off_ = 0;
 
   // V-list target tiles for the LDS-staged Hadamard
@@ -270,6 +265,7 @@ class DevicePlan final : public DevicePlanBase {
     hp_.bound = vbound_.p;
     hp_.run_scale = rs.p;
     hp_.run_scale_cap = (int)rs.n;
+    hp_.bound_vs = bound_vs_;
     return hp_;
   }
 
@@ -640,30 +636,27 @@ class DevicePlan final : public DevicePlanBase {
     n_vtrg_ = (int)v_trg_fc.size();
     v_src_fc_.upload(v_src_fc, &total); v_trg_fc_.upload(v_trg_fc, &total);
     v_src_scal_.upload(v_src_scal, &total); v_trg_scal_.upload(v_trg_scal, &total);
-    v_partner_.upload(v_partner, &total); v_offsets_.upload(offs, &total);
+    v_offsets_.upload(offs, &total);
     h_.v_partner = v_partner; h_.v_src_fc = v_src_fc; h_.v_trg_fc = v_trg_fc; h_.offs = offs;
     build_tiles(v_partner, n_vtrg_, n_vsrc_, vt_, &total);
+    // A V-list pass takes as many vectors as make about kVListSlots source or target parents (a
+    // parent is one block of a transform), so that a small tree's pass fills the chip; a large
+    // tree's takes one, whose spectra alone may be gigabytes.
+    vlist_nv_ = std::max(1, std::min(nvb_, kVListSlots / std::max(1, std::max(n_vsrc_, n_vtrg_))));
     if (split_) {
       // per slot and component; the adjoint's sources are the target slots
-      vbound_.alloc(std::max(1, std::max(n_vsrc_ * e0_, n_vtrg_ * e1_)), &total);
-      vrscale_.alloc(std::max(1, vt_.n), &total);
+      bound_vs_ = std::max(1, std::max(n_vsrc_ * e0_, n_vtrg_ * e1_));
+      vbound_.alloc(bound_vs_ * vlist_nv_, &total);
+      vrscale_.alloc((int64_t)std::max(1, vt_.n) * vlist_nv_, &total);
     }
     stats.v_tiles = vt_.n;
     stats.v_tile_partners = vt_.partners;
     stats.v_tile_max_partners = vt_.max_partners;
     stats.v_tile_staged = vt_.staged_delta;
-    X_.alloc((int64_t)n_vsrc_ * M_dim_ * 16 * e0_, &total);
-    Y_.alloc((int64_t)n_vtrg_ * M_dim_ * 16 * e1_, &total);
-    {
-      // 16-vector spectra when the plan batches 8 or more vectors and they fit in 64 GiB
-      const int64_t bytes = (int64_t)(n_vsrc_ + n_vtrg_) * M_dim_ * 256 * (int64_t)sizeof(Real);
-      vec16_ = std::is_same<Real, float>::value && e0_ == 1 && e1_ == 1 && nvb_ >= 8 && n_vtrg_ > 0 &&
-               bytes <= (int64_t(64) << 30);
-      if (vec16_) {
-        Xv_.alloc((int64_t)n_vsrc_ * M_dim_ * 256, &total);
-        Yv_.alloc((int64_t)n_vtrg_ * M_dim_ * 256, &total);
-      }
-    }
+    x_vs_ = (int64_t)n_vsrc_ * M_dim_ * 16 * e0_;
+    y_vs_ = (int64_t)n_vtrg_ * M_dim_ * 16 * e1_;
+    X_.alloc(x_vs_ * vlist_nv_, &total);
+    Y_.alloc(y_vs_ * vlist_nv_, &total);
 
     // ---- far field (L2T own surface + W list M2T) and U list per target leaf
     std::vector<int32_t> far_ptr{0}, far_node, u_ptr{0}, u_items;
@@ -926,7 +919,7 @@ class DevicePlan final : public DevicePlanBase {
       for (int t = 0; t < n_vtrg_; t++) fscal[t] = (Real)std::pow(2.0, ki.src_scal * (h_.vtrg_depth[t] + 1));
       a->n_vt = (int)fc.size();
       build_tiles(partner, a->n_vt, n_vtrg_, a->vt, &total);
-      if (split_) a->vrscale.alloc(std::max(1, a->vt.n), &total);
+      if (split_) a->vrscale.alloc((int64_t)std::max(1, a->vt.n) * vlist_nv_, &total);
       a->v_fc.upload(fc, &total);
       a->fft_scal.upload(fscal, &total);
       a->ifft_scal.upload(iscal, &total);
@@ -990,14 +983,15 @@ class DevicePlan final : public DevicePlanBase {
                    gemm_work_elems_, sp, nv, dn_vs_, eq_vs_);
     // V list^T: the M2L of offset -R from the target parents' children to the source parents'
     // (the spectra buffers swap roles: Y_ holds the new sources, X_ the new targets)
-    for (int v = 0; v < nv; v++) {
-      K::fft_up(st_, n_vtrg_, v_trg_fc_.p, dn_.p + v * dn_vs_, K1_, e1_, m_, ops_->lattice.p, ops_->lattice_inv.p, a.fft_scal.p, Y_.p,
-                1, 0, split_ ? vbound_.p : nullptr);
+    for (int v = 0; v < nv; v += vlist_nv_) {
+      const int g = std::min(vlist_nv_, nv - v);
+      K::fft_up(st_, n_vtrg_, v_trg_fc_.p, dn_.p + v * dn_vs_, K1_, e1_, m_, ops_->lattice.p, ops_->lattice_inv.p, a.fft_scal.p,
+                Y_.p, split_ ? vbound_.p : nullptr, g, dn_vs_, y_vs_, bound_vs_);
       K::hadamard_tiled(st_, a.vt.n, M_dim_, e0_, e1_, n_off_, a.vt.t0.p, a.vt.u0.p, a.vt.usrc.p, a.vt.d0.p, a.vt.dent.p,
                         a.vt.uidx.p, a.vt.gmask.p, v_offsets_.p, ops_->V.p, Y_.p, X_.p, tuning.hadamard_tpb,
-                        split_ ? &hparts(a.vrscale) : nullptr);
+                        split_ ? &hparts(a.vrscale) : nullptr, g, y_vs_, x_vs_);
       K::ifft_down(st_, a.n_vt, a.v_fc.p, X_.p, eq_.p + v * eq_vs_, K0_, e0_, m_, ops_->lattice.p, ops_->lattice_inv.p, ns_,
-                   a.ifft_scal.p);
+                   a.ifft_scal.p, g, x_vs_, eq_vs_);
     }
     // (X list S2L)^T: downward check surfaces (RAD0) -> source points
     K::far_points(st_, ek, a.n_x, a.x_leaf.p, a.x_ptr.p, a.x_node.p, a.x_den.p, a.x_rad.p, a.sb.p, a.se.p,
@@ -1081,34 +1075,26 @@ class DevicePlan final : public DevicePlanBase {
     K::p2p_surface(st_, ek, n_x_, x_node_.p, x_ptr_.p, x_items_.p, src_begin_.p, src_end_.p, center_.p, node_size_.p, kRad0,
                    ops_->unit_surf.p, ns_, sx_.p, sden_.p, n_src_, dn_.p, x_orow_.p, K1_, true, nv, den_vs, dn_vs_);
     mark(5);
-    // V list: groups of 16 vectors through the 16-vector Hadamard, or one vector at a time
-    // through the spectra buffers (with several passes the three sub-phases are timed per
-    // pass and summed)
-    const bool grouped = use_vec16(nv);
-    const int n_pass = grouped ? (nv + 15) / 16 : nv;
-    if (timing_ && n_pass > 1) ensure_vlist_events(n_pass);
-    for (int g = 0; g < n_pass; g++) {
-      const bool sub = timing_ && n_pass > 1;
-      const int v0 = grouped ? 16 * g : g, gn = grouped ? std::min(16, nv - v0) : 1;
-      if (sub) HIP_CHECK(hipEventRecord(vev_[4 * g], st_));
-      for (int v = v0; v < v0 + gn; v++)
-        K::fft_up(st_, n_vsrc_, v_src_fc_.p, eq_.p + v * eq_vs_, K0_, e0_, m_, ops_->lattice.p, ops_->lattice_inv.p, v_src_scal_.p,
-                  grouped ? Xv_.p : X_.p, grouped ? 16 : 1, grouped ? v - v0 : 0,
-                  split_ && !grouped ? vbound_.p : nullptr);
-      if (sub) HIP_CHECK(hipEventRecord(vev_[4 * g + 1], st_));
+    // V list: passes of up to vlist_nv_ vectors through the spectra buffers (with several passes
+    // the three sub-phases are timed per pass and summed)
+    const int n_pass = (nv + vlist_nv_ - 1) / vlist_nv_;
+    const bool sub = timing_ && n_pass > 1;
+    if (sub) ensure_vlist_events(n_pass);
+    for (int p = 0; p < n_pass; p++) {
+      const int v = p * vlist_nv_, g = std::min(vlist_nv_, nv - v);
+      if (sub) HIP_CHECK(hipEventRecord(vev_[4 * p], st_));
+      K::fft_up(st_, n_vsrc_, v_src_fc_.p, eq_.p + v * eq_vs_, K0_, e0_, m_, ops_->lattice.p, ops_->lattice_inv.p, v_src_scal_.p,
+                X_.p, split_ ? vbound_.p : nullptr, g, eq_vs_, x_vs_, bound_vs_);
+      if (sub) HIP_CHECK(hipEventRecord(vev_[4 * p + 1], st_));
       if (n_pass == 1) mark(6);
-      if (grouped)
-        K::hadamard_vec16(st_, n_vtrg_, M_dim_, v_partner_.p, ops_->vb(), Xv_.p, Yv_.p, tuning.hadamard_vec_tpw);
-      else
-        K::hadamard_tiled(st_, vt_.n, M_dim_, e0_, e1_, n_off_, vt_.t0.p, vt_.u0.p, vt_.usrc.p, vt_.d0.p, vt_.dent.p,
-                          vt_.uidx.p, vt_.gmask.p, v_offsets_.p, ops_->V.p, X_.p, Y_.p, tuning.hadamard_tpb,
-                          split_ ? &hparts(vrscale_) : nullptr);
-      if (sub) HIP_CHECK(hipEventRecord(vev_[4 * g + 2], st_));
+      K::hadamard_tiled(st_, vt_.n, M_dim_, e0_, e1_, n_off_, vt_.t0.p, vt_.u0.p, vt_.usrc.p, vt_.d0.p, vt_.dent.p,
+                        vt_.uidx.p, vt_.gmask.p, v_offsets_.p, ops_->V.p, X_.p, Y_.p, tuning.hadamard_tpb,
+                        split_ ? &hparts(vrscale_) : nullptr, g, x_vs_, y_vs_);
+      if (sub) HIP_CHECK(hipEventRecord(vev_[4 * p + 2], st_));
       if (n_pass == 1) mark(7);
-      for (int v = v0; v < v0 + gn; v++)
-        K::ifft_down(st_, n_vtrg_, v_trg_fc_.p, grouped ? Yv_.p : Y_.p, dn_.p + v * dn_vs_, K1_, e1_, m_, ops_->lattice.p,
-                     ops_->lattice_inv.p, ns_, v_trg_scal_.p, grouped ? 16 : 1, grouped ? v - v0 : 0);
-      if (sub) HIP_CHECK(hipEventRecord(vev_[4 * g + 3], st_));
+      K::ifft_down(st_, n_vtrg_, v_trg_fc_.p, Y_.p, dn_.p + v * dn_vs_, K1_, e1_, m_, ops_->lattice.p, ops_->lattice_inv.p, ns_,
+                   v_trg_scal_.p, g, y_vs_, dn_vs_);
+      if (sub) HIP_CHECK(hipEventRecord(vev_[4 * p + 3], st_));
     }
     if (n_pass > 1) {
       mark(6);

@@ -139,19 +139,6 @@ class DeviceOps final : public DeviceOpsBase {
 
   int64_t bytes() const override { return bytes_; }
 
-  // Three bf16 parts of the transfer blocks (FP32 scalar kernels), for the 16-vector Hadamard
-  const uint16_t* vb() {
-    std::lock_guard<std::mutex> lock(mutex_);
-    if (!Vb_.p) {
-      Stream st;
-      DBuf<double> G;
-      spectra(st.s, G);
-      Vb_.alloc((int64_t)13 * grid.M * 3 * 512, &bytes_);
-      transfer_bf16(st.s, grid.M, G.p, Vb_.p);
-      HIP_CHECK(hipStreamSynchronize(st.s));
-    }
-    return Vb_.p;
-  }
   // Boundary operator of a periodic boundary type (K0 x K1), and transposed
   const Real* bc(int bndry, bool transposed) {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -214,7 +201,6 @@ class DeviceOps final : public DeviceOpsBase {
   const Operators& O_;
   int64_t bytes_ = 0;
   std::mutex mutex_;
-  DBuf<uint16_t> Vb_;
   DBuf<Real> bc_[2][4];
   std::unique_ptr<Transposed> tr_;
 };

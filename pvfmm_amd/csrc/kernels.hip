@@ -9,8 +9,8 @@
 //    contiguously so a parent row is one 8*K row of the child block), on MFMA.
 //  * V list: pruned separable DFT of the m^3 surface lattice embedded in the (2m-1)^3 grid,
 //    one x-frequency slice at a time in LDS; a tiled frequency-domain Hadamard sum over the 26
-//    parent offsets on the matrix cores (FP32 scalar kernels on the bf16 cores with exact
-//    three-way operand splits); the inverse DFT evaluates only the check-surface points.
+//    parent offsets on the matrix cores (FP32 on the fp16 cores with two-way operand splits);
+//    the inverse DFT evaluates only the check-surface points.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -923,11 +923,12 @@ __device__ void init_twiddles(Real* twr, Real* twi, int n1, double sign) {
 template <typename Real>
 __global__ __launch_bounds__(512) void k_fft_up(const int32_t* __restrict__ first_child, const Real* __restrict__ up, int K0, int e0,
                                                 int m, int CB, const int32_t* __restrict__ lattice, const Real* __restrict__ scal,
-                                                Real* __restrict__ X, int vg, int vi) {
+                                                Real* __restrict__ X, int64_t up_vs, int64_t x_vs) {
   extern __shared__ unsigned char smem_raw[];
   Real* sm = reinterpret_cast<Real*>(smem_raw);
   const int n1 = 2 * m - 1, nh = m, M_dim = n1 * n1 * nh, ns = 6 * (m - 1) * (m - 1) + 2;
   const int m2 = m * m, m3 = m2 * m, mn = m * n1;
+  up += blockIdx.y * up_vs;        // density vector
   Real* cube = sm;                 // CB * m^3
   Real* twr = cube + CB * m3;      // n1
   Real* twi = twr + n1;
@@ -949,7 +950,7 @@ __global__ __launch_bounds__(512) void k_fft_up(const int32_t* __restrict__ firs
     cube[c * m3 + (z * m + y) * m + x] = up[(int64_t)(fc + c) * K0 + p * e0 + i] * sc;
   }
   __syncthreads();
-  Real* Xs = X + (((int64_t)slot * M_dim * vg + vi) * 8 * e0 + 8 * i + c0) * 2;
+  Real* Xs = X + blockIdx.y * x_vs + ((int64_t)slot * M_dim * 8 * e0 + 8 * i + c0) * 2;
   for (int kx = 0; kx < nh; kx++) {
     for (int o = tid; o < CB * m2; o += nt) {  // x: real -> complex
       const Real* line = &cube[(o / m2) * m3 + (o % m2) * m];
@@ -985,7 +986,7 @@ __global__ __launch_bounds__(512) void k_fft_up(const int32_t* __restrict__ firs
         ai += vr[z * n1] * twi[e] + vi[z * n1] * twr[e];
       }
       const int64_t f = kx + nh * (ky + n1 * kz);
-      Real* d = Xs + (f * vg * 8 * e0 + c) * 2;
+      Real* d = Xs + (f * 8 * e0 + c) * 2;
       d[0] = ar;
       d[1] = ai;
     }
@@ -1002,7 +1003,7 @@ template <typename Real>
 __global__ __launch_bounds__(512) void k_ifft_down(const int32_t* __restrict__ first_child, const Real* __restrict__ Y,
                                                    Real* __restrict__ dn, int K1, int e1, int m, int CB,
                                                    const int32_t* __restrict__ lattice, int ns, const Real* __restrict__ scal,
-                                                   int vg, int vi) {
+                                                   int64_t y_vs, int64_t dn_vs) {
   extern __shared__ unsigned char smem_raw[];
   Real* sm = reinterpret_cast<Real*>(smem_raw);
   const int n1 = 2 * m - 1, nh = m, M_dim = n1 * n1 * nh;
@@ -1024,13 +1025,14 @@ __global__ __launch_bounds__(512) void k_ifft_down(const int32_t* __restrict__ f
   Real acc[MAXQ];
 #pragma unroll
   for (int q = 0; q < MAXQ; q++) acc[q] = 0;
-  const Real* Ys = Y + (((int64_t)slot * M_dim * vg + vi) * 8 * e1 + 8 * j + c0) * 2;
+  dn += blockIdx.y * dn_vs;  // density vector
+  const Real* Ys = Y + blockIdx.y * y_vs + ((int64_t)slot * M_dim * 8 * e1 + 8 * j + c0) * 2;
   __syncthreads();
   for (int kx = 0; kx < nh; kx++) {
     for (int o = tid; o < CB * nn; o += nt) {  // children fastest: contiguous rows of Y
       const int c = o % CB, q = o / CB;         // q = ky + n1*kz
       const int64_t f = kx + (int64_t)nh * q;
-      const Real* src = Ys + (f * vg * 8 * e1 + c) * 2;
+      const Real* src = Ys + (f * 8 * e1 + c) * 2;
       yr[c * nn + q] = src[0];
       yi[c * nn + q] = src[1];
     }
@@ -1159,10 +1161,13 @@ __device__ __forceinline__ void cs_tw(Real gr, Real gi, Real& cr, Real& ci, Real
 template <typename Real>
 __global__ __launch_bounds__(256) void k_spectrum_bound(int n_slots, const int32_t* __restrict__ first_child,
                                                         const Real* __restrict__ up, int K0, int e0, int ns,
-                                                        const Real* __restrict__ scal, float* __restrict__ bound) {
+                                                        const Real* __restrict__ scal, float* __restrict__ bound,
+                                                        int64_t up_vs, int64_t bound_vs) {
   __shared__ Real red[256];
   const int slot = blockIdx.x, t = threadIdx.x;
   if (slot >= n_slots) return;  // whole block
+  up += blockIdx.y * up_vs;
+  bound += blockIdx.y * bound_vs;
   const int fc = first_child[slot];
   for (int i = 0; i < e0; i++) {
     Real a = 0;
@@ -1186,9 +1191,10 @@ __global__ __launch_bounds__(256) void k_spectrum_bound(int n_slots, const int32
 __global__ __launch_bounds__(256) void k_run_scale(int n_tiles, int tpb, const int32_t* __restrict__ tile_u0,
                                                    const int32_t* __restrict__ usrc, const int32_t* __restrict__ tile_d0,
                                                    const int32_t* __restrict__ dent, const float* __restrict__ bound,
-                                                   float* __restrict__ run_scale) {
+                                                   float* __restrict__ run_scale, int64_t bound_vs) {
   __shared__ float red[256];
   const int r = blockIdx.x, t = threadIdx.x, k0 = r * tpb, k1 = min(n_tiles, k0 + tpb);
+  bound += blockIdx.y * bound_vs;  // density vector
   float mx = 0.f;
   for (int u = tile_u0[k0] + t; u < tile_u0[k0 + 1]; u += 256) mx = fmaxf(mx, bound[usrc[u] >> 9]);
   if (k0 + 1 < k1)
@@ -1207,7 +1213,7 @@ __global__ __launch_bounds__(256) void k_run_scale(int n_tiles, int tpb, const i
       (void)frexpf(b, &e);  // b < 2^e
       sc = ldexpf(1.f, min(100, max(-100, 14 - e)));
     }
-    run_scale[r] = sc;
+    run_scale[blockIdx.y * gridDim.x + r] = sc;
   }
 }
 
@@ -1258,7 +1264,8 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_
                                                                          const Real* __restrict__ up, int K0, int e0,
                                                                          const int32_t* __restrict__ lat_inv,
                                                                          const Real* __restrict__ scal, Real* __restrict__ X,
-                                                                         int n_slots, int vg, int vi, float* __restrict__ bound) {
+                                                                         int n_slots, float* __restrict__ bound, int64_t up_vs,
+                                                                         int64_t x_vs, int64_t bound_vs) {
   using S = DftShape<Real, M>;
   constexpr int N1 = S::N1, NH = S::NH, MD = S::MD, M2 = S::M2, NT = S::NT, LPT = S::LPT, CG = S::CG, KC = S::KC_UP;
   constexpr int CST = KC * M2 + 1;  // child stride (odd, spreads the children over LDS banks)
@@ -1270,6 +1277,7 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_
   const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
   const int i = local % e0, slot = (local / e0) * 8 + xcd;
   if (slot >= n_slots) return;  // whole block
+  up += blockIdx.y * up_vs;  // density vector
   const int fc = first_child[slot];
   const Real sc = scal[slot];
   const int t = threadIdx.x, yz = t % M2, cg = t / M2, y = yz % M, z = yz / M;
@@ -1297,11 +1305,11 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_
       for (int u = t; u < NT; u += 64) b += s1r[u];
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) b += __shfl_xor(b, o);
-      if (t == 0) bound[(int64_t)slot * e0 + i] = (float)b;
+      if (t == 0) bound[blockIdx.y * bound_vs + (int64_t)slot * e0 + i] = (float)b;
     }
   }
   __syncthreads();
-  Real* Xs = X + (((int64_t)slot * MD * vg + vi) * 8 * e0 + 8 * i) * 2;
+  Real* Xs = X + blockIdx.y * x_vs + ((int64_t)slot * MD * 8 * e0 + 8 * i) * 2;
   for (int k0 = 0; k0 < NH; k0 += KC) {
     const int kn = (NH - k0 < KC) ? NH - k0 : KC;
 #pragma unroll
@@ -1333,7 +1341,7 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_
         // out of the unrolled loop (they would not fit in registers for FP64)
         Real* xb = Xs;
         asm volatile("" : "+s"(xb));
-        Real* d = xb + (f * vg * 8 * e0 + c) * 2;
+        Real* d = xb + (f * 8 * e0 + c) * 2;
         if constexpr (NTS) {
           __builtin_nontemporal_store(re, &d[0]);
           __builtin_nontemporal_store(im, &d[1]);
@@ -1421,8 +1429,8 @@ template <typename Real, int M>
 __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4)) void k_ifft_down_m(const int32_t* __restrict__ first_child,
                                                                             const Real* __restrict__ Y, Real* __restrict__ dn,
                                                                             int K1, int e1, const int32_t* __restrict__ lat_inv,
-                                                                            const Real* __restrict__ scal, int n_slots, int vg,
-                                                                            int vi) {
+                                                                            const Real* __restrict__ scal, int n_slots,
+                                                                            int64_t y_vs, int64_t dn_vs) {
   using S = DftShape<Real, M>;
   constexpr int N1 = S::N1, NH = S::NH, MD = S::MD, M2 = S::M2, NT = S::NT, LPT = S::LPT, CG = S::CG, KC = S::KC_DN;
   constexpr int PL = N1 * M;         // one plane of one child: [ky][z]
@@ -1444,7 +1452,8 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
   for (int q = 0; q < LPT; q++)
 #pragma unroll
     for (int x = 0; x < M; x++) acc[q][x] = 0;
-  const Real* Ys = Y + (((int64_t)slot * MD * vg + vi) * 8 * e1 + 8 * j) * 2;
+  dn += blockIdx.y * dn_vs;  // density vector
+  const Real* Ys = Y + blockIdx.y * y_vs + ((int64_t)slot * MD * 8 * e1 + 8 * j) * 2;
   for (int k0 = 0; k0 < NH; k0 += KC) {
     const int kn = (NH - k0 < KC) ? NH - k0 : KC;
     const int ntask = 8 * N1 * kn;
@@ -1453,14 +1462,14 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
       // sums and differences over kz and N - kz: out[z] = Y[0] + sum of P cos + i Q sin
       Real pr_[M], pi_[M], qr_[M], qi_[M];
       {
-        const Real* s0 = Ys + ((kx + (int64_t)NH * ky) * vg * 8 * e1 + c) * 2;
+        const Real* s0 = Ys + ((kx + (int64_t)NH * ky) * 8 * e1 + c) * 2;
         pr_[0] = s0[0];
         pi_[0] = s0[1];
       }
 #pragma unroll
       for (int a = 1; a < M; a++) {
-        const Real* s0 = Ys + ((kx + (int64_t)NH * (ky + N1 * a)) * vg * 8 * e1 + c) * 2;
-        const Real* s1 = Ys + ((kx + (int64_t)NH * (ky + N1 * (N1 - a))) * vg * 8 * e1 + c) * 2;
+        const Real* s0 = Ys + ((kx + (int64_t)NH * (ky + N1 * a)) * 8 * e1 + c) * 2;
+        const Real* s1 = Ys + ((kx + (int64_t)NH * (ky + N1 * (N1 - a))) * 8 * e1 + c) * 2;
         const Real ur = s0[0], ui = s0[1], vr = s1[0], vi = s1[1];
         pr_[a] = ur + vr; pi_[a] = ui + vi;
         qr_[a] = ur - vr; qi_[a] = ui - vi;
@@ -1562,7 +1571,7 @@ __global__ __launch_bounds__(256, (hadamard_blocks_per_cu<Real, E0, FB, UMAX>())
                                                         const uint16_t* __restrict__ uidx, const uint32_t* __restrict__ gmask,
                                                         const int32_t* __restrict__ offsets,
                                                         const Real* __restrict__ Vp, const Real* __restrict__ X,
-                                                        Real* __restrict__ Y) {
+                                                        Real* __restrict__ Y, int64_t x_vs, int64_t y_vs) {
   using MF = Mfma<Real>;
   using V4 = typename MF::V4;
   constexpr int NOFF = 26;                        // V1 parent offsets
@@ -1583,6 +1592,8 @@ __global__ __launch_bounds__(256, (hadamard_blocks_per_cu<Real, E0, FB, UMAX>())
   const int fg = (local / n_tiles) * 8 + xcd, tile = local % n_tiles;
   const int f0 = fg * FB;
   if (f0 >= M_dim) return;  // whole block
+  X += blockIdx.y * x_vs;  // density vector
+  Y += blockIdx.y * y_vs;
   const int t0 = tile_t0[tile], nt = tile_t0[tile + 1] - t0;
   const int u0 = tile_u0[tile], nu = tile_u0[tile + 1] - u0;
   const int fn = min(FB, M_dim - f0);
@@ -1779,11 +1790,6 @@ __global__ __launch_bounds__(256, (hadamard_blocks_per_cu<Real, E0, FB, UMAX>())
       }
 }
 
-// The three bf16 parts of an FP32 value x = x0 + x1 + x2 (x0 the top 8 significant bits, x1
-// the next 8, x2 the rest; each step exact): the operand split of k_hadamard_vec16, whose six
-// largest products x0 t0 + (x0 t1 + x1 t0) + (x0 t2 + x1 t1 + x2 t0) leave out less than
-// 2^-21 |x t| (transfer parts rounded to nearest: |t1| <= 2^-8 |t|, |t2| <= 2^-16 |t|).
-//
 // FP32 frequency-domain M2L for the scalar kernels (k_hadamard_split) on the fp16 matrix
 // cores: operands are scaled by powers of two into fp16 range and split exactly into two fp16
 // parts x = x0 + x1 (x0 = RN(x), x1 = RN(x - x0): 22 significant bits, |x - x0 - x1| <=
@@ -1810,25 +1816,10 @@ __global__ __launch_bounds__(256, (hadamard_blocks_per_cu<Real, E0, FB, UMAX>())
 // tiles list stays in its slot, so after the run's first tile only the partners new since the
 // previous tile are read and staged, into slots that the previous tile does not read (the host
 // assigns the slots).  Staging passes past the length of that list are skipped.
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSplitPool = 496;
-
-// the three bf16 parts of an FP32 value, by truncation (each step exact), as the high halves
-// of three words
-__device__ __forceinline__ void split3(float x, uint32_t& h0, uint32_t& h1, uint32_t& h2) {
-  const uint32_t u0 = __float_as_uint(x);
-  h0 = u0 & 0xFFFF0000u;
-  const float r1 = x - __uint_as_float(h0);
-  const uint32_t u1 = __float_as_uint(r1);
-  h1 = u1 & 0xFFFF0000u;
-  const float r2 = r1 - __uint_as_float(h1);
-  h2 = __float_as_uint(r2) & 0xFFFF0000u;  // at most 8 significant bits: exact
-}
-// two bf16 (the high halves of a and b, low halves zero) packed into one word, a in the low half
-__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) { return (a >> 16) | b; }
 
 template <int UMAX, int POOL>
 __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tiles, int tiles_per_block, int n_chunks,
@@ -1838,7 +1829,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
                                                           const uint16_t* __restrict__ uidx, const uint32_t* __restrict__ gmask,
                                                           const uint16_t* __restrict__ Vh, const float* __restrict__ tinv,
                                                           const float* __restrict__ run_scale, const float* __restrict__ X,
-                                                          float* __restrict__ Y) {
+                                                          float* __restrict__ Y, int64_t x_vs, int64_t y_vs) {
   constexpr int NOFF = 26, NPAIR = NOFF / 2;
   constexpr int RW = 16;                  // reals per staged entry and frequency
   constexpr int EST = 2 * RW / 2 + 4;     // words per staged entry: 2 parts x 16 fp16, padded
@@ -1861,6 +1852,8 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
   const int f = ((lp / n_chunks) * 8 + xcd) * 2 + (local & 1), chunk = lp % n_chunks;
   const int k0 = chunk * tiles_per_block, k1 = min(n_tiles, k0 + tiles_per_block);
   if (f >= M_dim || k0 >= k1) return;  // whole block
+  X += blockIdx.y * x_vs;  // density vector
+  Y += blockIdx.y * y_vs;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
   const int row = l & 15, kg = l >> 4;
   const int pa = kg >> 1;                   // the lane's offset within a pair (k = 16 pa + ...)
@@ -1876,7 +1869,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
     for (int p = 0; p < 2; p++)
       bq[j][p] = *reinterpret_cast<const halfx8*>(Vh + ((((int64_t)j * 2 + p) * M_dim + f) * 64 + l) * 8);
   // the run's scale, and the factor that undoes both scales
-  const float xsc = run_scale[chunk], ysc = tinv[f] / xsc;
+  const float xsc = run_scale[blockIdx.y * n_chunks + chunk], ysc = tinv[f] / xsc;
   for (int e = tid; e < EST; e += 256) Xl[POOL * EST + e] = 0u;
   const int nk = k1 - k0;
   for (int i = tid; i < 4 * nk; i += 256) m_g[i] = gmask[4 * k0 + i];
@@ -2041,7 +2034,8 @@ __global__ __launch_bounds__(256, 1) void k_hadamard_split3(int M_dim, int n_til
                                                            const int32_t* __restrict__ usrc, const uint16_t* __restrict__ uidx,
                                                            const uint32_t* __restrict__ gmask, const uint16_t* __restrict__ Vh,
                                                            const float* __restrict__ tinv, const float* __restrict__ bound,
-                                                           const float* __restrict__ X, float* __restrict__ Y) {
+                                                           const float* __restrict__ X, float* __restrict__ Y, int64_t x_vs,
+                                                           int64_t y_vs, int64_t bound_vs) {
   constexpr int NOFF = 26, NPAIR = NOFF / 2, RW = 48;
   constexpr int NB = 3, NCH = 3;          // output tiles of 16 reals, K chunks of a pair
   constexpr int EST = 52;                 // words per staged entry: 2 parts x 24 words, padded
@@ -2058,6 +2052,9 @@ __global__ __launch_bounds__(256, 1) void k_hadamard_split3(int M_dim, int n_til
   const int fp = (local / (2 * n_tiles)) * 8 + xcd, rem = local % (2 * n_tiles);
   const int tile = rem >> 1, f = 2 * fp + (rem & 1);
   if (f >= M_dim) return;  // whole block
+  X += blockIdx.y * x_vs;  // density vector
+  Y += blockIdx.y * y_vs;
+  bound += blockIdx.y * bound_vs;
   const int t0 = tile_t0[tile], nt = tile_t0[tile + 1] - t0;
   const int u0 = tile_u0[tile], nu = tile_u0[tile + 1] - u0;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, row = l & 15, kg = l >> 4;
@@ -2175,72 +2172,6 @@ __global__ __launch_bounds__(256, 1) void k_hadamard_split3(int M_dim, int n_til
       const int tg = 16 * w + 4 * kg + r;
       if (tg < nt) Y[((int64_t)(t0 + tg) * M_dim + f) * RW + 16 * nb + row] = s[r] * ysc;
     }
-  }
-}
-
-// The same products for 16 density vectors of one tree at once: the MFMA rows are the 16
-// vectors of one target (instead of 16 targets of one vector), so the 16 rows of an operand
-// read one partner's spectra, 16 consecutive 64-byte rows of X in the vector-group layout
-// [slot][f][vector 16][16 reals]; no partner table, no padding of absent partners and no LDS
-// staging are needed, the loads are whole 1 KiB blocks straight from L2.  A block owns one
-// frequency (its transfer-block parts in registers) and 4 waves; wave w computes targets
-// [t0 + w tpw, t0 + (w + 1) tpw) in turn, over the 13 offset pairs each, absent partners
-// read as zero.
-template <int NPAIR>
-__global__ __launch_bounds__(256, 2) void k_hadamard_vec16(int M_dim, int n_trg, int tpw, int n_chunks,
-                                                          const int32_t* __restrict__ partner, const uint16_t* __restrict__ Vb,
-                                                          const float* __restrict__ X, float* __restrict__ Y) {
-  constexpr int NOFF = 2 * NPAIR;
-  // all target chunks of one frequency run on one XCD, back to back (block b runs on XCD b mod
-  // 8), so the partners' spectra at that frequency are read into that XCD's L2 once and served
-  // from there to every target that lists them
-  const int b = blockIdx.x, xcd = b & 7, local = b >> 3;
-  const int chunk = local % n_chunks, f = (local / n_chunks) * 8 + xcd;
-  if (f >= M_dim) return;  // whole block
-  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
-  const int row = l & 15, kg = l >> 4, pa = kg >> 1, half = kg & 1;
-  bf16x8 bq[NPAIR][3];
-#pragma unroll
-  for (int j = 0; j < NPAIR; j++)
-#pragma unroll
-    for (int p = 0; p < 3; p++)
-      bq[j][p] = *reinterpret_cast<const bf16x8*>(Vb + ((((int64_t)j * 3 + p) * M_dim + f) * 64 + l) * 8);
-  const int t_begin = (chunk * 4 + w) * tpw, t_end = min(n_trg, t_begin + tpw);
-  for (int t = t_begin; t < t_end; t++) {
-    const int32_t* pt = partner + (int64_t)t * NOFF;
-    floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < NPAIR; j++) {
-      const int sl = pt[2 * j + pa];
-      floatx4 v0 = {0.f, 0.f, 0.f, 0.f}, v1 = {0.f, 0.f, 0.f, 0.f};
-      if (sl >= 0) {
-        const float* src = X + (((int64_t)sl * M_dim + f) * 16 + row) * 16 + 8 * half;
-        v0 = *reinterpret_cast<const floatx4*>(src);
-        v1 = *reinterpret_cast<const floatx4*>(src + 4);
-      }
-      uint32_t h[3][8];
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        split3(v0[q], h[0][q], h[1][q], h[2][q]);
-        split3(v1[q], h[0][q + 4], h[1][q + 4], h[2][q + 4]);
-      }
-      bf16x8 a[3];
-#pragma unroll
-      for (int p = 0; p < 3; p++) {
-        const u32x4 wd = {pack_hi(h[p][0], h[p][1]), pack_hi(h[p][2], h[p][3]), pack_hi(h[p][4], h[p][5]),
-                          pack_hi(h[p][6], h[p][7])};
-        a[p] = __builtin_bit_cast(bf16x8, wd);
-      }
-      acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], bq[j][0], acc1, 0, 0, 0);
-      acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], bq[j][0], acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], bq[j][1], acc1, 0, 0, 0);
-      acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bq[j][1], acc0, 0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bq[j][2], acc1, 0, 0, 0);
-      acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], bq[j][0], acc0, 0, 0, 0);
-    }
-    const floatx4 sum = acc0 + acc1;
-#pragma unroll
-    for (int r = 0; r < 4; r++) Y[(((int64_t)t * M_dim + f) * 16 + 4 * kg + r) * 16 + row] = sum[r];
   }
 }
 
@@ -2476,19 +2407,18 @@ static int fft_children_per_block(size_t per_child, size_t fixed) {
 
 template <typename Real>
 void DeviceKernels<Real>::fft_up(hipStream_t s, int n_slots, const int32_t* first_child, const Real* up, int K0, int e0, int m,
-                                 const int32_t* lattice, const int32_t* lat_inv, const Real* scal, Real* X, int vg, int vi,
-                                 float* bound) {
-  if (n_slots == 0) return;
-  if (bound && vg != 1) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
-  const dim3 g((unsigned)((n_slots + 7) / 8 * 8 * e0));  // whole XCD rounds of slots
+                                 const int32_t* lattice, const int32_t* lat_inv, const Real* scal, Real* X, float* bound, int nv,
+                                 int64_t up_vs, int64_t x_vs, int64_t bound_vs) {
+  if (n_slots == 0 || nv <= 0) return;
+  const dim3 g((unsigned)((n_slots + 7) / 8 * 8 * e0), nv);  // whole XCD rounds of slots
 #define PVFMM_FFT_UP_M(MM)                                                                                        \
   case MM:                                                                                                        \
-    if (e0 == 1 && vg == 1)                                                                                       \
+    if (e0 == 1)                                                                                                  \
       hipLaunchKernelGGL((k_fft_up_m<Real, MM, true>), g, dim3(DftShape<Real, MM>::NT), 0, s, first_child, up, K0, e0, \
-                         lat_inv, scal, X, n_slots, vg, vi, bound);                                               \
+                         lat_inv, scal, X, n_slots, bound, up_vs, x_vs, bound_vs);                               \
     else                                                                                                          \
       hipLaunchKernelGGL((k_fft_up_m<Real, MM, false>), g, dim3(DftShape<Real, MM>::NT), 0, s, first_child, up, K0, e0, \
-                         lat_inv, scal, X, n_slots, vg, vi, bound);                                               \
+                         lat_inv, scal, X, n_slots, bound, up_vs, x_vs, bound_vs);                               \
     HIP_LAUNCH_CHECK();                                                                                           \
     return;
   switch (m) {
@@ -2504,12 +2434,12 @@ void DeviceKernels<Real>::fft_up(hipStream_t s, int n_slots, const int32_t* firs
   const size_t per_child = sizeof(Real) * (m * m * m + 2 * m * m + 2 * m * n1), fixed = sizeof(Real) * 2 * n1;
   const int cb = fft_children_per_block<Real>(per_child, fixed);
   const size_t lds = fixed + cb * per_child;
-  hipLaunchKernelGGL(k_fft_up<Real>, dim3(n_slots * e0 * (8 / cb)), dim3(512), lds, s, first_child, up, K0, e0, m, cb, lattice,
-                     scal, X, vg, vi);
+  hipLaunchKernelGGL(k_fft_up<Real>, dim3(n_slots * e0 * (8 / cb), nv), dim3(512), lds, s, first_child, up, K0, e0, m, cb,
+                     lattice, scal, X, up_vs, x_vs);
   HIP_LAUNCH_CHECK();
   if (bound) {
-    hipLaunchKernelGGL(k_spectrum_bound<Real>, dim3(n_slots), dim3(256), 0, s, n_slots, first_child, up, K0, e0,
-                       6 * (m - 1) * (m - 1) + 2, scal, bound);
+    hipLaunchKernelGGL(k_spectrum_bound<Real>, dim3(n_slots, nv), dim3(256), 0, s, n_slots, first_child, up, K0, e0,
+                       6 * (m - 1) * (m - 1) + 2, scal, bound, up_vs, bound_vs);
     HIP_LAUNCH_CHECK();
   }
 }
@@ -2533,8 +2463,8 @@ void DeviceKernels<Real>::hadamard_tiled(hipStream_t s, int n_tiles, int M_dim, 
                                          const int32_t* tile_u0, const int32_t* usrc, const int32_t* tile_d0,
                                          const int32_t* dent, const uint16_t* uidx, const uint32_t* gmask,
                                          const int32_t* offsets, const Real* Vp, const Real* X, Real* Y, int tiles_per_block,
-                                         const HadamardParts* hp) {
-  if (n_tiles == 0) return;
+                                         const HadamardParts* hp, int nv, int64_t x_vs, int64_t y_vs) {
+  if (n_tiles == 0 || nv <= 0) return;
   if (n_off != 26) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);  // the 26 V1 parent offsets
   constexpr int FB = sizeof(Real) == 4 ? 4 : 2;
   const int n_fg = (M_dim + FB - 1) / FB;
@@ -2548,18 +2478,19 @@ void DeviceKernels<Real>::hadamard_tiled(hipStream_t s, int n_tiles, int M_dim, 
       const int TPB = std::min(64, std::max(1, tiles_per_block));
       const int n_chunks = (n_tiles + TPB - 1) / TPB;
       const int64_t nbs = (int64_t)n_chunks * ((M_dim + 15) / 16) * 16;
-      if (nbs >= (1ll << 31) || n_chunks > hp->run_scale_cap) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
-      hipLaunchKernelGGL(k_run_scale, dim3((unsigned)n_chunks), dim3(256), 0, s, n_tiles, TPB, tile_u0, usrc, tile_d0, dent,
-                         hp->bound, hp->run_scale);
+      if (nbs >= (1ll << 31) || (int64_t)n_chunks * nv > hp->run_scale_cap) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
+      hipLaunchKernelGGL(k_run_scale, dim3((unsigned)n_chunks, nv), dim3(256), 0, s, n_tiles, TPB, tile_u0, usrc, tile_d0, dent,
+                         hp->bound, hp->run_scale, hp->bound_vs);
       HIP_LAUNCH_CHECK();
-      hipLaunchKernelGGL((k_hadamard_split<250, kSplitPool>), dim3((unsigned)nbs), dim3(256), 0, s, M_dim, n_tiles, TPB,
-                         n_chunks, tile_t0, tile_u0, usrc, tile_d0, dent, uidx, gmask, hp->Vh, hp->tinv, hp->run_scale, X, Y);
+      hipLaunchKernelGGL((k_hadamard_split<250, kSplitPool>), dim3((unsigned)nbs, nv), dim3(256), 0, s, M_dim, n_tiles, TPB,
+                         n_chunks, tile_t0, tile_u0, usrc, tile_d0, dent, uidx, gmask, hp->Vh, hp->tinv, hp->run_scale, X, Y, x_vs,
+                         y_vs);
     } else {
       const int n_fgt = (M_dim + 1) / 2;
       const int64_t nbt = (int64_t)n_tiles * ((n_fgt + 7) / 8) * 8;
       if (nbt >= (1ll << 31)) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
-      hipLaunchKernelGGL((k_hadamard_tiled<Real, 1, 1, 2, 256, 1>), dim3((unsigned)nbt), dim3(256), 0, s, M_dim, n_tiles,
-                         tile_t0, tile_u0, usrc, uidx, gmask, offsets, Vp, X, Y);
+      hipLaunchKernelGGL((k_hadamard_tiled<Real, 1, 1, 2, 256, 1>), dim3((unsigned)nbt, nv), dim3(256), 0, s, M_dim, n_tiles,
+                         tile_t0, tile_u0, usrc, uidx, gmask, offsets, Vp, X, Y, x_vs, y_vs);
     }
   } else if (e0 == 3 && e1 == 3) {
     // tiles of up to 160 partners; FP32: one frequency per block on the fp16 matrix cores,
@@ -2570,11 +2501,11 @@ void DeviceKernels<Real>::hadamard_tiled(hipStream_t s, int n_tiles, int M_dim, 
     if (2 * nb2 >= (1ll << 31)) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
     if constexpr (std::is_same<Real, float>::value) {
       if (!hp || !hp->Vh || !hp->tinv || !hp->bound) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
-      hipLaunchKernelGGL((k_hadamard_split3<UMS>), dim3((unsigned)(2 * nb2)), dim3(256), 0, s, M_dim, n_tiles, tile_t0,
-                         tile_u0, usrc, uidx, gmask, hp->Vh, hp->tinv, hp->bound, X, Y);
+      hipLaunchKernelGGL((k_hadamard_split3<UMS>), dim3((unsigned)(2 * nb2), nv), dim3(256), 0, s, M_dim, n_tiles, tile_t0,
+                         tile_u0, usrc, uidx, gmask, hp->Vh, hp->tinv, hp->bound, X, Y, x_vs, y_vs, hp->bound_vs);
     } else {
-      hipLaunchKernelGGL((k_hadamard_tiled<Real, 3, 3, 2, UMS, 1>), dim3((unsigned)nb2), dim3(256), 0, s, M_dim, n_tiles,
-                         tile_t0, tile_u0, usrc, uidx, gmask, offsets, Vp, X, Y);
+      hipLaunchKernelGGL((k_hadamard_tiled<Real, 3, 3, 2, UMS, 1>), dim3((unsigned)nb2, nv), dim3(256), 0, s, M_dim, n_tiles,
+                         tile_t0, tile_u0, usrc, uidx, gmask, offsets, Vp, X, Y, x_vs, y_vs);
     }
   } else {
     throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
@@ -2583,33 +2514,15 @@ void DeviceKernels<Real>::hadamard_tiled(hipStream_t s, int n_tiles, int M_dim, 
 }
 
 template <typename Real>
-void DeviceKernels<Real>::hadamard_vec16(hipStream_t s, int n_trg, int M_dim, const int32_t* partner, const uint16_t* Vb,
-                                         const Real* X, Real* Y, int targets_per_wave) {
-  if (n_trg == 0) return;
-  if constexpr (std::is_same<Real, float>::value) {
-    if (!Vb) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
-    const int tpw = std::max(1, targets_per_wave);
-    const int n_chunks = (n_trg + 4 * tpw - 1) / (4 * tpw);
-    const int64_t nb = (int64_t)n_chunks * ((M_dim + 7) / 8) * 8;
-    if (nb >= (1ll << 31)) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
-    hipLaunchKernelGGL(k_hadamard_vec16<13>, dim3((unsigned)nb), dim3(256), 0, s, M_dim, n_trg, tpw, n_chunks, partner, Vb,
-                       X, Y);
-    HIP_LAUNCH_CHECK();
-  } else {
-    throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);  // FP32 scalar kernels only
-  }
-}
-
-template <typename Real>
 void DeviceKernels<Real>::ifft_down(hipStream_t s, int n_slots, const int32_t* first_child, const Real* Y, Real* dn, int K1, int e1,
-                                    int m, const int32_t* lattice, const int32_t* lat_inv, int ns, const Real* scal, int vg,
-                                    int vi) {
-  if (n_slots == 0) return;
-  const dim3 g((unsigned)((n_slots + 7) / 8 * 8 * e1));  // whole XCD rounds of slots
+                                    int m, const int32_t* lattice, const int32_t* lat_inv, int ns, const Real* scal, int nv,
+                                    int64_t y_vs, int64_t dn_vs) {
+  if (n_slots == 0 || nv <= 0) return;
+  const dim3 g((unsigned)((n_slots + 7) / 8 * 8 * e1), nv);  // whole XCD rounds of slots
 #define PVFMM_IFFT_DN_M(MM)                                                                                       \
   case MM:                                                                                                        \
     hipLaunchKernelGGL((k_ifft_down_m<Real, MM>), g, dim3(DftShape<Real, MM>::NT), 0, s, first_child, Y, dn, K1, e1,     \
-                       lat_inv, scal, n_slots, vg, vi);                                                           \
+                       lat_inv, scal, n_slots, y_vs, dn_vs);                                                      \
     HIP_LAUNCH_CHECK();                                                                                           \
     return;
   switch (m) {
@@ -2626,8 +2539,8 @@ void DeviceKernels<Real>::ifft_down(hipStream_t s, int n_slots, const int32_t* f
   const int cb = fft_children_per_block<Real>(per_child, fixed);
   if (cb * ns > 24 * 512) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);  // register accumulators
   const size_t lds = fixed + cb * per_child;
-  hipLaunchKernelGGL(k_ifft_down<Real>, dim3(n_slots * e1 * (8 / cb)), dim3(512), lds, s, first_child, Y, dn, K1, e1, m, cb, lattice,
-                     ns, scal, vg, vi);
+  hipLaunchKernelGGL(k_ifft_down<Real>, dim3(n_slots * e1 * (8 / cb), nv), dim3(512), lds, s, first_child, Y, dn, K1, e1, m, cb,
+                     lattice, ns, scal, y_vs, dn_vs);
   HIP_LAUNCH_CHECK();
 }
 

@@ -13,6 +13,7 @@ struct HadamardParts {
   const float* bound = nullptr;  // spectrum bound per source slot and component (fft_up's `bound`)
   float* run_scale = nullptr;    // scratch: one scale per run of tiles (scalar kernels)
   int run_scale_cap = 0;         // its length
+  int64_t bound_vs = 0;          // stride of bound per density vector
 };
 
 // Point-kernel kinds of the device code: 0 laplace potential (1x1), 1 laplace gradient
@@ -81,13 +82,12 @@ struct DeviceKernels {
   // V-list: forward DFT of the 8 children's equivalent densities of each source parent.
   // X layout [slot][f][8*e0] complex, component-major within a row ([slot][f][i][child]).  lattice[3p..3p+2] is the m^3 lattice cell of surface
   // point p; lat_inv[(z*m + y)*m + x] is its inverse (-1 inside the cube).
-  // vg, vi: X holds vector groups of vg density vectors, [slot][f][vector vg][8*e0 complex];
-  // this call writes vector vi of the group (vg = 1, vi = 0: one vector).  bound (vg = 1 only;
-  // may be null): bound[slot * e0 + i] = |scal[slot]| * sum of |up| of component i over the
-  // slot's children, which no frequency of that component's spectrum exceeds.
+  // bound (may be null): bound[slot * e0 + i] = |scal[slot]| * sum of |up| of component i over
+  // the slot's children, which no frequency of that component's spectrum exceeds.  The three
+  // V-list launchers take nv density vectors, vector v at + v * (the strides *_vs).
   static void fft_up(hipStream_t s, int n_slots, const int32_t* first_child, const Real* up, int K0, int e0,
-                     int m, const int32_t* lattice, const int32_t* lat_inv, const Real* scal, Real* X, int vg = 1,
-                     int vi = 0, float* bound = nullptr);
+                     int m, const int32_t* lattice, const int32_t* lat_inv, const Real* scal, Real* X,
+                     float* bound = nullptr, int nv = 1, int64_t up_vs = 0, int64_t x_vs = 0, int64_t bound_vs = 0);
   // Y[slot][f][8*e1] = sum_R V[R][f] X[partner[slot][R]][f] on MFMA (rows component-major,
   // as fft_up writes X and ifft_down reads Y); Vp is the transfer block
   // in real form, pre-permuted per lane (layout [R][f][kb][nb][lane 64][4]).  The target slots
@@ -106,7 +106,7 @@ struct DeviceKernels {
   // [part p][lane 64][8], lane l holding part p of B_{2j + a}[8 b + i][16 nb + l % 16] with
   // q = 4c + l/16, a = q / 6, b = q % 6; hp->tinv 1 / tau_f; hp->bound the spectrum bounds of
   // X's slots and components (fft_up); hp->run_scale (scalar kernels) room for
-  // ceil(n_tiles / tiles_per_block) scales.
+  // ceil(n_tiles / tiles_per_block) scales per vector.
   // They stage into an LDS pool of hadamard_pool_max() entries kept across a block's run of
   // tiles: usrc entries are (source slot << 9 | pool slot), uidx holds pool slots (the pool
   // size for none), and tile k's partners new since tile k-1 are dent[tile_d0[k] ..
@@ -118,19 +118,11 @@ struct DeviceKernels {
                              const int32_t* tile_u0, const int32_t* usrc, const int32_t* tile_d0, const int32_t* dent,
                              const uint16_t* uidx, const uint32_t* gmask, const int32_t* offsets,
                              const Real* Vp, const Real* X, Real* Y, int tiles_per_block = 16,
-                             const HadamardParts* hp = nullptr);
+                             const HadamardParts* hp = nullptr, int nv = 1, int64_t x_vs = 0, int64_t y_vs = 0);
   // inverse DFT, pick the check-surface points, dn[child] += scal * value
   static void ifft_down(hipStream_t s, int n_slots, const int32_t* first_child, const Real* Y, Real* dn,
                         int K1, int e1, int m, const int32_t* lattice, const int32_t* lat_inv, int ns,
-                        const Real* scal, int vg = 1, int vi = 0);
-  // The FP32 scalar-kernel Hadamard for a group of 16 density vectors: the MFMA rows are the
-  // 16 vectors of one target, X and Y in the vector-group layout of fft_up / ifft_down with
-  // vg = 16, partner[t * 26 + o] the source slot of target slot t at offset v1_offsets[o] (or
-  // -1), Vb the transfer blocks as three bf16 parts ([pair j][part p][f][lane 64][8], the lane
-  // layout of hadamard_tiled's fp16 parts, unscaled).  targets_per_wave: targets one wave
-  // computes in turn.
-  static void hadamard_vec16(hipStream_t s, int n_trg, int M_dim, const int32_t* partner, const uint16_t* Vb,
-                             const Real* X, Real* Y, int targets_per_wave = 16);
+                        const Real* scal, int nv = 1, int64_t y_vs = 0, int64_t dn_vs = 0);
 };
 
 // FP64 all-pairs sum on the device (AoS src[3n], den[k0 n], trg[3n], out[k1 n] device arrays);

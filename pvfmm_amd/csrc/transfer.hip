@@ -194,23 +194,6 @@ __global__ __launch_bounds__(256) void k_transfer_fp16_stokes(Blocks B, const do
   Vh[((u * 2 + 1) * 64 + l) * 8 + i] = half_bits(h1);
 }
 
-// three bf16 parts, each rounding the remainder of the FP64 value to nearest
-__global__ __launch_bounds__(256) void k_transfer_bf16(Blocks B, uint16_t* __restrict__ Vb) {
-  const int64_t idx = blockIdx.x * (int64_t)256 + threadIdx.x;
-  if (idx >= (int64_t)13 * B.M * 512) return;
-  const int i = (int)(idx & 7), l = (int)(idx >> 3) & 63;
-  const int64_t jf = idx >> 9;
-  const int j = (int)(jf / B.M), f = (int)(jf % B.M);
-  double r = B.entry(offset_of(2 * j + (l >> 5)), f, 8 * ((l >> 4) & 1) + i, l & 15);
-  for (int p = 0; p < 3; p++) {
-    uint32_t u = __float_as_uint((float)r);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    u &= 0xFFFF0000u;
-    Vb[((((int64_t)j * 3 + p) * B.M + f) * 64 + l) * 8 + i] = (uint16_t)(u >> 16);
-    r -= (double)__uint_as_float(u);
-  }
-}
-
 template <typename Real>
 __global__ __launch_bounds__(256) void k_convert(const double* __restrict__ in, int rows_in, int cols_in, Real* __restrict__ out,
                                                  int rows, int ld_out, bool transposed) {
@@ -282,12 +265,6 @@ void transfer_fp16(hipStream_t s, int e0, int e1, int M, const double* G, uint16
     throw Error(kErrInternal, "no fp16 transfer form for this kernel");
   TR_LAUNCH_CHECK();
   HIP_CHECK(hipStreamSynchronize(s));  // tau
-}
-
-void transfer_bf16(hipStream_t s, int M, const double* G, uint16_t* Vb) {
-  const Blocks B{reinterpret_cast<const double2*>(G), M, 1, 1};
-  hipLaunchKernelGGL(k_transfer_bf16, dim3(grid_of((int64_t)13 * M * 512)), dim3(256), 0, s, B, Vb);
-  TR_LAUNCH_CHECK();
 }
 
 template <typename Real>

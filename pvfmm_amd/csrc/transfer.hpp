@@ -28,10 +28,8 @@ void transfer_spectra(hipStream_t s, int kind, int m, double* G);
 // split forms):
 //   real:   Vp[((R * M + f) * e0 + kb) * e1 + nb][lane][q], FP64 kernels, R of 27
 //   fp16:   two parts of tau_f B, scalar and Stokes layouts of hadamard_tiled; tinv = 1 / tau_f
-//   bf16:   three parts of B, scalar, layout of hadamard_vec16
 void transfer_real(hipStream_t s, int e0, int e1, int M, const double* G, double* Vp);
 void transfer_fp16(hipStream_t s, int e0, int e1, int M, const double* G, uint16_t* Vh, float* tinv);
-void transfer_bf16(hipStream_t s, int M, const double* G, uint16_t* Vb);
 
 // out (rows x ld_out, Real) = in (rows_in x cols_in, FP64), zero outside it; transposed: out
 // (rows x ld_out) = in^T.

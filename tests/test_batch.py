@@ -158,3 +158,35 @@ def test_sixteen_vector_pass_and_its_tuning(kernel):
     assert chosen["hadamard_vec_targets_per_wave"] in (0, 4, 8, 16, 32)
     ub2 = tb.evaluate_device(q)
     assert float(torch.linalg.norm(ub2 - ub) / torch.linalg.norm(ub)) < 1e-6
+
+
+@pytest.mark.parametrize("kernel,m,prec,n,nv", [
+    ("laplace_poten", 6, "mixed", 65536, 10),   # 585 V-list parents: passes of 7 and 3 vectors
+    ("laplace_poten", 6, "fp64", 65536, 10),
+    ("stokes_vel", 4, "mixed", 9000, 5),        # one pass
+    ("laplace_grad", 2, "mixed", 3000, 3),      # the transforms of any m
+    ("laplace_poten", 14, "fp64", 3000, 3),
+    ("laplace_poten", 4, "mixed", 40, 4),       # no V list at all
+])
+def test_vlist_passes_of_several_vectors(kernel, m, prec, n, nv):
+    """The vectors of a V-list pass share its launches; each equals its evaluation alone to
+    the rounding of the up/down GEMMs (whose K splits depend on the number of rows): 1e-6 in
+    FP32, 1e-11 in FP64, forward and adjoint."""
+    import torch
+
+    rng = np.random.default_rng(12)
+    x = rng.random((n, 3))
+    k0, k1 = P.kernel_dims(kernel)
+    q = torch.tensor(rng.standard_normal((nv, k0 * n)), device="cuda:0")
+    g = torch.tensor(rng.standard_normal((nv, k1 * n)), device="cuda:0")
+    fmm = P.PtFMM(kernel, m, prec)
+    tb = P.PtFMMTree(x, x, 100).setup(fmm, n_vec_max=nv)
+    t1 = P.PtFMMTree(x, x, 100).setup(fmm)
+    pairs = [(tb.evaluate_device(q), [t1.evaluate_device(v) for v in q])]
+    if kernel != "laplace_grad":
+        pairs.append((tb.evaluate_adjoint_device(g), [t1.evaluate_adjoint_device(v) for v in g]))
+    tol = 1e-6 if prec == "mixed" else 1e-11
+    for got, ref in pairs:
+        for v in range(nv):
+            e = float(torch.linalg.norm(got[v] - ref[v]) / torch.linalg.norm(ref[v]))
+            assert e < tol, (v, e)
