@@ -1,0 +1,30 @@
+"""The U list stages its sources through windows of 64 leaves and chunks of 512 points: trees whose
+leaves hold one or a few points (more than 64 leaves to a chunk), exactly the chunk's or more than
+a block's points, and clusters of duplicated points, against the oracle on the same tree."""
+import numpy as np
+import pytest
+
+import oracle as O
+import pvfmm_amd as P
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("kernel,n,max_pts", [
+    ("laplace_poten", 600, 1), ("laplace_grad", 900, 3), ("stokes_vel", 500, 2),
+    ("laplace_poten", 512, 512), ("laplace_grad", 513, 600), ("laplace_grad", 3000, 700), ("stokes_vel", 1500, 400),
+])
+def test_ulist_staging_matches_oracle(gpu, kernel, n, max_pts, prec):
+    rng = np.random.default_rng(n + max_pts)
+    x = np.concatenate([rng.random((n - n // 4, 3)), 0.7 + 0.01 * rng.random((n // 4 - 5, 3)), np.full((5, 3), 0.31)])
+    k0, _ = P.kernel_dims(kernel)
+    q = rng.standard_normal(k0 * n)
+    m = 4
+    u = P.PtFMMTree(x, x, max_pts).setup(P.PtFMM(kernel, m, prec)).evaluate(q)
+    t = O.OracleTree(x, x, max_pts)
+    t.set_operators(O.precompute(kernel, m, "fp64" if prec == "fp64" else "fp32"))
+    ref = t.evaluate(q)
+    e = float(np.linalg.norm(u - ref) / np.linalg.norm(ref))
+    # rounding only: the FP64 and FP32 bars of the parity tests
+    assert e < (1e-10 if prec == "fp64" else 1e-5), e
