@@ -378,6 +378,11 @@ class DevicePlan final : public DevicePlanBase {
   DBuf<int32_t> t_leaf_, far_ptr_, far_node_, u_ptr_, u_items_;
   DBuf<int64_t> far_den_;
   DBuf<double> far_rad_;
+  // far rows with much more work than most, split over blocks (FarSplit)
+  DBuf<int32_t> fs_row_, fs_begin_, fs_end_, fs_rows_, fs_ptr_;
+  DBuf<int64_t> fs_part_;
+  DBuf<double> fs_sums_;
+  FarSplit far_split_;
   int n_tleaf_ = 0;
   std::vector<hipEvent_t> ev_;
   std::vector<hipEvent_t> vev_;  // per-vector V-list sub-phase events (timing of multi-vector passes)
@@ -695,6 +700,7 @@ class DevicePlan final : public DevicePlanBase {
     }
     far_ptr_.upload(far_ptr, &total); far_node_.upload(far_node, &total); far_den_.upload(far_den, &total);
     far_rad_.upload(far_rad, &total);
+    split_far_rows(T, tleaf, far_ptr, &total);
     u_ptr_.upload(u_ptr, &total); u_items_.upload(u_items, &total);
     if (bndry_ != kFreeSpace) {  // FMM_Pts::PeriodicBC and PostProcessing (include/fmm_pts.txx:2641-2657,5740-5774)
       bc_ = ops_->bc(bndry_, false);
@@ -724,6 +730,51 @@ class DevicePlan final : public DevicePlanBase {
     stats.far_items = (int64_t)far_node.size(); stats.far_pairs = far_pairs; stats.s2m_pairs = s2m_pairs;
     stats.device_bytes = total;
     device_bytes_ = total;
+  }
+
+  // Splits the far rows of more than kFarRowPairs pairs into segments of about kFarSegPairs.  A
+  // block of 256 threads does the mean row's 5,000-20,000 pairs in 10-30 us; a row of 16 such
+  // units would outlast the rest of most launches.  Segments go first.
+  static constexpr int64_t kFarRowPairs = 131072, kFarSegPairs = 32768;
+  void split_far_rows(const Octree& T, const std::vector<int32_t>& tleaf, const std::vector<int32_t>& far_ptr, int64_t* total) {
+    std::vector<int32_t> row, begin, end, rows, ptr{0};
+    std::vector<int64_t> part;
+    std::vector<char> heavy(tleaf.size(), 0);
+    int64_t sums = 0;
+    for (size_t r = 0; r < tleaf.size(); r++) {
+      const int64_t nt = T.pt_cnt1(tleaf[r]);
+      const int n = far_ptr[r + 1] - far_ptr[r];
+      if (n < 2 || n * nt * ns_ <= kFarRowPairs) continue;
+      const int per = (int)std::max<int64_t>(1, kFarSegPairs / (nt * ns_));
+      for (int i = far_ptr[r]; i < far_ptr[r + 1]; i += per) {
+        row.push_back((int32_t)r);
+        begin.push_back(i);
+        end.push_back(std::min(far_ptr[r + 1], i + per));
+        part.push_back(sums);
+        sums += nt * k1_;
+      }
+      heavy[r] = 1;
+      rows.push_back((int32_t)r);
+      ptr.push_back((int32_t)row.size());
+    }
+    if (rows.empty()) return;
+    for (size_t r = 0; r < tleaf.size(); r++)
+      if (!heavy[r]) {
+        row.push_back((int32_t)r);
+        begin.push_back(far_ptr[r]);
+        end.push_back(far_ptr[r + 1]);
+        part.push_back(-1);
+      }
+    fs_row_.upload(row, total); fs_begin_.upload(begin, total); fs_end_.upload(end, total); fs_part_.upload(part, total);
+    fs_rows_.upload(rows, total); fs_ptr_.upload(ptr, total);
+    fs_sums_.alloc(sums * std::min(8, nvb_), total);
+    far_split_.n_blk = (int)row.size();
+    far_split_.n_rows = (int)rows.size();
+    far_split_.blk_row = fs_row_.p; far_split_.blk_begin = fs_begin_.p; far_split_.blk_end = fs_end_.p;
+    far_split_.blk_part = fs_part_.p;
+    far_split_.row = fs_rows_.p; far_split_.row_ptr = fs_ptr_.p;
+    far_split_.part = fs_sums_.p;
+    far_split_.part_vs = sums;
   }
 
   // ---- adjoint evaluation: the transpose of the evaluation's linear map, phase by phase in
@@ -1123,7 +1174,8 @@ class DevicePlan final : public DevicePlanBase {
     mark(10);
     // equivalent surfaces -> targets (own downward equivalent + W list)
     K::far_points(st_, pk, n_tleaf_, t_leaf_.p, far_ptr_.p, far_node_.p, far_den_.p, far_rad_.p, trg_begin_.p, trg_end_.p,
-                  center_.p, node_size_.p, ops_->unit_surf.p, ns_, tx_.p, n_trg_, eq_.p, tval_.p, false, nv, eq_vs_, val_vs);
+                  center_.p, node_size_.p, ops_->unit_surf.p, ns_, tx_.p, n_trg_, eq_.p, tval_.p, false, nv, eq_vs_, val_vs,
+                  far_split_);
     mark(11);
     // U list: near-field P2P
     K::p2p_points(st_, pk, n_tleaf_, t_leaf_.p, u_ptr_.p, u_items_.p, trg_begin_.p, trg_end_.p, src_begin_.p, src_end_.p,

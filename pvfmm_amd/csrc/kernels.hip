@@ -542,6 +542,10 @@ __global__ __launch_bounds__(256) void k_p2p_leaf(const int32_t* __restrict__ tl
 
 // Equivalent surfaces -> targets (own L2T surface and W-list M2T) with the leaf-block layout
 // of k_p2p_leaf; a staged source is the surface point o + r * size * unit_surf[p] of its node.
+// A row with many W items is split over several blocks (split.blk_*, see far_points): a coarse
+// leaf beside a fine surface has up to 148 of them, 122 times the mean work, and one block then
+// decided the time of the kernel (Stokes FP64, 150k sources on an ellipsoid and 70k targets around
+// it: 543 us whole, 162 us split; 1M adaptive FP64 936 and 800 us).
 template <typename Real, int KIND, int VB>
 __global__ __launch_bounds__(256) void k_far_leaf(const int32_t* __restrict__ tleaf, const int32_t* __restrict__ item_ptr,
                                                   const int32_t* __restrict__ item_node, const int64_t* __restrict__ item_den,
@@ -550,16 +554,18 @@ __global__ __launch_bounds__(256) void k_far_leaf(const int32_t* __restrict__ tl
                                                   const float* __restrict__ node_size, const Real* __restrict__ unit_surf,
                                                   int ns, const Real* __restrict__ tx, int64_t n_trg,
                                                   const Real* __restrict__ dens, int64_t den_vs, double* __restrict__ out,
-                                                  int64_t out_vs, bool accumulate) {
+                                                  int64_t out_vs, bool accumulate, FarSplit split) {
   constexpr int K0 = KDims<KIND>::k0, K1 = KDims<KIND>::k1, NT = 256, SC = VB * K0 >= 8 ? 256 : 512;
   __shared__ Real lc[3 * SC];
   __shared__ Real ld[VB * K0 * SC];
   __shared__ double red[K1 * NT];
-  const int row = blockIdx.x, tid = threadIdx.x;
+  const bool sp = split.blk_row != nullptr;
+  const int row = sp ? split.blk_row[blockIdx.x] : blockIdx.x, tid = threadIdx.x;
   const int T = tleaf[row];
   const int tb = trg_begin[T], nt = trg_end[T] - tb;
   const double ct0 = center[3 * T], ct1 = center[3 * T + 1], ct2 = center[3 * T + 2];
-  const int ib = item_ptr[row], ie = item_ptr[row + 1];
+  const int ib = sp ? split.blk_begin[blockIdx.x] : item_ptr[row], ie = sp ? split.blk_end[blockIdx.x] : item_ptr[row + 1];
+  const int64_t part_at = sp ? split.blk_part[blockIdx.x] : -1;  // a segment's sums go to split.part
   for (int c0 = 0; c0 < nt; c0 += NT) {
     const int ntc = min(NT, nt - c0), nsplit = NT / ntc;
     const int t = tid % ntc, j = tid / ntc;
@@ -637,12 +643,32 @@ __global__ __launch_bounds__(256) void k_far_leaf(const int32_t* __restrict__ tl
         for (int k = 0; k < K1; k++) {
           double sum = 0;
           for (int jj = 0; jj < nsplit; jj++) sum += red[k * NT + tid + jj * ntc];
-          double* d = &out[v * out_vs + k * n_trg + tb + c0 + tid];
           sum *= kscale<KIND>();
-          *d = accumulate ? *d + sum : sum;
+          if (part_at >= 0) {
+            split.part[v * split.part_vs + part_at + k * nt + c0 + tid] = sum;
+          } else {
+            double* d = &out[v * out_vs + k * n_trg + tb + c0 + tid];
+            *d = accumulate ? *d + sum : sum;
+          }
         }
       }
     }
+  }
+}
+
+// The segments of split row blockIdx.x, added in order (blockIdx.y: density vector)
+__global__ __launch_bounds__(256) void k_far_reduce(int k1, const int32_t* __restrict__ tleaf, const int32_t* __restrict__ trg_begin,
+                                                    const int32_t* __restrict__ trg_end, int64_t n_trg, FarSplit split,
+                                                    double* __restrict__ out, int64_t out_vs, bool accumulate) {
+  const int T = tleaf[split.row[blockIdx.x]], tb = trg_begin[T], nt = trg_end[T] - tb;
+  const double* part = split.part + blockIdx.y * split.part_vs;
+  out += blockIdx.y * out_vs;
+  const int s0 = split.row_ptr[blockIdx.x], s1 = split.row_ptr[blockIdx.x + 1];
+  for (int e = threadIdx.x; e < k1 * nt; e += 256) {
+    double sum = 0;
+    for (int sg = s0; sg < s1; sg++) sum += part[split.blk_part[sg] + e];
+    double* d = &out[(e / nt) * n_trg + tb + e % nt];
+    *d = accumulate ? *d + sum : sum;
   }
 }
 
@@ -2379,14 +2405,16 @@ void DeviceKernels<Real>::far_points(hipStream_t s, int kind, int n_rows, const 
                                      const int32_t* item_node, const int64_t* item_den, const double* item_rad,
                                      const int32_t* trg_begin, const int32_t* trg_end, const double* center,
                                      const float* node_size, const Real* unit_surf, int ns, const Real* tx, int64_t n_trg,
-                                     const Real* dens, double* out, bool accumulate, int nv, int64_t den_vs, int64_t out_vs) {
+                                     const Real* dens, double* out, bool accumulate, int nv, int64_t den_vs, int64_t out_vs,
+                                     const FarSplit& split) {
   if (n_rows == 0 || nv <= 0) return;
+  const int n_blk = split.blk_row ? split.n_blk : n_rows;
   for_density_chunks(nv, [&](int v0, int vb) {
     const Real* d = dens + v0 * den_vs;
     double* o = out + v0 * out_vs;
 #define FAR_LAUNCH(KD, VB)                                                                                                   \
-  hipLaunchKernelGGL((k_far_leaf<Real, KD, VB>), dim3(n_rows), dim3(256), 0, s, tleaf, item_ptr, item_node, item_den, item_rad, \
-                     trg_begin, trg_end, center, node_size, unit_surf, ns, tx, n_trg, d, den_vs, o, out_vs, accumulate)
+  hipLaunchKernelGGL((k_far_leaf<Real, KD, VB>), dim3(n_blk), dim3(256), 0, s, tleaf, item_ptr, item_node, item_den, item_rad, \
+                     trg_begin, trg_end, center, node_size, unit_surf, ns, tx, n_trg, d, den_vs, o, out_vs, accumulate, split)
 #define FAR_VB(KD)                   \
   switch (vb) {                      \
     case 8: FAR_LAUNCH(KD, 8); break; \
@@ -2398,6 +2426,11 @@ void DeviceKernels<Real>::far_points(hipStream_t s, int kind, int n_rows, const 
 #undef FAR_VB
 #undef FAR_LAUNCH
     HIP_LAUNCH_CHECK();
+    if (split.blk_row) {
+      hipLaunchKernelGGL(k_far_reduce, dim3(split.n_rows, vb), dim3(256), 0, s, kind == 0 ? 1 : 3, tleaf, trg_begin, trg_end, n_trg,
+                         split, o, out_vs, accumulate);
+      HIP_LAUNCH_CHECK();
+    }
   });
 }
 

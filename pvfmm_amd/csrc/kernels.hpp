@@ -16,6 +16,20 @@ struct HadamardParts {
   int64_t bound_vs = 0;          // stride of bound per density vector
 };
 
+// Rows of far_points split over several blocks (device arrays; blk_row null: a block per row).
+// Block b < n_blk handles items [blk_begin[b], blk_end[b]) of row blk_row[b]; blocks [0,
+// row_ptr[n_rows]) are the segments of the rows row[0 .. n_rows), whose sums go to part +
+// blk_part[b] ([component][target], part_vs apart per density vector, room for 8 vectors) and are
+// added in segment order; the others have blk_part -1 and write their row.
+struct FarSplit {
+  int n_blk = 0, n_rows = 0;
+  const int32_t *blk_row = nullptr, *blk_begin = nullptr, *blk_end = nullptr;
+  const int64_t* blk_part = nullptr;
+  const int32_t *row = nullptr, *row_ptr = nullptr;
+  double* part = nullptr;
+  int64_t part_vs = 0;
+};
+
 // Point-kernel kinds of the device code: 0 laplace potential (1x1), 1 laplace gradient
 // (1x3, r = x_trg - x_src, i.e. minus the gradient of the potential), 2 stokes velocity (3x3).
 template <typename Real>
@@ -67,7 +81,7 @@ struct DeviceKernels {
                          const int32_t* trg_begin, const int32_t* trg_end, const double* center,
                          const float* node_size, const Real* unit_surf, int ns, const Real* tx, int64_t n_trg,
                          const Real* dens, double* out, bool accumulate, int nv = 1, int64_t den_vs = 0,
-                         int64_t out_vs = 0);
+                         int64_t out_vs = 0, const FarSplit& split = {});
 
   // C[rc[i]*ldc : +N] (+)= alpha[i] * A[ra[i]*lda : +K] * B[K x N] on MFMA; `work` (work_elems
   // Reals, may be null) enables a deterministic split-K for grids too small to fill the GPU.
