@@ -229,6 +229,11 @@ class DevicePlan final : public DevicePlanBase {
   int nvb_ = 1;  // density vectors per evaluation pass (buffers hold this many)
   int64_t eq_vs_ = 0, dn_vs_ = 0, chk_vs_ = 0, ctmp_vs_ = 0;  // per-vector strides  // room for 4 K-split partials of the largest GEMM output, at most 2^25
   int ru_ = 0, rd_ = 0;
+  // The coarsest level whose upward equivalent densities anything reads (V or W list, boundary
+  // operator), and whose downward check potentials anything writes: U2U and D2D stop there (in
+  // free space the two coarsest levels have no V or W list and their translations were zeros or
+  // unread; 20 of 250 us at 4099 points)
+  int up_min_ = 0, dn_min_ = 0;
   // S2M
   DBuf<int32_t> s2m_node_, s2m_ptr_, s2m_items_, s2m_orow_;
   DBuf<Real> s2m_alpha_;
@@ -556,8 +561,9 @@ class DevicePlan final : public DevicePlanBase {
     t_leaf_.upload(tleaf, &total);
     eq_vs_ = (int64_t)(N + n_l2t_) * K0_;
     dn_vs_ = (int64_t)N * K1_;
-    eq_.alloc(eq_vs_ * nvb_, &total);
-    dn_.alloc(dn_vs_ * nvb_, &total);
+    auto words = [](int64_t count) { return (count + 3) / 4 * 4; };  // whole 16-byte words (begin)
+    eq_.alloc(words(eq_vs_ * nvb_), &total);
+    dn_.alloc(words(dn_vs_ * nvb_), &total);
 
     // ---- M2M / L2L rows per level
     m2m_.clear(); l2l_.clear();
@@ -662,6 +668,23 @@ class DevicePlan final : public DevicePlanBase {
     y_vs_ = (int64_t)n_vtrg_ * M_dim_ * 16 * e1_;
     X_.alloc(x_vs_ * vlist_nv_, &total);
     Y_.alloc(y_vs_ * vlist_nv_, &total);
+
+    up_min_ = dn_min_ = bndry_ != kFreeSpace ? 0 : max_depth_ + 1;
+    {
+      const int nl_vw = T.list_count(kW);
+      std::vector<char> used_src(n_vsrc_, 0);
+      for (int32_t sl : v_partner)
+        if (sl >= 0) used_src[sl] = 1;
+      for (int sl = 0; sl < n_vsrc_; sl++)
+        if (used_src[sl]) up_min_ = std::min(up_min_, h_.vsrc_depth[sl] + 1);
+      for (int d : h_.vtrg_depth) dn_min_ = std::min(dn_min_, d + 1);
+      for (int i : x_node) dn_min_ = std::min(dn_min_, (int)T.depth[i]);
+      for (int t : tleaf)
+        for (int k = 0; k < nl_vw; k++) {
+          const int32_t w = T.lists[kW][(size_t)t * nl_vw + k];
+          if (w >= 0) up_min_ = std::min(up_min_, (int)T.depth[w]);
+        }
+    }
 
     // ---- far field (L2T own surface + W list M2T) and U list per target leaf
     std::vector<int32_t> far_ptr{0}, far_node, u_ptr{0}, u_items;
@@ -1016,7 +1039,7 @@ class DevicePlan final : public DevicePlanBase {
     K::gemm_rows(st_, n_l2t_, K1_, rd_, ctmp_.p, l2t_seq_.p, rd_, a.op->dc2de0.p, dn_.p, l2t_ra_.p, K1_, l2t_alpha_.p, true,
                  gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, dn_vs_);
     // D2D^T, bottom-up: parent += [8 children] x [D2D_0 .. D2D_7]^T
-    for (int l = max_depth_; l >= 1; l--) {
+    for (int l = max_depth_; l >= dn_min_ + 1; l--) {
       const LevelRows& L = *l2l_[l - 1];
       if (ops_->d2d_fact && L.n >= kFactorRows) {
         K::gemm_rows(st_, L.n, rd_, 8 * K1_, dn_.p, L.rc.p, K1_, a.op->d2dr.p, ctmp_.p, lvl_seq_.p, rd_, nullptr, false,
@@ -1048,7 +1071,7 @@ class DevicePlan final : public DevicePlanBase {
     K::far_points(st_, ek, a.n_x, a.x_leaf.p, a.x_ptr.p, a.x_node.p, a.x_den.p, a.x_rad.p, a.sb.p, a.se.p,
                   a.center.p, a.nsz.p, ops_->unit_surf.p, ns_, sx_.p, n_src_, dn_.p, a.sval.p, true, nv, dn_vs_, o_vs);
     // U2U^T, top-down: [8 children] += parent x [U2U_0 .. U2U_7]^T
-    for (int l = 0; l <= max_depth_ - 1; l++) {
+    for (int l = up_min_; l <= max_depth_ - 1; l++) {
       const LevelRows& L = *m2m_[l];
       if (ops_->u2u_fact && L.n >= kFactorRows) {
         K::gemm_rows(st_, L.n, ru_, K0_, eq_.p, L.rc.p, K0_, a.op->uc2ue1.p, ctmp_.p, lvl_seq_.p, ru_, nullptr, false,
@@ -1091,9 +1114,7 @@ class DevicePlan final : public DevicePlanBase {
     const int64_t den_vs = (int64_t)k0_ * n_src_, val_vs = (int64_t)k1_ * n_trg_;
     const int sp = tuning.gemm_split_blocks;
     mark(0);
-    K::gather_density(st_, n_src_, k0_, d_den, src_perm_.p, den_scale, sden_.p, nv, den_vs);
-    K::fill(st_, eq_.p, eq_vs_ * nv);
-    K::fill(st_, dn_.p, dn_vs_ * nv);
+    K::begin(st_, n_src_, k0_, d_den, src_perm_.p, den_scale, sden_.p, nv, den_vs, eq_.p, eq_vs_ * nv, dn_.p, dn_vs_ * nv);
     mark(1);
     // S2U: sources -> upward check surface (RAD1), then check -> equivalent
     K::p2p_surface(st_, ek, n_s2m_, s2m_node_.p, s2m_ptr_.p, s2m_items_.p, src_begin_.p, src_end_.p, center_.p, node_size_.p,
@@ -1105,7 +1126,7 @@ class DevicePlan final : public DevicePlanBase {
                  gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, eq_vs_);
     mark(3);
     // U2U, bottom-up: parent row = [8 children] x stacked U2U
-    for (int l = max_depth_ - 1; l >= 0; l--) {
+    for (int l = max_depth_ - 1; l >= up_min_; l--) {
       const LevelRows& L = *m2m_[l];
       if (ops_->u2u_fact && L.n >= kFactorRows) {  // [8 children] -> rank coordinates -> parent
         K::gemm_rows(st_, L.n, ru_, 8 * K0_, eq_.p, L.ra.p, K0_, ops_->u2ur.p, ctmp_.p, lvl_seq_.p, ru_, nullptr, false,
@@ -1153,7 +1174,7 @@ class DevicePlan final : public DevicePlanBase {
     }
     mark(8);
     // D2D, top-down: 8 children rows += parent x [D2D_0 .. D2D_7]
-    for (int l = 1; l <= max_depth_; l++) {
+    for (int l = dn_min_ + 1; l <= max_depth_; l++) {
       const LevelRows& L = *l2l_[l - 1];
       if (ops_->d2d_fact && L.n >= kFactorRows) {  // parent check -> rank coordinates -> [8 children]
         K::gemm_rows(st_, L.n, rd_, K1_, dn_.p, L.ra.p, K1_, ops_->dc2de0.p, ctmp_.p, lvl_seq_.p, rd_, nullptr, false,

@@ -41,6 +41,10 @@ struct DeviceKernels {
   static void scatter_output(hipStream_t s, int64_t n, int k1, const double* val, const int64_t* perm,
                              double scal, double* out, int n_vec, int64_t out_stride);
   static void fill(hipStream_t s, Real* p, int64_t n);
+  // gather_density, and za[0, na) and zb[0, nb) zeroed, up to the next 16-byte word (16-byte
+  // aligned buffers of whole words), in one launch
+  static void begin(hipStream_t s, int64_t n, int k0, const double* in, const int64_t* perm, double scal, Real* den, int n_vec,
+                    int64_t in_stride, Real* za, int64_t na, Real* zb, int64_t nb);
   // Periodic (PXYZ) post-processing of FMM_Pts::PostProcessing (include/fmm_pts.txx:5740-5774):
   // val[j*n + i] -= sum_c avg_c V_cj(x_i), avg_c the sum of component c over the root's K0
   // equivalent values eq_root[p*e0 + c], V the kernel's analytic potential of a uniform unit
@@ -86,7 +90,7 @@ struct DeviceKernels {
   // C[rc[i]*ldc : +N] (+)= alpha[i] * A[ra[i]*lda : +K] * B[K x N] on MFMA; `work` (work_elems
   // Reals, may be null) enables a deterministic split-K for grids too small to fill the GPU.
   // split_blocks: K is split (through work[], work_elems reals) when the tile grid has fewer
-  // blocks than this, so that about twice as many run.  nv density vectors run as one GEMM of
+  // blocks than this, so that about that many run.  nv density vectors run as one GEMM of
   // nv * M rows: vector v reads A + v * avs and writes C + v * cvs (same ra, rc, alpha).
   static void gemm_rows(hipStream_t s, int M, int N, int K, const Real* A, const int32_t* ra, int64_t lda,
                         const Real* B, Real* C, const int32_t* rc, int64_t ldc, const Real* alpha,
