@@ -195,16 +195,17 @@ int pvfmm_amd_tree_set_tuning(void* tree, const int* params, int n);
 /* Many set-up trees evaluated together (independent point clouds); no counterpart in the
  * reference, whose callers keep one context per cloud.  The first evaluation records every
  * tree's evaluation (one density vector each, device-resident) into one HIP graph with one
- * branch per tree; later calls with the same device pointers replay it with a single graph
- * launch on the batch's stream.  Other pointers, changed launch shapes of a tree, or a tree
- * set up again (its new plan has new device buffers) record the graph again.  A launch is
+ * branch per tree; later calls replay it with a single graph launch on the batch's stream, on
+ * whatever buffers they pass.  Changed launch shapes of a tree, or a tree set up again (its new
+ * plan has new device buffers), record the graph again.  A launch is
  * ordered after the work already queued on every tree's stream and before work queued there
  * later, so eager and batched evaluations of one tree may be mixed, also with async = 1.  The
  * trees must outlive the batch. */
 void* pvfmm_amd_batch_create(void* const* trees, int n_trees);
 int pvfmm_amd_batch_evaluate_device(void* batch, const double* const* d_den, double* const* d_out, int async);
 void* pvfmm_amd_batch_stream(void* batch);
-/* number of times the graph was recorded (1 while the pointers stay the same) */
+/* number of times the graph was recorded or replayed on buffers other than the last call's
+ * (1 while the pointers stay the same) */
 int pvfmm_amd_batch_records(void* batch);
 void pvfmm_amd_batch_destroy(void* batch);
 

@@ -133,7 +133,9 @@ void eval_device(TreeHandle* t, const double* d_den, double* d_out, int n_vec, d
 }
 
 // Independent trees evaluated as one HIP graph: a fork event on the batch stream, each
-// tree's evaluation on its own stream, a join back.  Recorded once per set of device pointers.
+// tree's evaluation on its own stream, a join back.  The recorded evaluations read their buffers'
+// addresses from `slots`, which every call sets first, so other buffers need no new recording
+// (recording and instantiating 24 clouds took 1.8 ms of a 5.6 ms call).
 struct BatchHandle {
   std::vector<TreeHandle*> trees;
   hipStream_t stream = nullptr;
@@ -174,8 +176,12 @@ struct BatchHandle {
     exec = nullptr;
     graph = nullptr;
   }
-  void record(const double* const* d_den, double* const* d_out) {
+  DeviceArray slots;  // n density buffer addresses, then n output buffer addresses
+  void record() {
     drop_graph();
+    const size_t n = trees.size();
+    const double* const* den_slot = (const double* const*)slots.p;
+    double* const* out_slot = (double* const*)slots.p + n;
     std::vector<bool> timing(trees.size());
     HIP_CHECK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     try {
@@ -183,7 +189,7 @@ struct BatchHandle {
       for (size_t i = 0; i < trees.size(); i++) {
         TreeHandle* t = trees[i];
         HIP_CHECK(hipStreamWaitEvent(t->stream, fork, 0));
-        t->plan->evaluate(d_den[i], d_out[i], 1, 1.0, 1.0);
+        t->plan->evaluate_slots(den_slot + i, out_slot + i);
         HIP_CHECK(hipEventRecord(joins[i], t->stream));
         HIP_CHECK(hipStreamWaitEvent(stream, joins[i], 0));
       }
@@ -195,11 +201,8 @@ struct BatchHandle {
     }
     HIP_CHECK(hipStreamEndCapture(stream, &graph));
     HIP_CHECK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    den_key.assign(d_den, d_den + trees.size());
-    out_key.assign(d_out, d_out + trees.size());
     tune_key = tunings();
     plan_key = plans();
-    records++;
   }
 };
 
@@ -231,10 +234,24 @@ void batch_eval(BatchHandle* b, const double* const* d_den, double* const* d_out
     b->trees[i]->plan->set_timing(false);  // event records stay out of the graph
   }
   // a tree set up again has a new plan (new device buffers): the graph is recorded again
-  const bool same = b->exec && std::equal(b->den_key.begin(), b->den_key.end(), d_den) &&
-                    std::equal(b->out_key.begin(), b->out_key.end(), d_out) && b->tune_key == b->tunings() &&
-                    b->plan_key == b->plans();
-  if (!same) b->record(d_den, d_out);
+  const bool recorded = b->exec && b->tune_key == b->tunings() && b->plan_key == b->plans();
+  if (!recorded) {
+    b->slots.ensure(2 * n * sizeof(void*));
+    b->record();
+  }
+  // counts the recordings and the calls that bind other buffers
+  if (!recorded || !std::equal(b->den_key.begin(), b->den_key.end(), d_den) ||
+      !std::equal(b->out_key.begin(), b->out_key.end(), d_out)) {
+    b->den_key.assign(d_den, d_den + n);
+    b->out_key.assign(d_out, d_out + n);
+    b->records++;
+  }
+  std::vector<void*> ptr(2 * n);
+  for (size_t i = 0; i < n; i++) {
+    ptr[i] = const_cast<double*>(d_den[i]);
+    ptr[n + i] = d_out[i];
+  }
+  set_pointers(b->stream, (int)(2 * n), ptr.data(), (void**)b->slots.p);
   // the replay uses each plan's scratch buffers, as eager evaluations on the tree's own stream
   // do: it starts after the work queued there and that work resumes after it
   for (size_t i = 0; i < n; i++) {

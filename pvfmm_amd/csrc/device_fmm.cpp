@@ -151,6 +151,10 @@ class DevicePlan final : public DevicePlanBase {
                    std::min(nvb_, n_vec - v));
   }
 
+  void evaluate_slots(const double* const* den_slot, double* const* out_slot) override {
+    evaluate_one(nullptr, nullptr, 1.0, 1.0, 1, den_slot, out_slot);
+  }
+
   Tuning autotune(const double* d_den, double* d_out, int n_vec) override {
     if (n_vec < 1 || n_vec > nvb_) throw Error(kErrInvalidArgument, "autotune takes 1 to n_vec_max density vectors");
     const bool was = timing_;
@@ -1109,12 +1113,14 @@ class DevicePlan final : public DevicePlanBase {
   }
 
  private:
-  void evaluate_one(const double* d_den, double* d_out, double den_scale, double out_scale, int nv) {
+  void evaluate_one(const double* d_den, double* d_out, double den_scale, double out_scale, int nv,
+                    const double* const* den_slot = nullptr, double* const* out_slot = nullptr) {
     const int pk = O_.ker.pt_kind, ek = O_.ker.exp_kind;
     const int64_t den_vs = (int64_t)k0_ * n_src_, val_vs = (int64_t)k1_ * n_trg_;
     const int sp = tuning.gemm_split_blocks;
     mark(0);
-    K::begin(st_, n_src_, k0_, d_den, src_perm_.p, den_scale, sden_.p, nv, den_vs, eq_.p, eq_vs_ * nv, dn_.p, dn_vs_ * nv);
+    K::begin(st_, n_src_, k0_, d_den, src_perm_.p, den_scale, sden_.p, nv, den_vs, eq_.p, eq_vs_ * nv, dn_.p, dn_vs_ * nv,
+             den_slot);
     mark(1);
     // S2U: sources -> upward check surface (RAD1), then check -> equivalent
     K::p2p_surface(st_, ek, n_s2m_, s2m_node_.p, s2m_ptr_.p, s2m_items_.p, src_begin_.p, src_end_.p, center_.p, node_size_.p,
@@ -1205,7 +1211,7 @@ class DevicePlan final : public DevicePlanBase {
       K::vol_correction(st_, pk, n_trg_, txa_.p, eq_.p, K0_, e0_, tval_.p, nv, eq_vs_, val_vs);
     mark(12);
     // targets not in any leaf with targets are impossible; every target lies in exactly one leaf
-    K::scatter_output(st_, n_trg_, k1_, tval_.p, trg_perm_.p, out_scale, d_out, nv, val_vs);
+    K::scatter_output(st_, n_trg_, k1_, tval_.p, trg_perm_.p, out_scale, d_out, nv, val_vs, out_slot);
     mark(13);
     if (timing_) {
       HIP_CHECK(hipEventSynchronize(ev_[kPhaseCount]));

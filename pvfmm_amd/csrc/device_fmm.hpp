@@ -62,6 +62,9 @@ class DevicePlanBase {
   // d_den: user layout (k0 per source, input order) for n_vec vectors with stride k0*n_src;
   // d_out: user layout (k1 per target, input order), overwritten.
   virtual void evaluate(const double* d_den, double* d_out, int n_vec, double den_scale, double out_scale) = 0;
+  // One vector, with the addresses of d_den and d_out read from device memory when the launches
+  // run: the form a recorded graph replays on any buffers.
+  virtual void evaluate_slots(const double* const* den_slot, double* const* out_slot) = 0;
   // The transpose of evaluate's linear map (same scales): d_g in the user layout of the
   // targets (k1 per target), d_out in that of the sources (k0 per source), overwritten.  Built
   // on first use; symmetric kernels only (adjoint_supported()).

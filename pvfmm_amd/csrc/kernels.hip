@@ -117,7 +117,9 @@ constexpr int kFillPerThread = 8;
 template <typename Real>
 __global__ __launch_bounds__(256) void k_begin(int64_t n, int k0, const double* __restrict__ in, const int64_t* __restrict__ perm,
                                                double scal, Real* __restrict__ den, int64_t in_stride, int gb, int nv,
-                                               uint4* __restrict__ a, int64_t na, int fa, uint4* __restrict__ b, int64_t nb) {
+                                               uint4* __restrict__ a, int64_t na, int fa, uint4* __restrict__ b, int64_t nb,
+                                               const double* const* __restrict__ in_slot) {
+  if (in_slot) in = *in_slot;
   int blk = blockIdx.x;
   if (blk < gb * nv) {
     const int v = blk / gb;
@@ -143,7 +145,8 @@ __global__ __launch_bounds__(256) void k_begin(int64_t n, int k0, const double* 
 }
 
 __global__ void k_scatter_output(int64_t n, int k1, const double* __restrict__ val, const int64_t* __restrict__ perm,
-                                 double scal, double* __restrict__ out, int64_t out_stride) {
+                                 double scal, double* __restrict__ out, int64_t out_stride, double* const* __restrict__ out_slot) {
+  if (out_slot) out = *out_slot;
   const int v = blockIdx.y;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t p = perm[i];
@@ -2288,6 +2291,20 @@ __global__ __launch_bounds__(256, 1) void k_hadamard_split3(int M_dim, int n_til
   }
 }
 
+// dst[i] = src.p[i], i < n: buffer addresses into device memory, as kernel arguments
+__global__ void k_set_pointers(int n, PointerList src, void** __restrict__ dst) {
+  if ((int)threadIdx.x < n) dst[threadIdx.x] = src.p[threadIdx.x];
+}
+void set_pointers(hipStream_t s, int n, void* const* src, void** dst) {
+  for (int i = 0; i < n; i += kPointerList) {
+    const int m = std::min(kPointerList, n - i);
+    PointerList l = {};
+    for (int q = 0; q < m; q++) l.p[q] = src[i + q];
+    hipLaunchKernelGGL(k_set_pointers, dim3(1), dim3(kPointerList), 0, s, m, l, dst + i);
+    HIP_LAUNCH_CHECK();
+  }
+}
+
 // ----------------------------------------------------------------------------- launchers
 static inline int grid_for(int64_t n, int block) {
   int64_t g = (n + block - 1) / block;
@@ -2305,20 +2322,21 @@ void DeviceKernels<Real>::gather_density(hipStream_t s, int64_t n, int k0, const
 }
 template <typename Real>
 void DeviceKernels<Real>::begin(hipStream_t s, int64_t n, int k0, const double* in, const int64_t* perm, double scal, Real* den,
-                                int n_vec, int64_t in_stride, Real* za, int64_t na, Real* zb, int64_t nb) {
+                                int n_vec, int64_t in_stride, Real* za, int64_t na, Real* zb, int64_t nb,
+                                const double* const* in_slot) {
   const int64_t per = 256 * kFillPerThread, na16 = (na * (int64_t)sizeof(Real) + 15) / 16, nb16 = (nb * (int64_t)sizeof(Real) + 15) / 16;
   const int64_t gb = (n + 255) / 256, fa = (na16 + per - 1) / per, fb = (nb16 + per - 1) / per, blocks = gb * n_vec + fa + fb;
   if (blocks == 0) return;
   if (blocks >= (1ll << 31)) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
   hipLaunchKernelGGL(k_begin<Real>, dim3((unsigned)blocks), dim3(256), 0, s, n, k0, in, perm, scal, den, in_stride, (int)gb, n_vec,
-                     reinterpret_cast<uint4*>(za), na16, (int)fa, reinterpret_cast<uint4*>(zb), nb16);
+                     reinterpret_cast<uint4*>(za), na16, (int)fa, reinterpret_cast<uint4*>(zb), nb16, in_slot);
   HIP_LAUNCH_CHECK();
 }
 template <typename Real>
 void DeviceKernels<Real>::scatter_output(hipStream_t s, int64_t n, int k1, const double* val, const int64_t* perm,
-                                         double scal, double* out, int n_vec, int64_t out_stride) {
+                                         double scal, double* out, int n_vec, int64_t out_stride, double* const* out_slot) {
   if (n == 0) return;
-  hipLaunchKernelGGL(k_scatter_output, dim3(grid_for(n, 256), n_vec), dim3(256), 0, s, n, k1, val, perm, scal, out, out_stride);
+  hipLaunchKernelGGL(k_scatter_output, dim3(grid_for(n, 256), n_vec), dim3(256), 0, s, n, k1, val, perm, scal, out, out_stride, out_slot);
   HIP_LAUNCH_CHECK();
 }
 // zeroes n values of T: 16-byte stores over the aligned whole words, scalar stores for the rest

@@ -39,12 +39,16 @@ struct DeviceKernels {
                              double scal, Real* den, int n_vec, int64_t in_stride);
   // out[k1*perm[i] + j] = val[j*n + i] * scal (user AoS output, in input order)
   static void scatter_output(hipStream_t s, int64_t n, int k1, const double* val, const int64_t* perm,
-                             double scal, double* out, int n_vec, int64_t out_stride);
+                             double scal, double* out, int n_vec, int64_t out_stride, double* const* out_slot = nullptr);
   static void fill(hipStream_t s, Real* p, int64_t n);
+  // A non-null slot (here and in scatter_output) is a device address that holds the address of the
+  // caller's buffer, which the kernel then takes instead: a recorded launch works on whatever
+  // buffers the slots name when it runs (set_pointers).
   // gather_density, and za[0, na) and zb[0, nb) zeroed, up to the next 16-byte word (16-byte
   // aligned buffers of whole words), in one launch
   static void begin(hipStream_t s, int64_t n, int k0, const double* in, const int64_t* perm, double scal, Real* den, int n_vec,
-                    int64_t in_stride, Real* za, int64_t na, Real* zb, int64_t nb);
+                    int64_t in_stride, Real* za, int64_t na, Real* zb, int64_t nb,
+                    const double* const* in_slot = nullptr);
   // Periodic (PXYZ) post-processing of FMM_Pts::PostProcessing (include/fmm_pts.txx:5740-5774):
   // val[j*n + i] -= sum_c avg_c V_cj(x_i), avg_c the sum of component c over the root's K0
   // equivalent values eq_root[p*e0 + c], V the kernel's analytic potential of a uniform unit
@@ -142,6 +146,13 @@ struct DeviceKernels {
                         int K1, int e1, int m, const int32_t* lattice, const int32_t* lat_inv, int ns,
                         const Real* scal, int nv = 1, int64_t y_vs = 0, int64_t dn_vs = 0);
 };
+
+// Writes n addresses to device memory, in stream order (they travel as kernel arguments).
+constexpr int kPointerList = 256;
+struct PointerList {
+  void* p[kPointerList];
+};
+void set_pointers(hipStream_t s, int n, void* const* src, void** dst);
 
 // FP64 all-pairs sum on the device (AoS src[3n], den[k0 n], trg[3n], out[k1 n] device arrays);
 // kind as in DeviceKernels (0 laplace potential, 1 laplace gradient, 2 stokes velocity).

@@ -381,10 +381,10 @@ class PtFMMTree:
 
 class PtFMMBatch:
     """Set-up trees of independent point clouds evaluated together: the first evaluation
-    records every tree's evaluation into one HIP graph (one branch per tree), later calls with
-    the same tensors replay it with one graph launch.  A tree set up again (with another PtFMM
-    or n_vec_max) or retuned makes the next call record the graph again.  Replays are ordered
-    against eager evaluations of the same trees (they share the trees' scratch buffers), also
+    records every tree's evaluation into one HIP graph (one branch per tree), later calls replay
+    it with one graph launch, on whatever tensors they pass.  A tree set up again (with another
+    PtFMM or n_vec_max) or retuned makes the next call record the graph again.  Replays are
+    ordered against eager evaluations of the same trees (they share the trees' scratch buffers), also
     with sync=False.  The trees must stay alive and set up."""
 
     def __init__(self, trees):
