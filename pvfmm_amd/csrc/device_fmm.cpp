@@ -266,6 +266,21 @@ class DevicePlan final : public DevicePlanBase {
     int64_t partners = 0, max_partners = 0, staged_delta = 0;
   };
   TileSet vt_;
+  // rows of A (K) -> rank R -> rows of C (N): one launch where that is the faster form, else two
+  // products with the intermediate rows seq of ctmp_
+  void pair(const typename DeviceOps<Real>::PackedPair& p, const DBuf<Real>& B1, const DBuf<Real>& B2, int M, int K, int R, int N,
+            const Real* A, const int32_t* ra, const Real* alpha1, const int32_t* seq, Real* C, const int32_t* rc,
+            const Real* alpha2, bool accumulate, int nv, int64_t avs, int64_t cvs) {
+    if (p.use && DeviceKernels<Real>::gemm_pair_pays(K, (int64_t)M * nv)) {
+      DeviceKernels<Real>::gemm_pair(st_, M, K, R, N, A, ra, K, p.B1.p, alpha1, p.B2.p, C, rc, N, alpha2, accumulate, nv, avs, cvs);
+      return;
+    }
+    const int sp = tuning.gemm_split_blocks;
+    DeviceKernels<Real>::gemm_rows(st_, M, R, K, A, ra, K, B1.p, ctmp_.p, seq, R, alpha1, false, gemm_work_.p, gemm_work_elems_, sp,
+                                   nv, avs, ctmp_vs_);
+    DeviceKernels<Real>::gemm_rows(st_, M, N, R, ctmp_.p, seq, R, B2.p, C, rc, N, alpha2, accumulate, gemm_work_.p,
+                                   gemm_work_elems_, sp, nv, ctmp_vs_, cvs);
+  }
   // operands of the fp16 Hadamard with run scales in `rs` (kept until the launch returns)
   HadamardParts hp_;
   const HadamardParts& hparts(DBuf<float>& rs) {
@@ -1038,10 +1053,8 @@ class DevicePlan final : public DevicePlanBase {
     K::p2p_surface(st_, ek, a.n_w, a.w_node.p, a.w_ptr.p, a.w_items.p, a.tb.p, a.te.p, a.center.p, a.nsz.p, kRad0,
                    ops_->unit_surf.p, ns_, tx_.p, a.tden.p, n_trg_, eq_.p, a.w_node.p, K0_, true, nv, g_vs, eq_vs_);
     // D2T GEMMs^T: equivalent -> check potential of each target leaf
-    K::gemm_rows(st_, n_l2t_, rd_, K0_, eq_.p, l2t_rc_.p, K0_, a.op->dc2de1.p, ctmp_.p, l2t_seq_.p, rd_, nullptr, false,
-                 gemm_work_.p, gemm_work_elems_, sp, nv, eq_vs_, ctmp_vs_);
-    K::gemm_rows(st_, n_l2t_, K1_, rd_, ctmp_.p, l2t_seq_.p, rd_, a.op->dc2de0.p, dn_.p, l2t_ra_.p, K1_, l2t_alpha_.p, true,
-                 gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, dn_vs_);
+    pair(a.op->d2t_pair, a.op->dc2de1, a.op->dc2de0, n_l2t_, K0_, rd_, K1_, eq_.p, l2t_rc_.p, nullptr, l2t_seq_.p, dn_.p, l2t_ra_.p,
+         l2t_alpha_.p, true, nv, eq_vs_, dn_vs_);
     // D2D^T, bottom-up: parent += [8 children] x [D2D_0 .. D2D_7]^T
     for (int l = max_depth_; l >= dn_min_ + 1; l--) {
       const LevelRows& L = *l2l_[l - 1];
@@ -1088,10 +1101,8 @@ class DevicePlan final : public DevicePlanBase {
       }
     }
     // S2U GEMMs^T: upward equivalent -> check potential of each source leaf
-    K::gemm_rows(st_, n_s2m_, ru_, K0_, eq_.p, s2m_node_.p, K0_, a.op->uc2ue1.p, ctmp_.p, s2m_orow_.p, ru_, nullptr, false,
-                 gemm_work_.p, gemm_work_elems_, sp, nv, eq_vs_, ctmp_vs_);
-    K::gemm_rows(st_, n_s2m_, K1_, ru_, ctmp_.p, s2m_orow_.p, ru_, a.op->uc2ue0.p, chk_.p, s2m_orow_.p, K1_, s2m_alpha_.p, false,
-                 gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, chk_vs_);
+    pair(a.op->s2u_pair, a.op->uc2ue1, a.op->uc2ue0, n_s2m_, K0_, ru_, K1_, eq_.p, s2m_node_.p, nullptr, s2m_orow_.p, chk_.p,
+         s2m_orow_.p, s2m_alpha_.p, false, nv, eq_vs_, chk_vs_);
     // (S2U P2P)^T: upward check surface (RAD1) -> the leaf's source points
     K::far_points(st_, ek, n_s2m_, s2m_node_.p, a.iota.p, s2m_node_.p, a.s2u_den.p, a.s2u_rad.p, a.sb.p, a.se.p,
                   a.center.p, a.nsz.p, ops_->unit_surf.p, ns_, sx_.p, n_src_, chk_.p, a.sval.p, true, nv, chk_vs_, o_vs);
@@ -1126,10 +1137,8 @@ class DevicePlan final : public DevicePlanBase {
     K::p2p_surface(st_, ek, n_s2m_, s2m_node_.p, s2m_ptr_.p, s2m_items_.p, src_begin_.p, src_end_.p, center_.p, node_size_.p,
                    kRad1, ops_->unit_surf.p, ns_, sx_.p, sden_.p, n_src_, chk_.p, s2m_orow_.p, K1_, false, nv, den_vs, chk_vs_);
     mark(2);
-    K::gemm_rows(st_, n_s2m_, ru_, K1_, chk_.p, s2m_orow_.p, K1_, ops_->uc2ue0.p, ctmp_.p, s2m_orow_.p, ru_, s2m_alpha_.p, false,
-                 gemm_work_.p, gemm_work_elems_, sp, nv, chk_vs_, ctmp_vs_);
-    K::gemm_rows(st_, n_s2m_, K0_, ru_, ctmp_.p, s2m_orow_.p, ru_, ops_->uc2ue1.p, eq_.p, s2m_node_.p, K0_, nullptr, false,
-                 gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, eq_vs_);
+    pair(ops_->s2u_pair, ops_->uc2ue0, ops_->uc2ue1, n_s2m_, K1_, ru_, K0_, chk_.p, s2m_orow_.p, s2m_alpha_.p, s2m_orow_.p, eq_.p,
+         s2m_node_.p, nullptr, false, nv, chk_vs_, eq_vs_);
     mark(3);
     // U2U, bottom-up: parent row = [8 children] x stacked U2U
     for (int l = max_depth_ - 1; l >= up_min_; l--) {
@@ -1194,10 +1203,8 @@ class DevicePlan final : public DevicePlanBase {
     }
     mark(9);
     // D2T: check -> equivalent
-    K::gemm_rows(st_, n_l2t_, rd_, K1_, dn_.p, l2t_ra_.p, K1_, ops_->dc2de0.p, ctmp_.p, l2t_seq_.p, rd_, l2t_alpha_.p, false,
-                 gemm_work_.p, gemm_work_elems_, sp, nv, dn_vs_, ctmp_vs_);
-    K::gemm_rows(st_, n_l2t_, K0_, rd_, ctmp_.p, l2t_seq_.p, rd_, ops_->dc2de1.p, eq_.p, l2t_rc_.p, K0_, nullptr, false,
-                 gemm_work_.p, gemm_work_elems_, sp, nv, ctmp_vs_, eq_vs_);
+    pair(ops_->d2t_pair, ops_->dc2de0, ops_->dc2de1, n_l2t_, K1_, rd_, K0_, dn_.p, l2t_ra_.p, l2t_alpha_.p, l2t_seq_.p, eq_.p,
+         l2t_rc_.p, nullptr, false, nv, dn_vs_, eq_vs_);
     mark(10);
     // equivalent surfaces -> targets (own downward equivalent + W list)
     K::far_points(st_, pk, n_tleaf_, t_leaf_.p, far_ptr_.p, far_node_.p, far_den_.p, far_rad_.p, trg_begin_.p, trg_end_.p,

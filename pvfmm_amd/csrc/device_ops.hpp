@@ -54,6 +54,13 @@ class DeviceOps final : public DeviceOpsBase {
   // products).  Applied as two GEMMs they cost 9 K r instead of 8 K^2 multiply-adds per row.
   bool u2u_fact = false, d2d_fact = false;
   DBuf<Real> u2ur, d2dr;  // 8 K0 x ru, rd x 8 K1
+  // the factors packed for the one-launch product of the leaves' maps, where their shapes fit it and
+  // some number of rows takes it
+  struct PackedPair {
+    DBuf<Real> B1, B2;
+    bool use = false;
+  };
+  PackedPair s2u_pair, d2t_pair;  // uc2ue0 uc2ue1, dc2de0 dc2de1
   DBuf<Real> unit_surf;
   DBuf<int32_t> lattice, lattice_inv;
   VGrid grid;
@@ -116,6 +123,10 @@ class DeviceOps final : public DeviceOpsBase {
       }
     }
     HIP_CHECK(hipStreamSynchronize(s));
+    DeviceKernels<Real>::gemm_pair_init();
+    pack_pair(s, uc2ue0, K1, ru, uc2ue1, K0, s2u_pair);
+    pack_pair(s, dc2de0, K1, rd, dc2de1, K0, d2t_pair);
+    HIP_CHECK(hipStreamSynchronize(s));
     unit_surf.upload(std::vector<Real>(O.unit_surf.begin(), O.unit_surf.end()), total);
     lattice.upload(O.lattice, total);
     std::vector<int32_t> inv((size_t)O.m * O.m * O.m, -1);
@@ -153,6 +164,7 @@ class DeviceOps final : public DeviceOpsBase {
   // The transposed operators of the adjoint evaluation, in the padded layouts of the forward ones
   struct Transposed {
     DBuf<Real> uc2ue0, uc2ue1, dc2de0, dc2de1, u2u, d2d, u2ur, d2dr;
+    PackedPair d2t_pair, s2u_pair;  // dc2de1^T dc2de0^T, uc2ue1^T uc2ue0^T
   };
   const Transposed& transposed() {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -173,6 +185,8 @@ class DeviceOps final : public DeviceOpsBase {
       turn(d2d, K1, 8 * K1, t->d2d);
       turn(u2ur, 8 * K0, ru, t->u2ur);
       turn(d2dr, rd, 8 * K1, t->d2dr);
+      pack_pair(st.s, t->dc2de1, K0, rd, t->dc2de0, K1, t->d2t_pair);
+      pack_pair(st.s, t->uc2ue1, K0, ru, t->uc2ue0, K1, t->s2u_pair);
       HIP_CHECK(hipStreamSynchronize(st.s));
       tr_ = std::move(t);
     }
@@ -185,6 +199,15 @@ class DeviceOps final : public DeviceOpsBase {
     Stream() { HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking)); }
     ~Stream() { (void)hipStreamDestroy(s); }
   };
+  void pack_pair(hipStream_t s, const DBuf<Real>& f0, int K, int r, const DBuf<Real>& f1, int N, PackedPair& p) {
+    using D = DeviceKernels<Real>;
+    p.use = D::gemm_pair_fits(K, r) && D::gemm_pair_pays(K, 4 * (int64_t)K);
+    if (!p.use) return;
+    p.B1.alloc(D::packed_size(K, r), &bytes_);
+    p.B2.alloc(D::packed_size(r, N), &bytes_);
+    D::pack_matrix(s, f0.p, K, r, p.B1.p);
+    D::pack_matrix(s, f1.p, r, N, p.B2.p);
+  }
   void spectra(hipStream_t s, DBuf<double>& G) {
     G.alloc((int64_t)2 * 343 * O_.ker.e0 * O_.ker.e1 * grid.M, nullptr);
     transfer_spectra(s, O_.ker.exp_kind, O_.m, G.p);

@@ -1019,6 +1019,144 @@ __global__ void k_gemm_reduce(int M, int N, int ksplit, const Real* __restrict__
   }
 }
 
+// ----------------------------------------------------------------------------- product with two factors
+// C[rc[i]] (+)= alpha2[i] * (alpha1[i] * A[ra[i]] * B1) * B2 for the check-to-equivalent maps of the
+// leaves (K -> rank R -> N), in one launch.  A block of 8 waves keeps 16 rows of A over the whole of
+// K in LDS, its waves take the 16-column tiles of the product in turn (two at a time) with B read
+// from L2 in the lane order of the matrix instruction (pack_matrix: one 4-vector per lane and
+// 16x16 block), the 16 rows of A B1 go to LDS and the same happens with B2.  There is no barrier
+// and no LDS store among the products, and nothing but A and C moves through memory; the loads of B
+// run four steps ahead, which 8 waves of up to 256 registers per CU leave room for (half as many
+// spill in FP64).  Bound by the matrix rate where the blocks fill the chip (FP64), by the one pass of
+// a CU over both factors where they do not.  gemm_pair_pays has the figures of both forms.
+template <typename Real>
+struct PairShape {
+  static constexpr int BM = 16, NT = 512, PAD = 16 / (int)sizeof(Real);  // an odd number of 16-byte words per row
+  static int cols(int k) { return (k + 15) / 16 * 16; }
+  static size_t lds(int K, int R) { return (size_t)BM * (cols(K) + cols(R) + 2 * PAD) * sizeof(Real); }
+};
+
+// 4 consecutive values from LDS (16-byte aligned)
+__device__ __forceinline__ floatx4 lds4(const float* p) { return *reinterpret_cast<const floatx4*>(p); }
+__device__ __forceinline__ doublex4 lds4(const double* p) {
+  const double2 a = reinterpret_cast<const double2*>(p)[0], b = reinterpret_cast<const double2*>(p)[1];
+  return doublex4{a.x, a.y, b.x, b.y};
+}
+
+template <typename Real>
+__device__ __forceinline__ void pair_tiles(const Real* __restrict__ As, int lda, int nk, const Real* __restrict__ Bp, int nt, int t0,
+                                           int t1, typename Mfma<Real>::V4 (&acc)[2]) {
+  using MF = Mfma<Real>;
+  using V4 = typename MF::V4;
+  const int l = threadIdx.x & 63;
+  const Real* a = As + (l & 15) * lda + 4 * (l >> 4);
+  const V4* b0 = reinterpret_cast<const V4*>(Bp) + (int64_t)t0 * 64 + l;
+  const V4* b1 = reinterpret_cast<const V4*>(Bp) + (int64_t)t1 * 64 + l;
+  acc[0] = acc[1] = V4{0, 0, 0, 0};
+  // B of PF steps is read ahead of the products of the PF before
+  constexpr int PF = 4;
+  V4 vb[2][PF][2];
+  auto load = [&](int buf, int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < PF; i++) {
+      const int64_t at = (int64_t)min(k0 + i, nk - 1) * nt * 64;
+      vb[buf][i][0] = b0[at];
+      vb[buf][i][1] = b1[at];
+    }
+  };
+  auto step = [&](int buf, int k0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < PF; i++)
+      if (k0 + i < nk) {
+        const V4 av = lds4(a + 16 * (k0 + i));
+#pragma unroll
+        for (int q = 0; q < 4; q++) acc[0] = MF::mma(av[q], vb[buf][i][0][q], acc[0]);
+#pragma unroll
+        for (int q = 0; q < 4; q++) acc[1] = MF::mma(av[q], vb[buf][i][1][q], acc[1]);
+      }
+  };
+  load(0, 0);
+  for (int k0 = 0; k0 < nk; k0 += 2 * PF) {
+    load(1, k0 + PF);
+    step(0, k0);
+    load(0, k0 + 2 * PF);
+    step(1, k0 + PF);
+  }
+}
+
+template <typename Real>
+__global__ __launch_bounds__(512, 2) void k_gemm_pair(int M, int K, int R, int N, const Real* __restrict__ A,
+                                                      const int32_t* __restrict__ ra, int64_t lda, const Real* __restrict__ B1,
+                                                      const Real* __restrict__ alpha1, const Real* __restrict__ B2,
+                                                      Real* __restrict__ C, const int32_t* __restrict__ rc, int64_t ldc,
+                                                      const Real* __restrict__ alpha2, bool accumulate, int Mv, int64_t avs,
+                                                      int64_t cvs) {
+  using MF = Mfma<Real>;
+  using V4 = typename MF::V4;
+  constexpr int BM = PairShape<Real>::BM, NT = PairShape<Real>::NT, PAD = PairShape<Real>::PAD, NW = NT / 64;
+  extern __shared__ __align__(32) unsigned char pair_smem[];
+  const int kt = (K + 15) / 16, rt = (R + 15) / 16, ct = (N + 15) / 16;
+  const int la = 16 * kt + PAD, lt = 16 * rt + PAD;
+  Real* As = reinterpret_cast<Real*>(pair_smem);
+  Real* T = As + BM * la;
+  const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, m0 = blockIdx.x * BM;
+  for (int e = tid; e < BM * 4 * kt; e += NT) {
+    const int row = e / (4 * kt), k = 4 * (e - row * 4 * kt), gm = m0 + row;
+    V4 v = {0, 0, 0, 0};
+    if (gm < M && k < K) {  // K is a multiple of 4
+      const int vec = gm / Mv, i = gm - vec * Mv;
+      v = *reinterpret_cast<const V4*>(A + vec * avs + (int64_t)ra[i] * lda + k);
+    }
+    Real* d = As + row * la + k;
+#pragma unroll
+    for (int q = 0; q < 4; q++) d[q] = v[q];
+  }
+  __syncthreads();
+  V4 acc[2];
+  for (int t = w; t < rt; t += 2 * NW) {
+    const int t1 = t + NW < rt ? t + NW : t;  // a lone tile runs twice
+    pair_tiles<Real>(As, la, kt, B1, rt, t, t1, acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int row = MF::row(l, r), gm = m0 + row;
+      const Real al = alpha1 && gm < M ? alpha1[gm % Mv] : Real(1);
+      T[row * lt + 16 * t + (l & 15)] = al * acc[0][r];
+      if (t1 != t) T[row * lt + 16 * t1 + (l & 15)] = al * acc[1][r];
+    }
+  }
+  __syncthreads();
+  for (int t = w; t < ct; t += 2 * NW) {
+    const int t1 = t + NW < ct ? t + NW : t;
+    pair_tiles<Real>(T, lt, rt, B2, ct, t, t1, acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int gm = m0 + MF::row(l, r);
+      if (gm >= M) continue;
+      const int vec = gm / Mv, i = gm - vec * Mv;
+      Real* c = C + vec * cvs + (int64_t)rc[i] * ldc;
+      const Real al = alpha2 ? alpha2[i] : Real(1);
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int n = 16 * (h ? t1 : t) + (l & 15);
+        if ((h && t1 == t) || n >= N) continue;
+        c[n] = accumulate ? fma(al, acc[h][r], c[n]) : al * acc[h][r];
+      }
+    }
+  }
+}
+
+// out[(kt * nt + n) * 64 + l][q] = in[16 kt + 4 (l / 16) + q][16 n + l % 16], zero outside rows x cols
+template <typename Real>
+__global__ __launch_bounds__(256) void k_pack_matrix(const Real* __restrict__ in, int rows, int cols, Real* __restrict__ out) {
+  const int nt = (cols + 15) / 16;
+  const int64_t idx = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (idx >= (int64_t)((rows + 15) / 16) * nt * 256) return;
+  const int q = (int)(idx & 3), l = (int)(idx >> 2) & 63;
+  const int64_t b = idx >> 8;
+  const int k = 16 * (int)(b / nt) + 4 * (l >> 4) + q, n = 16 * (int)(b % nt) + (l & 15);
+  out[idx] = k < rows && n < cols ? in[(int64_t)k * cols + n] : Real(0);
+}
+
 // ----------------------------------------------------------------------------- V list: DFTs
 // Twiddles w[k] = exp(sign * 2 pi i k / n1), kept in LDS
 template <typename Real>
@@ -2548,6 +2686,57 @@ void DeviceKernels<Real>::gemm_rows(hipStream_t s, int M, int N, int K, const Re
     GEMM_LAUNCH(false, false);
   }
 #undef GEMM_LAUNCH
+  HIP_LAUNCH_CHECK();
+}
+
+template <typename Real>
+int64_t DeviceKernels<Real>::packed_size(int rows, int cols) {
+  return (int64_t)((rows + 15) / 16) * ((cols + 15) / 16) * 256;
+}
+template <typename Real>
+void DeviceKernels<Real>::pack_matrix(hipStream_t s, const Real* in, int rows, int cols, Real* out) {
+  const int64_t n = packed_size(rows, cols);
+  if (n == 0) return;
+  hipLaunchKernelGGL(k_pack_matrix<Real>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, rows, cols, out);
+  HIP_LAUNCH_CHECK();
+}
+template <typename Real>
+bool DeviceKernels<Real>::gemm_pair_fits(int K, int R) {
+  return K % 4 == 0 && PairShape<Real>::lds(K, R) <= kPairLds;
+}
+// Both forms in us, one product pair, at 512 / 2047 / 4093 / 8189 / 32700 rows, one launch : two
+// products of tiles (split over K where the rows are few):
+//   FP64 K = 152:  22 : 22    23 : 32    25 : 44    45 : 59   163 : 120
+//        K = 296:  43 : 32    46 : 53    49 : 76    91 : 104  336 : 296
+//        K = 488:  77 : 42    84 : 78    88 : 122  169 : 184  604 : 648
+//   FP32 K = 152:  15 : 19    15 : 22    16 : 27    26 : 37    83 : 57
+//        K = 296:  21 : 21    22 : 31    24 : 43    41 : 46   141 : 115
+//        K = 488:  28 : 22    30 : 38    33 : 52    58 : 62   213 : 185
+//        K = 888:  86 : 37    90 : 75    99 : 110  200 : 188  717 : 635
+// Up to 4096 rows (16 per CU) the one launch takes the time of one block, which grows with K, and two
+// blocks per CU that of two; with few rows the K split of the two products is the shorter chain, and with
+// many rows their tiles read the factors less often (which at large K in FP64 the matrix rate covers).
+template <typename Real>
+bool DeviceKernels<Real>::gemm_pair_pays(int K, int64_t rows) {
+  if constexpr (sizeof(Real) == 8) return rows >= 4 * (int64_t)K && (rows <= 8192 || K >= 384);
+  return K <= 512 && rows <= 8192 && (K <= 256 || rows >= 4 * (int64_t)K);
+}
+template <typename Real>
+void DeviceKernels<Real>::gemm_pair_init() {
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_pair<Real>), hipFuncAttributeMaxDynamicSharedMemorySize, kPairLds) !=
+      hipSuccess)
+    throw_device_error(hipGetLastError(), __FILE__, __LINE__);
+}
+template <typename Real>
+void DeviceKernels<Real>::gemm_pair(hipStream_t s, int M, int K, int R, int N, const Real* A, const int32_t* ra, int64_t lda,
+                                    const Real* B1, const Real* alpha1, const Real* B2, Real* C, const int32_t* rc, int64_t ldc,
+                                    const Real* alpha2, bool accumulate, int nv, int64_t avs, int64_t cvs) {
+  if (M <= 0 || N <= 0 || K <= 0 || R <= 0 || nv <= 0) return;
+  const int64_t rows = (int64_t)M * nv;
+  if (rows >= (1ll << 31) || !gemm_pair_fits(K, R) || lda % 4 != 0 || avs % 4 != 0 || (reinterpret_cast<uintptr_t>(A) % 32) != 0)
+    throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
+  hipLaunchKernelGGL(k_gemm_pair<Real>, dim3((unsigned)((rows + 15) / 16)), dim3(512), PairShape<Real>::lds(K, R), s, (int)rows, K, R,
+                     N, A, ra, lda, B1, alpha1, B2, C, rc, ldc, alpha2, accumulate, M, avs, cvs);
   HIP_LAUNCH_CHECK();
 }
 

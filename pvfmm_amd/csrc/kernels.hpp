@@ -30,6 +30,8 @@ struct FarSplit {
   int64_t part_vs = 0;
 };
 
+constexpr int kPairLds = 160 * 1024;  // most LDS of a gemm_pair block
+
 // Point-kernel kinds of the device code: 0 laplace potential (1x1), 1 laplace gradient
 // (1x3, r = x_trg - x_src, i.e. minus the gradient of the potential), 2 stokes velocity (3x3).
 template <typename Real>
@@ -100,6 +102,20 @@ struct DeviceKernels {
                         const Real* B, Real* C, const int32_t* rc, int64_t ldc, const Real* alpha,
                         bool accumulate, Real* work = nullptr, int64_t work_elems = 0, int split_blocks = 1024,
                         int nv = 1, int64_t avs = 0, int64_t cvs = 0);
+
+  // C[rc[i]*ldc : +N] (+)= alpha2[i] * (alpha1[i] * A[ra[i]*lda : +K] * B1) * B2, B1 (K x R) and B2
+  // (R x N) in packed form (pack_matrix into packed_size values), alphas may be null, vectors as
+  // gemm_rows.  For shapes that fit (gemm_pair_fits: K a multiple of 4, rows of A and A B1 within
+  // the LDS); A 32-byte aligned, lda and avs multiples of 4; gemm_pair_init once per device.
+  static bool gemm_pair_fits(int K, int R);
+  // whether it is faster than two gemm_rows at this many rows
+  static bool gemm_pair_pays(int K, int64_t rows);
+  static void gemm_pair_init();
+  static int64_t packed_size(int rows, int cols);
+  static void pack_matrix(hipStream_t s, const Real* in, int rows, int cols, Real* out);
+  static void gemm_pair(hipStream_t s, int M, int K, int R, int N, const Real* A, const int32_t* ra, int64_t lda, const Real* B1,
+                        const Real* alpha1, const Real* B2, Real* C, const int32_t* rc, int64_t ldc, const Real* alpha2,
+                        bool accumulate, int nv, int64_t avs, int64_t cvs);
 
   // V-list: forward DFT of the 8 children's equivalent densities of each source parent.
   // X layout [slot][f][8*e0] complex, component-major within a row ([slot][f][i][child]).  lattice[3p..3p+2] is the m^3 lattice cell of surface
