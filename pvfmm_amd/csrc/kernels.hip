@@ -1052,7 +1052,11 @@ __device__ __forceinline__ void pair_tiles(const Real* __restrict__ As, int lda,
   const Real* a = As + (l & 15) * lda + 4 * (l >> 4);
   const V4* b0 = reinterpret_cast<const V4*>(Bp) + (int64_t)t0 * 64 + l;
   const V4* b1 = reinterpret_cast<const V4*>(Bp) + (int64_t)t1 * 64 + l;
-  acc[0] = acc[1] = V4{0, 0, 0, 0};
+  // FP32: one partial sum per value of q, as accurate as the K split of the two products
+  constexpr int NA = sizeof(Real) == 4 ? 4 : 1;
+  V4 part[NA][2];
+#pragma unroll
+  for (int q = 0; q < NA; q++) part[q][0] = part[q][1] = V4{0, 0, 0, 0};
   // B of PF steps is read ahead of the products of the PF before
   constexpr int PF = 4;
   V4 vb[2][PF][2];
@@ -1070,9 +1074,9 @@ __device__ __forceinline__ void pair_tiles(const Real* __restrict__ As, int lda,
       if (k0 + i < nk) {
         const V4 av = lds4(a + 16 * (k0 + i));
 #pragma unroll
-        for (int q = 0; q < 4; q++) acc[0] = MF::mma(av[q], vb[buf][i][0][q], acc[0]);
+        for (int q = 0; q < 4; q++) part[q % NA][0] = MF::mma(av[q], vb[buf][i][0][q], part[q % NA][0]);
 #pragma unroll
-        for (int q = 0; q < 4; q++) acc[1] = MF::mma(av[q], vb[buf][i][1][q], acc[1]);
+        for (int q = 0; q < 4; q++) part[q % NA][1] = MF::mma(av[q], vb[buf][i][1][q], part[q % NA][1]);
       }
   };
   load(0, 0);
@@ -1082,6 +1086,8 @@ __device__ __forceinline__ void pair_tiles(const Real* __restrict__ As, int lda,
     load(0, k0 + 2 * PF);
     step(1, k0 + PF);
   }
+#pragma unroll
+  for (int t = 0; t < 2; t++) acc[t] = NA == 4 ? (part[0][t] + part[1 % NA][t]) + (part[2 % NA][t] + part[3 % NA][t]) : part[0][t];
 }
 
 template <typename Real>
