@@ -2049,6 +2049,210 @@ __global__ __launch_bounds__(256, (hadamard_blocks_per_cu<Real, E0, FB, UMAX>())
       }
 }
 
+constexpr int kRunUnion = 240;  // most partners of a tile (an aligned 4x4x4 cube of parents has 216)
+
+// FP64 frequency-domain M2L for the scalar kernels over runs of tiles: one block of 8 waves per CU,
+// each with an equal share of the (pair of frequencies, tile) products.  Wave (fl, half, gp) multiplies
+// the 16-target groups 2 gp and 2 gp + 1 of a tile by 13 of the 26 transfer blocks of frequency fl,
+// which stay in its registers from tile to tile; a group's 4 MFMAs at an offset where none of its
+// targets has a partner are skipped.  While a tile's MFMAs run, the next tile's partner table and
+// spectra are read to registers and stored to the other half of the LDS, and the sums of the tile
+// before are added and written, with one barrier per tile.  The two halves of the offsets are added in
+// the order of k_hadamard_tiled.
+// FP64 MFMAs and the VALU take turns on a SIMD, so the operand addresses are kept to one exclusive or:
+// entry u is at byte 256 u of a half, its pair p of 16-byte chunks at p ^ (u % 8) (which spreads the
+// rows of an operand read over the banks as a pad would; two buffers leave no room for one), and the
+// partner table holds these byte offsets.
+// Against blocks that stage a tile, multiply and leave (k_hadamard_tiled, two per CU, 66% of the
+// cycles in MFMAs): 4612 -> 3912 us at 1M points of a nonuniform tree, m = 10, 663 -> 590 us at 10
+// tiles of a uniform one, m = 6 143 -> 133 us at 10 tiles, 39 -> 34 us at 2.  Of the 4612 us the
+// overlap took 3%, the cheaper addresses 6%, the skipped products 3%, the equal shares 3%.
+template <int UMAX>
+__global__ __launch_bounds__(512, 2) void k_hadamard_run(int M_dim, int n_tiles, int n_groups,
+                                                         const int32_t* __restrict__ tile_t0, const int32_t* __restrict__ tile_u0,
+                                                         const int32_t* __restrict__ usrc, const uint16_t* __restrict__ uidx,
+                                                         const uint32_t* __restrict__ gmask, const int32_t* __restrict__ offsets,
+                                                         const double* __restrict__ Vp, const double* __restrict__ X,
+                                                         double* __restrict__ Y, int64_t x_vs, int64_t y_vs) {
+  using MF = Mfma<double>;
+  using V4 = doublex4;
+  using V2 = double __attribute__((ext_vector_type(2)));
+  constexpr int NOFF = 26, NOW = NOFF / 2;   // offsets per wave
+  constexpr int RW = 16;                     // reals of a (slot, frequency) spectrum row
+  constexpr int EC = 16;                     // 16-byte chunks of an entry (2 frequencies)
+  constexpr int EPP = 512 / EC;              // entries per staging pass
+  constexpr int NPASS = (UMAX + EPP - 1) / EPP;
+  constexpr int UW = 64 * NOFF / 4;          // a tile's partner table as 8-byte words
+  static_assert(NPASS == 8 && NOW == 13 && UW <= 512, "staging schedule");
+  // a 64 KB half per tile: entries (entry UMAX stays zero), then the partner table [offset][row][group]
+  // as byte offsets of the entries; then the sums handed to the other half of the offsets
+  constexpr int HALF = 65536, TAB = (UMAX + 1) * EC * 16;
+  static_assert(TAB + 8 * UW <= HALF && UMAX < 256, "a half's layout");
+  __shared__ __align__(256) unsigned char smem[2 * HALF + 2 * 8 * 64 * sizeof(V4)];
+  V4* const ex = reinterpret_cast<V4*>(smem + 2 * HALF);
+  X += blockIdx.y * x_vs;  // density vector
+  Y += blockIdx.y * y_vs;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+  const int fl = w >> 2, half = (w >> 1) & 1, gp = w & 1;
+  const int row = l & 15, kg = l >> 4;
+  const int ob = half * NOW;
+  const int sc = tid & 15, su = tid >> 4;  // staging: chunk sc of entries su + EPP * i
+
+  if (tid < 2 * EC) *reinterpret_cast<V2*>(smem + (tid >> 4) * HALF + UMAX * 256 + 16 * (tid & 15)) = V2{0., 0.};
+
+  // the (frequency pair, tile) products, tiles fastest, in equal shares: block b runs on XCD b % 8,
+  // whose blocks take consecutive shares
+  const int64_t items = (int64_t)n_groups * n_tiles;
+  const int nb = gridDim.x, share = (blockIdx.x & 7) * (nb >> 3) + (blockIdx.x >> 3);
+  const int64_t i_end = items * (share + 1) / nb;
+  for (int64_t i0 = items * share / nb; i0 < i_end;) {
+    // a run of tiles of one frequency pair
+    const int fg = (int)(i0 / n_tiles), k0 = (int)(i0 - (int64_t)fg * n_tiles);
+    const int k1 = (int)min((int64_t)n_tiles, k0 + (i_end - i0));
+    i0 += k1 - k0;
+    const int f0 = 2 * fg, fn = min(2, M_dim - f0);
+    const bool live = fl < fn;  // waves past the last frequency compute, not store
+    const int f = f0 + (live ? fl : 0);
+    V4 bq[NOW];
+#pragma unroll
+    for (int j = 0; j < NOW; j++)
+      bq[j] = *reinterpret_cast<const V4*>(Vp + ((int64_t)offsets[ob + j] * M_dim + f) * 256 + l * 4);
+
+    int src[NPASS];
+    V2 val[NPASS / 2];  // two rounds of passes per tile
+    uint2 uw;
+    auto u0_of = [&](int k) __attribute__((always_inline)) { return tile_u0[min(k, k1)]; };
+    auto load_src = [&](int i, int at, int n) __attribute__((always_inline)) { src[i] = usrc[at + min(su + EPP * i, max(n - 1, 0))]; };
+    const double* xf = X + (int64_t)f0 * RW + 2 * (fn == 2 ? sc : sc & 7);
+    const uint32_t xstride = (uint32_t)M_dim * RW * sizeof(double);  // of a source slot; the host bounds M_dim
+    auto load_val = [&](int i) __attribute__((always_inline)) {
+      val[i % (NPASS / 2)] = *reinterpret_cast<const V2*>(reinterpret_cast<const char*>(xf) + (uint64_t)(uint32_t)src[i] * xstride);
+    };
+    auto load_uw = [&](int k) __attribute__((always_inline)) {
+      uw = reinterpret_cast<const uint2*>(uidx + (int64_t)min(k, k1 - 1) * 64 * NOFF)[min(tid, UW - 1)];
+    };
+    auto store_val = [&](int i, int buf, int n) __attribute__((always_inline)) {
+      const int u = su + EPP * i;
+      if (u < n) *reinterpret_cast<V2*>(smem + buf * HALF + u * 256 + ((16 * sc) ^ (32 * (u & 7)))) = val[i % (NPASS / 2)];
+    };
+    auto store_uw = [&](int buf) __attribute__((always_inline)) {
+      // byte offsets of the entries, with the key of their chunks
+      auto at = [](uint32_t two) { return (two << 8) | ((two & 0x00070007u) << 5); };
+      if (tid < UW) *reinterpret_cast<uint2*>(smem + buf * HALF + TAB + 8 * tid) = uint2{at(uw.x), at(uw.y)};
+    };
+    int ua = u0_of(k0), ub = u0_of(k0 + 1), uc = u0_of(k0 + 2);
+    {
+      const int n0 = ub - ua;
+#pragma unroll
+      for (int i = 0; i < NPASS; i++) load_src(i, ua, n0);
+      load_uw(k0);
+#pragma unroll
+      for (int h = 0; h < NPASS; h += NPASS / 2) {
+#pragma unroll
+        for (int i = h; i < h + NPASS / 2; i++) load_val(i);
+#pragma unroll
+        for (int i = h; i < h + NPASS / 2; i++) load_src(i, ub, uc - ub);
+#pragma unroll
+        for (int i = h; i < h + NPASS / 2; i++) store_val(i, 0, n0);
+      }
+      store_uw(0);
+    }
+#pragma unroll
+    for (int i = 0; i < NPASS; i++) asm volatile("" : "+v"(src[i]));
+#pragma unroll
+    for (int j = 0; j < NOW; j++) asm volatile("" : "+v"(bq[j]));
+    __syncthreads();
+
+    // a tile's sums: this wave finishes group 2 gp + half and hands the other to the wave of the other
+    // offsets; both are added and stored while the next tile's products run
+    V4 mine, theirs;
+    auto store_y = [&](int k) __attribute__((always_inline)) {
+      if (!live) return;
+      const int t0 = tile_t0[k], nt = tile_t0[k + 1] - t0, g = 2 * gp + half;
+      double* y = Y + ((int64_t)(t0 + 16 * g) * M_dim + f) * RW + row;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int tg = MF::row(l, r);
+        if (16 * g + tg < nt) y[(int64_t)tg * M_dim * RW] = mine[r] + theirs[r];
+      }
+    };
+    for (int k = k0; k < k1; k++) {
+      const int buf = (k - k0) & 1;
+      const int ud = u0_of(k + 3);
+      const int n1 = uc - ub, n2 = ud - uc;  // partners of tiles k + 1 and k + 2, 0 past the run
+      // offsets of the wave's half at which a target of group 2 gp + g has a partner
+      const uint32_t gm0 = __builtin_amdgcn_readfirstlane(gmask[4 * k + 2 * gp]) >> ob;
+      const uint32_t gm1 = __builtin_amdgcn_readfirstlane(gmask[4 * k + 2 * gp + 1]) >> ob;
+      const unsigned char* tab = smem + buf * HALF + TAB + ((ob * 16 + row) * 2 + gp) * 4;
+      const uint32_t lane_at = (uint32_t)(128 * fl + 32 * kg) | (uint32_t)(buf * HALF);
+      auto aop = [&](uint32_t u) __attribute__((always_inline)) {
+        const V2* e = reinterpret_cast<const V2*>(smem + (u ^ lane_at));
+        const V2 lo = e[0], hi = e[1];
+        return V4{lo.x, lo.y, hi.x, hi.y};
+      };
+      auto idx = [&](int j) __attribute__((always_inline)) { return *reinterpret_cast<const uint32_t*>(tab + 128 * j); };
+      V4 acc[2] = {V4{0, 0, 0, 0}, V4{0, 0, 0, 0}}, an[2];
+      uint32_t un = idx(0);
+      an[0] = aop(un & 0xFFFFu);
+      an[1] = aop(un >> 16);
+      un = idx(1);
+#pragma unroll
+      for (int j = 0; j < NOW; j++) {
+        V4 ac[2] = {an[0], an[1]};
+        if (j + 1 < NOW) {
+          an[0] = aop(un & 0xFFFFu);
+          an[1] = aop(un >> 16);
+        }
+        if (j + 2 < NOW) un = idx(j + 2);
+        // tile k + 1 in two rounds of four passes (with the entries of tile k + 2): read at steps 0, 1
+        // and 6, 7, two passes a step, stored four steps later
+        const int rd = j < 2 ? 2 * j : (j == 6 || j == 7) ? 2 * (j - 4) : NPASS;
+        const int wr = j == 4 || j == 5 ? 2 * (j - 4) : (j == 10 || j == 11) ? 2 * (j - 8) : NPASS;
+#pragma unroll
+        for (int i = 0; i < NPASS; i++) {
+          if (i != rd && i != rd + 1) continue;
+          if (EPP * i < n1) load_val(i);
+          if (EPP * i < n2) load_src(i, uc, n2);
+        }
+#pragma unroll
+        for (int i = 0; i < NPASS; i++)
+          if (i == wr || i == wr + 1) store_val(i, buf ^ 1, n1);
+        if (j == 2) load_uw(k + 1);
+        if (j == 8) store_uw(buf ^ 1);
+        if (j == 1) theirs = ex[(buf ^ 1) * 512 + (w ^ 2) * 64 + l];  // not used in the first tile
+        if (j == 3 && k > k0) store_y(k - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if ((gm0 >> j) & 1u) {
+#pragma unroll
+          for (int q = 0; q < 4; q++) acc[0] = MF::mma(ac[0][q], bq[j][q], acc[0]);
+        }
+        if ((gm1 >> j) & 1u) {
+#pragma unroll
+          for (int q = 0; q < 4; q++) acc[1] = MF::mma(ac[1][q], bq[j][q], acc[1]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // the entries of tile k + 2 are waited for here, where they have long arrived: at their first use
+      // the wait would cover loads and stores issued since
+#pragma unroll
+      for (int i = 0; i < NPASS; i++) asm volatile("" : "+v"(src[i]));
+      V4 other;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const double s0 = acc[0][r], s1 = acc[1][r];
+        mine[r] = half ? s1 : s0;
+        other[r] = half ? s0 : s1;
+      }
+      ex[buf * 512 + w * 64 + l] = other;
+      __syncthreads();
+      ub = uc;
+      uc = ud;
+    }
+    theirs = ex[((k1 - 1 - k0) & 1) * 512 + (w ^ 2) * 64 + l];
+    store_y(k1 - 1);
+  }
+}
+
 // FP32 frequency-domain M2L for the scalar kernels (k_hadamard_split) on the fp16 matrix
 // cores: operands are scaled by powers of two into fp16 range and split exactly into two fp16
 // parts x = x0 + x1 (x0 = RN(x), x1 = RN(x - x0): 22 significant bits, |x - x0 - x1| <=
@@ -2798,7 +3002,7 @@ int DeviceKernels<Real>::hadamard_union_max(int e0) {
   // blocks (one frequency each, fp16 parts) or one FP64 block (2 frequencies) in a CU's 160 KiB
   // of LDS (fuller tiles pay for the per-tile transfer-block loads over more targets)
   if (e0 != 1) return 160;
-  return sizeof(Real) == 4 ? 250 : 256;
+  return sizeof(Real) == 4 ? 250 : kRunUnion;
 }
 
 template <typename Real>
@@ -2837,7 +3041,16 @@ void DeviceKernels<Real>::hadamard_tiled(hipStream_t s, int n_tiles, int M_dim, 
       const int n_fgt = (M_dim + 1) / 2;
       const int64_t nbt = (int64_t)n_tiles * ((n_fgt + 7) / 8) * 8;
       if (nbt >= (1ll << 31)) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
-      hipLaunchKernelGGL((k_hadamard_tiled<Real, 1, 1, 2, 256, 1>), dim3((unsigned)nbt, nv), dim3(256), 0, s, M_dim, n_tiles,
+      // equal shares on one block per CU, where k_hadamard_tiled would not have all its blocks resident
+      // at once (two per CU): with fewer products (m = 4, 196 of them: 15 : 17 us) a block has one
+      // tile, and nothing to overlap it with
+      if ((int64_t)n_fgt * n_tiles > 512 && (int64_t)M_dim * 128 < (1ll << 32)) {
+        hipLaunchKernelGGL((k_hadamard_run<kRunUnion>), dim3(256, nv), dim3(512), 0, s, M_dim, n_tiles, n_fgt, tile_t0, tile_u0,
+                           usrc, uidx, gmask, offsets, Vp, X, Y, x_vs, y_vs);
+        HIP_LAUNCH_CHECK();
+        return;
+      }
+      hipLaunchKernelGGL((k_hadamard_tiled<Real, 1, 1, 2, kRunUnion, 1>), dim3((unsigned)nbt, nv), dim3(256), 0, s, M_dim, n_tiles,
                          tile_t0, tile_u0, usrc, uidx, gmask, offsets, Vp, X, Y, x_vs, y_vs);
     }
   } else if (e0 == 3 && e1 == 3) {
