@@ -842,8 +842,13 @@ template <> struct Mfma<double> {
 // time in LDS with k contiguous for both operands so each lane feeds its four k values of an
 // MFMA group from one 4-vector read.  With ksplit > 1 the block handles one k range and writes
 // its partial tile to work[z][i][n]; k_gemm_reduce then sums the partials in a fixed order.
+// FP32 adds its products in chains of 64 k (SEG), so that the rounding does not depend on how many
+// blocks the K split makes: with one chain per block, fewer blocks left Stokes (80k points, m = 8)
+// 5% and 3 Laplace potentials (50k, m = 8) 6% further from the direct sum (8.26e-7 : 7.81e-7, 2.89e-7
+// : 2.71e-7).  The second set of sums takes 78 registers, 6 waves per SIMD instead of 8: 1% of the
+// 2M adaptive and 1M Stokes evaluations, less than the additional K split would.
 template <typename Real, bool ACC, bool SPLIT, bool VEC>
-__global__ __launch_bounds__(256, (sizeof(Real) == 4 ? 8 : 4)) void k_gemm_rows(int M, int N, int K, int kchunk, const Real* __restrict__ A,
+__global__ __launch_bounds__(256, (sizeof(Real) == 4 ? 6 : 4)) void k_gemm_rows(int M, int N, int K, int kchunk, const Real* __restrict__ A,
                                                    const int32_t* __restrict__ ra, int64_t lda, const Real* __restrict__ B,
                                                    Real* __restrict__ C, const int32_t* __restrict__ rc, int64_t ldc,
                                                    const Real* __restrict__ alpha, Real* __restrict__ work, int Mv,
@@ -903,6 +908,8 @@ __global__ __launch_bounds__(256, (sizeof(Real) == 4 ? 8 : 4)) void k_gemm_rows(
   for (int i = 0; i < 2; i++)
 #pragma unroll
     for (int j = 0; j < 2; j++) acc[i][j] = V4{0, 0, 0, 0};
+  constexpr bool SEG = sizeof(Real) == 4;
+  V4 sum[2][2] = {{V4{0, 0, 0, 0}, V4{0, 0, 0, 0}}, {V4{0, 0, 0, 0}, V4{0, 0, 0, 0}}};
   if (kb0 < kb1) load(kb0);
   for (int k0 = kb0; k0 < kb1; k0 += BK) {
 #pragma unroll
@@ -935,7 +942,24 @@ __global__ __launch_bounds__(256, (sizeof(Real) == 4 ? 8 : 4)) void k_gemm_rows(
           acc[i][j] = MF::mma(av[i][3], bv[j][3], acc[i][j]);
         }
     }
+    if constexpr (SEG) {
+      if (((k0 - kb0) & BK) || k0 + BK >= kb1) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int j = 0; j < 2; j++) {
+            sum[i][j] += acc[i][j];
+            acc[i][j] = V4{0, 0, 0, 0};
+          }
+      }
+    }
     __syncthreads();
+  }
+  if constexpr (SEG) {
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) acc[i][j] = sum[i][j];
   }
   if constexpr (!SPLIT && ACC) {
     // read-modify-write: every C value of the lane is loaded before any is stored, so the
