@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void k_lattice_kernel(int m, int n, double h, 
 }
 
 // Twiddles exp(-2 pi i k / n) of the block
-constexpr int kMaxN = 128;
+constexpr int kMaxN = 1024;  // points per axis
 __device__ __forceinline__ void load_twiddles(double2* tw, int n) {
   for (int k = threadIdx.x; k < n; k += 256) {
     double s, c;
