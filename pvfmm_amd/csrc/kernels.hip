@@ -2278,19 +2278,22 @@ __global__ __launch_bounds__(512, 2) void k_hadamard_run(int M_dim, int n_tiles,
 }
 
 // FP32 frequency-domain M2L for the scalar kernels (k_hadamard_split) on the fp16 matrix
-// cores: operands are scaled by powers of two into fp16 range and split exactly into two fp16
-// parts x = x0 + x1 (x0 = RN(x), x1 = RN(x - x0): 22 significant bits, |x - x0 - x1| <=
-// 2^-22 |x|), and the three largest products are summed in FP32,
-//   x.t ~ x0 t0 + (x0 t1 + x1 t0),
-// each exact in FP32 (11 x 11 bits); the dropped x1 t1 stays below 2^-22 |x t|.  The spectra
-// of the sources a block stages are scaled by its run's power of two s (k_run_scale: s times
-// the largest bound of their spectra is below 2^14), the transfer blocks of frequency f by
-// tau_f (host: tau_f times the block's largest entry below 2^14), and the result is divided by
-// s tau_f (exact).  Spectra far below their run's largest bound lose relative precision in x1
-// (fp16 subnormals) but stay within about 2^-24 of that bound, the FP32 rounding of the run's
-// largest values.
+// cores: operands are scaled by powers of two into fp16 range and split into two fp16 parts
+// x = x0 + 2^-11 x1 (x0 = RN(x), x1 = RN(2^11 (x - x0)): 22 significant bits, |x - x0 - 2^-11 x1|
+// <= 2^-22 |x|), whose four products are exact in FP32 (11 x 11 bits) and summed by weight,
+//   x.t ~ x0 t0 + 2^-11 ((x0 t1 + x1 t0) + 2^-11 x1 t1).
+// The spectra of the sources a block stages are scaled by its run's power of two s (k_run_scale:
+// s times the largest bound of their spectra is below 2^14), the transfer blocks of frequency f
+// by tau_f (k_transfer_tau: tau_f times the blocks' largest entry below 2^14), and the result is
+// divided by s tau_f (exact).  The factor 2^11 puts x1 where x0 was, so values down to 2^-28 of
+// their run's bound keep the 22 bits and smaller ones an error of 2^-50 of that bound.  With x1
+// unscaled that error was 2^-39, and two clusters far apart whose charges differ by 2^20 in size
+// (8 vectors, gradient, m = 10) came out 1.1e-5 off at the weak one, 2.2e-7 with it; the factor
+// costs nothing.  x1 t1 (2^-24 of a product on average) is a third more products: 60,000 points,
+// m = 8: 2.62e-7 -> 2.51e-7 from the FP64 sums; 32 vectors on 1M points 46.7 -> 47.9 ms, the 2M
+// adaptive tree 10.4 -> 10.6 ms.
 // One v_mfma_f32_16x16x32_f16 covers two parent offsets (k = 16 a + real index, a the offset
-// of the pair), so an offset pair of a 16-target group costs 3 MFMAs of K = 32 instead of the 8
+// of the pair), so an offset pair of a 16-target group costs 4 MFMAs of K = 32 instead of the 8
 // FP32 MFMAs of K = 4 per offset.  A block owns one frequency and a run of consecutive tiles;
 // wave w computes target group w (targets 16w..16w+15 of a tile) over the 13 offset pairs, with
 // the transfer-block parts of its frequency held in registers for the run.  The partners'
@@ -2404,7 +2407,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
       for (int q = 0; q < 4; q++) {
         const float x = val[i][q] * xsc;  // exact (power of two)
         h0[q] = (_Float16)x;
-        h1[q] = (_Float16)(x - (float)h0[q]);
+        h1[q] = (_Float16)((x - (float)h0[q]) * kSplitLow);
       }
       uint32_t* d = &Xl[dst[i] * EST + 2 * sr];
       *reinterpret_cast<halfx4*>(d) = h0;
@@ -2453,7 +2456,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
     auto aop = [&](int pos, int p) __attribute__((always_inline)) {
       return *reinterpret_cast<const halfx8*>(&xb[pos * EST + 8 * p + lane_off]);
     };
-    floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+    floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
     halfx8 an[2];
     {
       const int p0 = pidx(0);
@@ -2481,6 +2484,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
       if ((wm >> (2 * j)) & 3u) {
         acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[1], bq[j][0], acc1, 0, 0, 0);
         acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][0], acc0, 0, 0, 0);
+        acc2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[1], bq[j][1], acc2, 0, 0, 0);
         acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][1], acc1, 0, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -2488,7 +2492,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
     store_lds(buf ^ 1, nd1);  // tile k+1 (slots that tile k does not read; the other table buffer is free since the last barrier)
     {
       const int t0 = m_t[k - k0], nt = m_t[k - k0 + 1] - t0;
-      const floatx4 sum = (acc0 + acc1) * ysc;
+      const floatx4 sum = (acc0 + (acc1 + acc2 * (1.f / kSplitLow)) * (1.f / kSplitLow)) * ysc;
       float* yr = Y + ((int64_t)(t0 + 16 * w + 4 * kg) * M_dim + f) * RW + row;
 #pragma unroll
       for (int r = 0; r < 4; r++)
@@ -2499,7 +2503,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
 }
 
 // FP32 frequency-domain M2L for Stokes (3x3 blocks, 48 reals per spectrum row) on the fp16
-// matrix cores, with the operand split of k_hadamard_split: the tile's partner spectra are
+// matrix cores, split into x0 = RN(x) and x1 = RN(x - x0): the tile's partner spectra are
 // scaled by the power of two s with s times their largest bound below 2^14 (the bounds are per
 // source slot and component) and the transfer blocks of frequency f by tau_f, each split into
 // two fp16 parts, and the three largest products are summed in FP32; the result is divided by

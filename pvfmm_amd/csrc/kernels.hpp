@@ -6,6 +6,10 @@
 
 namespace pvfmm_amd {
 
+// Scale of the second fp16 part of the FP32 scalar Hadamard's operands (k_hadamard_split): it
+// stores 2^11 (x - RN(x)), which is at most as large as the first part.
+constexpr float kSplitLow = 2048.f;
+
 // Operands of the FP32 Hadamard kernels on the fp16 matrix cores (see hadamard_tiled).
 struct HadamardParts {
   const uint16_t* Vh = nullptr;  // transfer blocks as two fp16 parts, scaled by tau_f
@@ -139,8 +143,8 @@ struct DeviceKernels {
   // run of tiles one block of the FP32 scalar kernel handles.  hp (FP32 only, else null): the
   // FP32 kernels run on the fp16 matrix cores and need it.  hp->Vh the transfer blocks as two
   // fp16 parts of tau_f B for the offsets in the order of uidx, taken in pairs (2j, 2j+1):
-  // scalar kernels [pair j][part p][f][lane 64][8], lane l holding part p of
-  // B_{2j + l/32}[8 ((l/16) % 2) + i][l % 16], i < 8; Stokes [f][pair j][chunk c][tile nb]
+  // scalar kernels [pair j][part p][f][lane 64][8], lane l holding part p (part 1 times
+  // kSplitLow) of B_{2j + l/32}[8 ((l/16) % 2) + i][l % 16], i < 8; Stokes [f][pair j][chunk c][tile nb]
   // [part p][lane 64][8], lane l holding part p of B_{2j + a}[8 b + i][16 nb + l % 16] with
   // q = 4c + l/16, a = q / 6, b = q % 6; hp->tinv 1 / tau_f; hp->bound the spectrum bounds of
   // X's slots and components (fft_up); hp->run_scale (scalar kernels) room for

@@ -10,6 +10,7 @@
 
 #include "common.hpp"
 #include "device_fmm.hpp"
+#include "kernels.hpp"
 #include "transfer.hpp"
 
 namespace pvfmm_amd {
@@ -167,7 +168,7 @@ __global__ __launch_bounds__(256) void k_transfer_tau(Blocks B, double* __restri
 
 __device__ __forceinline__ uint16_t half_bits(_Float16 h) { return __builtin_bit_cast(uint16_t, h); }
 
-// scalar kernels: [pair j][part p][f][lane][i]
+// scalar kernels: [pair j][part p][f][lane][i], part 1 times kSplitLow
 __global__ __launch_bounds__(256) void k_transfer_fp16_scalar(Blocks B, const double* __restrict__ tau, uint16_t* __restrict__ Vh) {
   const int64_t idx = blockIdx.x * (int64_t)256 + threadIdx.x;
   if (idx >= (int64_t)13 * B.M * 512) return;
@@ -175,7 +176,7 @@ __global__ __launch_bounds__(256) void k_transfer_fp16_scalar(Blocks B, const do
   const int64_t jf = idx >> 9;
   const int j = (int)(jf / B.M), f = (int)(jf % B.M);
   const double x = B.entry(offset_of(2 * j + (l >> 5)), f, 8 * ((l >> 4) & 1) + i, l & 15) * tau[f];
-  const _Float16 h0 = (_Float16)x, h1 = (_Float16)(x - (double)h0);
+  const _Float16 h0 = (_Float16)x, h1 = (_Float16)((x - (double)h0) * (double)kSplitLow);
   Vh[((((int64_t)j * 2 + 0) * B.M + f) * 64 + l) * 8 + i] = half_bits(h0);
   Vh[((((int64_t)j * 2 + 1) * B.M + f) * 64 + l) * 8 + i] = half_bits(h1);
 }

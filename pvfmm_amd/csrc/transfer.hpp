@@ -27,7 +27,8 @@ void transfer_spectra(hipStream_t s, int kind, int m, double* G);
 // forms the Hadamard kernels read (offsets R in increasing order without 13, in pairs for the
 // split forms):
 //   real:   Vp[((R * M + f) * e0 + kb) * e1 + nb][lane][q], FP64 kernels, R of 27
-//   fp16:   two parts of tau_f B, scalar and Stokes layouts of hadamard_tiled; tinv = 1 / tau_f
+//   fp16:   two parts of tau_f B, scalar (the second times kSplitLow) and Stokes layouts of
+//           hadamard_tiled; tinv = 1 / tau_f
 void transfer_real(hipStream_t s, int e0, int e1, int M, const double* G, double* Vp);
 void transfer_fp16(hipStream_t s, int e0, int e1, int M, const double* G, uint16_t* Vh, float* tinv);
 
