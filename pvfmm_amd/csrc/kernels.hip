@@ -1531,7 +1531,13 @@ struct DftShape {
 // convolution of the m-point lattices free of wrap-around (displacements -(m-1) .. m-1), so a
 // spectrum has m N^2 values, 18% (m = 10) to 28% (m = 6) fewer than on the usual 2m grid, in
 // every V-list kernel (2M adaptive, m = 10, FP32: Hadamard 3.78 -> 2.84 ms, inverse DFT 1.57 ->
-// 1.37, forward 1.10 -> 1.00; 1M FP64: 5.65 -> 4.61, 1.53 -> 1.42, 0.95 -> 0.82).
+// 1.37, forward 1.10 -> 1.00; 1M FP64: 5.65 -> 4.61, 1.53 -> 1.42, 0.95 -> 0.82).  The rounding of
+// the spectra spreads over N^3 points of which m^3 are results: on the smaller grid an FP32 result
+// holds 8 to 10% more of it (60,000 points, m = 8: 2.49e-7 -> 2.68e-7 from the FP64 sums).  The sums
+// below make up for that, for less than 1% of the time: the forward stages add even and odd terms apart in
+// FP32 (2.62e-7 -> 2.58e-7 by itself), the inverse adds from the high frequencies, which are small,
+// down to 0 (2.62e-7 -> 2.56e-7), and the Hadamard's main products go to two sums (2.68e-7 ->
+// 2.62e-7); with its fourth product 2.41e-7.
 //
 // Forward DFT of the 8 children of one source parent, component i (grid n_slots * e0).
 // x stage (real -> complex, kx < m) on thread-owned lattice lines into LDS; then one task per
@@ -1553,6 +1559,7 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_
   using S = DftShape<Real, M>;
   constexpr int N1 = S::N1, NH = S::NH, MD = S::MD, M2 = S::M2, NT = S::NT, LPT = S::LPT, CG = S::CG, KC = S::KC_UP;
   constexpr int CST = KC * M2 + 1;  // child stride (odd, spreads the children over LDS banks)
+  constexpr bool PAIRED = sizeof(Real) == 4;  // even and odd terms summed apart
   constexpr TwTable<N1> TW{};
   __shared__ Real twc[N1], tws[N1];
   __shared__ Real s1r[8 * CST], s1i[8 * CST];
@@ -1639,11 +1646,20 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_
       auto zstage = [&](const Real* gr, const Real* gi, int kyy) __attribute__((always_inline)) {
         sfor<M>([&](auto ikz) __attribute__((always_inline)) {
           constexpr int kz = decltype(ikz)::value;
-          Real cr = gr[0], ci = gi[0], sr = 0, si = 0;
+          Real cr = gr[0], ci = gi[0], sr = 0, si = 0, cr1 = 0, ci1 = 0, sr1 = 0, si1 = 0;
           sfor<M - 1>([&](auto iz1) __attribute__((always_inline)) {
             constexpr int zz = decltype(iz1)::value + 1;
-            cs_tw<N1, (kz * zz) % N1>(gr[zz], gi[zz], cr, ci, sr, si);
+            if constexpr (PAIRED && zz % 2 == 1)
+              cs_tw<N1, (kz * zz) % N1>(gr[zz], gi[zz], cr1, ci1, sr1, si1);
+            else
+              cs_tw<N1, (kz * zz) % N1>(gr[zz], gi[zz], cr, ci, sr, si);
           });
+          if constexpr (PAIRED) {
+            cr += cr1;
+            ci += ci1;
+            sr += sr1;
+            si += si1;
+          }
           store(kx + (int64_t)NH * (kyy + N1 * kz), cr + si, ci - sr);
           if constexpr (kz > 0) store(kx + (int64_t)NH * (kyy + N1 * (N1 - kz)), cr - si, ci + sr);
         });
@@ -1653,16 +1669,24 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_
         cr = pr[zz * M];
         ci = pi[zz * M];
         sr = si = 0;
+        Real cr1 = 0, ci1 = 0, sr1 = 0, si1 = 0;
 #pragma unroll
         for (int yy = 1, e = 0; yy < M; yy++) {
           e += ky;
           if (e >= N1) e -= N1;
           const Real dr = pr[zz * M + yy], di = pi[zz * M + yy];
           const Real wc = twc[e], ws = tws[e];
-          cr = fma(dr, wc, cr);
-          ci = fma(di, wc, ci);
-          sr = fma(dr, ws, sr);
-          si = fma(di, ws, si);
+          const bool odd = PAIRED && yy % 2 == 1;  // known when unrolled
+          (odd ? cr1 : cr) = fma(dr, wc, odd ? cr1 : cr);
+          (odd ? ci1 : ci) = fma(di, wc, odd ? ci1 : ci);
+          (odd ? sr1 : sr) = fma(dr, ws, odd ? sr1 : sr);
+          (odd ? si1 : si) = fma(di, ws, odd ? si1 : si);
+        }
+        if constexpr (PAIRED) {
+          cr += cr1;
+          ci += ci1;
+          sr += sr1;
+          si += si1;
         }
       };
       if constexpr (S::SPLIT_H) {
@@ -1706,7 +1730,9 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_
 // per (c, kx, ky) task straight from Y (the sums and differences over kz and N - kz) into LDS;
 // then each thread runs the y stage
 // of its own lines (c, y, z) and accumulates the c2r x sum in registers; the lattice values
-// are added into dn at the end.
+// are added into dn at the end.  In FP32 all sums go from the highest frequency to 0; in FP64, whose
+// results are as accurate as m allows either way, that order costs 8 registers at m = 6 and with them
+// a wave per SIMD (64k points: 386 -> 393 us).
 // FP64: one block per CU, so that the compiler keeps the y/z stage in registers instead of
 // spilling them to fit four (measured at m = 10: 3.78 -> 2.82 ms; the FP32 form is fastest at 4)
 template <typename Real, int M>
@@ -1738,7 +1764,11 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
     for (int x = 0; x < M; x++) acc[q][x] = 0;
   dn += blockIdx.y * dn_vs;  // density vector
   const Real* Ys = Y + blockIdx.y * y_vs + ((int64_t)slot * MD * 8 * e1 + 8 * j) * 2;
-  for (int k0 = 0; k0 < NH; k0 += KC) {
+  constexpr bool DOWN = sizeof(Real) == 4;  // sums from the highest frequency to 0
+  const int y_top = (M - 1) * y % N1;
+  constexpr int NCH = (NH + KC - 1) / KC;
+  for (int ch = 0; ch < NCH; ch++) {
+    const int k0 = (DOWN ? NCH - 1 - ch : ch) * KC;
     const int kn = (NH - k0 < KC) ? NH - k0 : KC;
     const int ntask = 8 * N1 * kn;
     for (int T = t; T < ntask; T += NT) {  // z stage
@@ -1762,9 +1792,9 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
       Real* di = &s1i[c * CST + kl * PL + ky * M];
       sfor<M>([&](auto izz) __attribute__((always_inline)) {
         constexpr int zz = decltype(izz)::value;
-        Real sr = pr_[0], si = pi_[0];
+        Real sr = DOWN ? Real(0) : pr_[0], si = DOWN ? Real(0) : pi_[0];
         sfor<M - 1>([&](auto ia) __attribute__((always_inline)) {
-          constexpr int a = decltype(ia)::value + 1;
+          constexpr int a = DOWN ? M - 1 - decltype(ia)::value : decltype(ia)::value + 1;
           constexpr double wc = ct_cs((a * zz) % N1, N1, false), ws = ct_cs((a * zz) % N1, N1, true);
           sr = fma(pr_[a], (Real)wc, sr);
           si = fma(pi_[a], (Real)wc, si);
@@ -1773,13 +1803,13 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
             si = fma(qr_[a], (Real)ws, si);
           }
         });
-        dr[zz] = sr;
-        di[zz] = si;
+        dr[zz] = DOWN ? sr + pr_[0] : sr;
+        di[zz] = DOWN ? si + pi_[0] : si;
       });
     }
     __syncthreads();
-    for (int kl = 0; kl < kn; kl++) {  // y stage and c2r x sum of the owned lines
-      const int kx = k0 + kl;
+    for (int kk = 0; kk < kn; kk++) {  // y stage and c2r x sum of the owned lines
+      const int kl = DOWN ? kn - 1 - kk : kk, kx = k0 + kl;
       const Real wk = kx == 0 ? Real(1) : Real(2);
       Real sr[LPT], si[LPT];
 #pragma unroll
@@ -1787,18 +1817,24 @@ __global__ __launch_bounds__((DftShape<Real, M>::NT), (sizeof(Real) == 8 ? 1 : 4
         const int c = cg + CG * q;
         const Real* pr = &s1r[c * CST + kl * PL + z];
         const Real* pi = &s1i[c * CST + kl * PL + z];
-        Real ar = pr[0], ai = pi[0];
+        Real ar = DOWN ? Real(0) : pr[0], ai = DOWN ? Real(0) : pi[0];
 #pragma unroll
-        for (int a = 1, e = 0; a < M; a++) {
-          e += y;
-          if (e >= N1) e -= N1;
+        for (int b = 1, e = DOWN ? y_top : y; b < M; b++) {
+          const int a = DOWN ? M - b : b;
           const Real wc = twc[e], ws = tws[e];
           const Real ur = pr[a * M], ui = pi[a * M], vr = pr[(N1 - a) * M], vi = pi[(N1 - a) * M];
           ar += (ur + vr) * wc - (ui - vi) * ws;
           ai += (ui + vi) * wc + (ur - vr) * ws;
+          if constexpr (DOWN) {
+            e -= y;
+            if (e < 0) e += N1;
+          } else {
+            e += y;
+            if (e >= N1) e -= N1;
+          }
         }
-        sr[q] = wk * ar;
-        si[q] = wk * ai;
+        sr[q] = wk * (DOWN ? ar + pr[0] : ar);
+        si[q] = wk * (DOWN ? ai + pi[0] : ai);
       }
 #pragma unroll
       for (int x = 0, e = 0; x < M; x++) {
@@ -2456,7 +2492,8 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
     auto aop = [&](int pos, int p) __attribute__((always_inline)) {
       return *reinterpret_cast<const halfx8*>(&xb[pos * EST + 8 * p + lane_off]);
     };
-    floatx4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
+    floatx4 acc0[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // even and odd pairs
+    floatx4 acc1 = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
     halfx8 an[2];
     {
       const int p0 = pidx(0);
@@ -2483,7 +2520,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
       __builtin_amdgcn_sched_barrier(0);
       if ((wm >> (2 * j)) & 3u) {
         acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[1], bq[j][0], acc1, 0, 0, 0);
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][0], acc0, 0, 0, 0);
+        acc0[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][0], acc0[j & 1], 0, 0, 0);
         acc2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[1], bq[j][1], acc2, 0, 0, 0);
         acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][1], acc1, 0, 0, 0);
       }
@@ -2492,7 +2529,7 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
     store_lds(buf ^ 1, nd1);  // tile k+1 (slots that tile k does not read; the other table buffer is free since the last barrier)
     {
       const int t0 = m_t[k - k0], nt = m_t[k - k0 + 1] - t0;
-      const floatx4 sum = (acc0 + (acc1 + acc2 * (1.f / kSplitLow)) * (1.f / kSplitLow)) * ysc;
+      const floatx4 sum = ((acc0[0] + acc0[1]) + (acc1 + acc2 * (1.f / kSplitLow)) * (1.f / kSplitLow)) * ysc;
       float* yr = Y + ((int64_t)(t0 + 16 * w + 4 * kg) * M_dim + f) * RW + row;
 #pragma unroll
       for (int r = 0; r < 4; r++)
