@@ -207,6 +207,8 @@ void* pvfmm_amd_batch_stream(void* batch);
 /* number of times the graph was recorded or replayed on buffers other than the last call's
  * (1 while the pointers stay the same) */
 int pvfmm_amd_batch_records(void* batch);
+/* number of times the graph was recorded (1 on whatever buffers, while the trees stay as they are) */
+int pvfmm_amd_batch_recordings(void* batch);
 void pvfmm_amd_batch_destroy(void* batch);
 
 /* Introspection for parity checks. */

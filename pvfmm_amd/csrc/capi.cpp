@@ -150,7 +150,8 @@ struct BatchHandle {
   // ordering of a replay against eager work on the trees' own streams (outside the graph)
   std::vector<hipEvent_t> before;
   hipEvent_t after = nullptr;
-  int records = 0;
+  int records = 0;     // recordings, and replays on buffers other than the last call's
+  int recordings = 0;  // recordings alone
   std::vector<std::pair<int, int>> tunings() const {
     std::vector<std::pair<int, int>> v;
     for (TreeHandle* t : trees)
@@ -203,6 +204,7 @@ struct BatchHandle {
     HIP_CHECK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
     tune_key = tunings();
     plan_key = plans();
+    recordings++;
   }
 };
 
@@ -239,7 +241,6 @@ void batch_eval(BatchHandle* b, const double* const* d_den, double* const* d_out
     b->slots.ensure(2 * n * sizeof(void*));
     b->record();
   }
-  // counts the recordings and the calls that bind other buffers
   if (!recorded || !std::equal(b->den_key.begin(), b->den_key.end(), d_den) ||
       !std::equal(b->out_key.begin(), b->out_key.end(), d_out)) {
     b->den_key.assign(d_den, d_den + n);
@@ -605,6 +606,7 @@ int pvfmm_amd_batch_evaluate_device(void* batch, const double* const* d_den, dou
 }
 void* pvfmm_amd_batch_stream(void* batch) { return batch ? (void*)((BatchHandle*)batch)->stream : nullptr; }
 int pvfmm_amd_batch_records(void* batch) { return batch ? ((BatchHandle*)batch)->records : -1; }
+int pvfmm_amd_batch_recordings(void* batch) { return batch ? ((BatchHandle*)batch)->recordings : -1; }
 void pvfmm_amd_batch_destroy(void* batch) { delete (BatchHandle*)batch; }
 
 int64_t pvfmm_amd_tree_num_nodes(void* tree) { return tree ? ((TreeHandle*)tree)->T.n_nodes() : -1; }

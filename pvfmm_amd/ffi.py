@@ -79,6 +79,7 @@ def _declare(L):
         "pvfmm_amd_batch_evaluate_device": (i, [vp, ctypes.POINTER(vp), ctypes.POINTER(vp), i]),
         "pvfmm_amd_batch_stream": (vp, [vp]),
         "pvfmm_amd_batch_records": (i, [vp]),
+        "pvfmm_amd_batch_recordings": (i, [vp]),
         "pvfmm_amd_batch_destroy": (None, [vp]),
         "pvfmm_amd_tree_num_nodes": (i64, [vp]),
         "pvfmm_amd_tree_nodes": (i, [vp, c_int64_p]),

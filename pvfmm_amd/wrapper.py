@@ -430,7 +430,12 @@ class PtFMMBatch:
         return ffi.lib().pvfmm_amd_batch_stream(self._h) or 0
 
     def records(self) -> int:
+        """Recordings of the graph, and replays on tensors other than the last call's."""
         return ffi.lib().pvfmm_amd_batch_records(self._h)
+
+    def recordings(self) -> int:
+        """Recordings of the graph alone: 1 on whatever tensors, while the trees stay as they are."""
+        return ffi.lib().pvfmm_amd_batch_recordings(self._h)
 
 
 def device_count() -> int:
