@@ -154,8 +154,7 @@ struct BatchHandle {
   int recordings = 0;  // recordings alone
   std::vector<std::pair<int, int>> tunings() const {
     std::vector<std::pair<int, int>> v;
-    for (TreeHandle* t : trees)
-      v.emplace_back(t->plan->tuning.hadamard_tpb, t->plan->tuning.gemm_split_blocks * 64 + t->plan->tuning.hadamard_vec_tpw);
+    for (TreeHandle* t : trees) v.emplace_back(t->plan->tuning.hadamard_tpb, t->plan->tuning.gemm_split_blocks);
     return v;
   }
   std::vector<uint64_t> plans() const {

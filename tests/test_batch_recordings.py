@@ -43,3 +43,22 @@ def test_other_buffers_replay_the_recorded_graph(gpu):
     trees[1].setup(P.PtFMM("laplace_poten", 8, "mixed"))
     batch.evaluate_device(sets[1])
     assert batch.recordings() == 2
+
+
+def test_changed_launch_shapes_record_the_graph_again(gpu):
+    """Every change of a shape that the launches use, whatever the value without effect beside it: a
+    key that adds the two up takes (1024, 16) and (1023, 80) for the same shapes."""
+    trees, batch, den = _batch([3000, 5000], 8)
+    batch.evaluate_device(den)
+    trees[0].set_tuning(hadamard_tiles_per_block=16, gemm_split_blocks=1024, hadamard_vec_targets_per_wave=16)
+    batch.evaluate_device(den)
+    assert batch.recordings() == 1
+    trees[0].set_tuning(hadamard_tiles_per_block=16, gemm_split_blocks=1023, hadamard_vec_targets_per_wave=80)
+    batch.evaluate_device(den)
+    assert batch.recordings() == 2
+    trees[0].set_tuning(hadamard_tiles_per_block=16, gemm_split_blocks=1023, hadamard_vec_targets_per_wave=3)
+    batch.evaluate_device(den)
+    assert batch.recordings() == 2
+    trees[1].set_tuning(hadamard_tiles_per_block=8, gemm_split_blocks=1024)
+    batch.evaluate_device(den)
+    assert batch.recordings() == 3
