@@ -155,6 +155,8 @@ class DevicePlan final : public DevicePlanBase {
     evaluate_one(nullptr, nullptr, 1.0, 1.0, 1, den_slot, out_slot);
   }
 
+  int64_t device_bytes() const override { return device_bytes_ + ops_->bytes(); }
+
   Tuning autotune(const double* d_den, double* d_out, int n_vec) override {
     if (n_vec < 1 || n_vec > nvb_) throw Error(kErrInvalidArgument, "autotune takes 1 to n_vec_max density vectors");
     const bool was = timing_;
@@ -430,7 +432,7 @@ class DevicePlan final : public DevicePlanBase {
   }
 
   void build(const Octree& T, const double* src_xyz, const double* trg_xyz) {
-    int64_t total = ops_->bytes();
+    int64_t total = 0;
     const KernelInfo& ki = O_.ker;
     k0_ = ki.k0; k1_ = ki.k1; e0_ = ki.e0; e1_ = ki.e1;
     ns_ = O_.ns; m_ = O_.m; K0_ = O_.K0(); K1_ = O_.K1(); M_dim_ = ops_->grid.M;
@@ -770,7 +772,6 @@ class DevicePlan final : public DevicePlanBase {
     stats.u_rows = n_tleaf_; stats.u_items = (int64_t)u_items.size(); stats.u_pairs = u_pairs;
     stats.u_src_points_streamed = u_stream;
     stats.far_items = (int64_t)far_node.size(); stats.far_pairs = far_pairs; stats.s2m_pairs = s2m_pairs;
-    stats.device_bytes = total;
     device_bytes_ = total;
   }
 
@@ -834,7 +835,7 @@ class DevicePlan final : public DevicePlanBase {
     std::vector<int32_t> sb, se, tb, te;
     std::vector<std::pair<int32_t, int>> imgs;
   } h_;
-  int64_t device_bytes_ = 0;
+  int64_t device_bytes_ = 0;  // of the plan itself
 
   struct AdjointPlan {
     const typename DeviceOps<Real>::Transposed* op = nullptr;  // the transposed operators
@@ -1026,7 +1027,6 @@ class DevicePlan final : public DevicePlanBase {
       if (vol_) a->volpart.alloc((int64_t)K::vol_adjoint_blocks() * 3 * nvb_, &total);
     }
     device_bytes_ += total;
-    stats.device_bytes = device_bytes_;
     adj_ = std::move(a);
   }
 

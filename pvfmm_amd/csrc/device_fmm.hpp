@@ -34,7 +34,6 @@ struct PlanStats {
   int64_t v_src_slots = 0, v_trg_slots = 0, v_pairs = 0;
   int64_t u_rows = 0, u_items = 0, u_pairs = 0, far_items = 0, far_pairs = 0, s2m_pairs = 0;
   int64_t u_src_points_streamed = 0;
-  int64_t device_bytes = 0;
   int64_t v_tiles = 0, v_tile_partners = 0, v_tile_max_partners = 0;
   int64_t v_tile_staged = 0;  // partner spectra staged per pass (the FP32 scalar kernel stages deltas)
 };
@@ -65,6 +64,8 @@ class DevicePlanBase {
   // One vector, with the addresses of d_den and d_out read from device memory when the launches
   // run: the form a recorded graph replays on any buffers.
   virtual void evaluate_slots(const double* const* den_slot, double* const* out_slot) = 0;
+  // Device memory of the plan, and of the operators it shares with the other plans of its handle
+  virtual int64_t device_bytes() const = 0;
   // The transpose of evaluate's linear map (same scales): d_g in the user layout of the
   // targets (k1 per target), d_out in that of the sources (k0 per source), overwritten.  Built
   // on first use; symmetric kernels only (adjoint_supported()).

@@ -4,6 +4,7 @@
 // own lists only.
 #pragma once
 #include <algorithm>
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include <type_traits>
@@ -70,7 +71,7 @@ class DeviceOps final : public DeviceOpsBase {
   bool split = false;    // FP32: the fp16 Hadamard kernels
 
   explicit DeviceOps(const Operators& O) : O_(O) {
-    int64_t* total = &bytes_;
+    int64_t sum = 0, *total = &sum;
     const int K0 = O.K0(), K1 = O.K1(), e0 = O.ker.e0, e1 = O.ker.e1;
     Stream st;
     const hipStream_t s = st.s;
@@ -124,8 +125,8 @@ class DeviceOps final : public DeviceOpsBase {
     }
     HIP_CHECK(hipStreamSynchronize(s));
     DeviceKernels<Real>::gemm_pair_init();
-    pack_pair(s, uc2ue0, K1, ru, uc2ue1, K0, s2u_pair);
-    pack_pair(s, dc2de0, K1, rd, dc2de1, K0, d2t_pair);
+    pack_pair(s, uc2ue0, K1, ru, uc2ue1, K0, s2u_pair, total);
+    pack_pair(s, dc2de0, K1, rd, dc2de1, K0, d2t_pair, total);
     HIP_CHECK(hipStreamSynchronize(s));
     unit_surf.upload(std::vector<Real>(O.unit_surf.begin(), O.unit_surf.end()), total);
     lattice.upload(O.lattice, total);
@@ -146,9 +147,10 @@ class DeviceOps final : public DeviceOpsBase {
       transfer_real(s, e0, e1, grid.M, G.p, V.p);
     }
     HIP_CHECK(hipStreamSynchronize(s));
+    bytes_ = sum;
   }
 
-  int64_t bytes() const override { return bytes_; }
+  int64_t bytes() const override { return bytes_; }  // grows with the first bc() and transposed()
 
   // Boundary operator of a periodic boundary type (K0 x K1), and transposed
   const Real* bc(int bndry, bool transposed) {
@@ -171,10 +173,11 @@ class DeviceOps final : public DeviceOpsBase {
     if (!tr_) {
       auto t = std::make_unique<Transposed>();
       const int K0 = O_.K0(), K1 = O_.K1();
+      int64_t sum = 0;
       Stream st;
       auto turn = [&](const DBuf<Real>& in, int rows, int cols, DBuf<Real>& out) {
         if (!in.p) return;
-        out.alloc((int64_t)rows * cols, &bytes_);
+        out.alloc((int64_t)rows * cols, &sum);
         transpose_matrix<Real>(st.s, in.p, rows, cols, out.p);
       };
       turn(uc2ue0, K1, ru, t->uc2ue0);
@@ -185,9 +188,10 @@ class DeviceOps final : public DeviceOpsBase {
       turn(d2d, K1, 8 * K1, t->d2d);
       turn(u2ur, 8 * K0, ru, t->u2ur);
       turn(d2dr, rd, 8 * K1, t->d2dr);
-      pack_pair(st.s, t->dc2de1, K0, rd, t->dc2de0, K1, t->d2t_pair);
-      pack_pair(st.s, t->uc2ue1, K0, ru, t->uc2ue0, K1, t->s2u_pair);
+      pack_pair(st.s, t->dc2de1, K0, rd, t->dc2de0, K1, t->d2t_pair, &sum);
+      pack_pair(st.s, t->uc2ue1, K0, ru, t->uc2ue0, K1, t->s2u_pair, &sum);
       HIP_CHECK(hipStreamSynchronize(st.s));
+      bytes_ += sum;
       tr_ = std::move(t);
     }
     return *tr_;
@@ -199,12 +203,12 @@ class DeviceOps final : public DeviceOpsBase {
     Stream() { HIP_CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking)); }
     ~Stream() { (void)hipStreamDestroy(s); }
   };
-  void pack_pair(hipStream_t s, const DBuf<Real>& f0, int K, int r, const DBuf<Real>& f1, int N, PackedPair& p) {
+  void pack_pair(hipStream_t s, const DBuf<Real>& f0, int K, int r, const DBuf<Real>& f1, int N, PackedPair& p, int64_t* total) {
     using D = DeviceKernels<Real>;
     p.use = D::gemm_pair_fits(K, r) && D::gemm_pair_pays(K, 4 * (int64_t)K);
     if (!p.use) return;
-    p.B1.alloc(D::packed_size(K, r), &bytes_);
-    p.B2.alloc(D::packed_size(r, N), &bytes_);
+    p.B1.alloc(D::packed_size(K, r), total);
+    p.B2.alloc(D::packed_size(r, N), total);
     D::pack_matrix(s, f0.p, K, r, p.B1.p);
     D::pack_matrix(s, f1.p, r, N, p.B2.p);
   }
@@ -216,13 +220,15 @@ class DeviceOps final : public DeviceOpsBase {
     Stream st;
     DBuf<double> in;
     in.upload(h, nullptr);
-    out.alloc((int64_t)rows * cols, &bytes_);
+    int64_t sum = 0;
+    out.alloc((int64_t)rows * cols, &sum);
     convert_matrix<Real>(st.s, in.p, rows, cols, out.p, transposed ? cols : rows, transposed ? rows : cols, transposed);
     HIP_CHECK(hipStreamSynchronize(st.s));
+    bytes_ += sum;
   }
 
   const Operators& O_;
-  int64_t bytes_ = 0;
+  std::atomic<int64_t> bytes_{0};  // read by plans that other threads set up
   std::mutex mutex_;
   DBuf<Real> bc_[2][4];
   std::unique_ptr<Transposed> tr_;
