@@ -775,20 +775,36 @@ class DevicePlan final : public DevicePlanBase {
     device_bytes_ = total;
   }
 
-  // Splits the far rows of more than kFarRowPairs pairs into segments of about kFarSegPairs.  A
-  // block of 256 threads does the mean row's 5,000-20,000 pairs in 10-30 us; a row of 16 such
-  // units would outlast the rest of most launches.  Segments go first.
-  static constexpr int64_t kFarRowPairs = 131072, kFarSegPairs = 32768;
+  // Splits the far rows of more than kFarRowPairs pairs into segments of about kFarSegPairs, or of
+  // one item where that is more (with m = 10 from 67 targets on).  A block of 256 threads does
+  // 5,000-20,000 pairs, the mean row of ordinary trees, in 10-30 us; a row of 16 such units would
+  // outlast the rest of most launches.  Trees of few large leaves need it most: with rows split
+  // above 4 times their mean only, 200,000 points in leaves of up to 3000 (m = 10) took 2.45 ms
+  // instead of 0.40.  But there nearly every row with W items is split, and a sum per segment and
+  // target was up to 17 times the outputs: where the sums would be more than kFarSums times the
+  // outputs (and 2^20 values per vector), the segments are longer.  Segments go first.
+  static constexpr int64_t kFarRowPairs = 131072, kFarSegPairs = 32768, kFarSums = 4;
   void split_far_rows(const Octree& T, const std::vector<int32_t>& tleaf, const std::vector<int32_t>& far_ptr, int64_t* total) {
     std::vector<int32_t> row, begin, end, rows, ptr{0};
     std::vector<int64_t> part;
     std::vector<char> heavy(tleaf.size(), 0);
-    int64_t sums = 0;
+    int64_t sums = 0, seg_pairs = kFarSegPairs;
+    auto per_seg = [&](size_t r) {  // items of a segment of row r, 0: the row stays whole
+      const int64_t item = (int64_t)T.pt_cnt1(tleaf[r]) * ns_, n = far_ptr[r + 1] - far_ptr[r];
+      const int64_t per = std::max<int64_t>(1, seg_pairs / item);
+      return n * item <= kFarRowPairs || per >= n ? 0 : (int)per;
+    };
+    for (;; seg_pairs *= 2) {
+      int64_t room = std::max<int64_t>(kFarSums * n_trg_ * k1_, 1 << 20);
+      for (size_t r = 0; r < tleaf.size() && room >= 0; r++)
+        if (const int per = per_seg(r))
+          room -= (far_ptr[r + 1] - far_ptr[r] + per - 1) / per * (int64_t)T.pt_cnt1(tleaf[r]) * k1_;
+      if (room >= 0) break;
+    }
     for (size_t r = 0; r < tleaf.size(); r++) {
       const int64_t nt = T.pt_cnt1(tleaf[r]);
-      const int n = far_ptr[r + 1] - far_ptr[r];
-      if (n < 2 || n * nt * ns_ <= kFarRowPairs) continue;
-      const int per = (int)std::max<int64_t>(1, kFarSegPairs / (nt * ns_));
+      const int per = per_seg(r);
+      if (per == 0) continue;
       for (int i = far_ptr[r]; i < far_ptr[r + 1]; i += per) {
         row.push_back((int32_t)r);
         begin.push_back(i);
