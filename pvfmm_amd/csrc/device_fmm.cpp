@@ -225,6 +225,7 @@ class DevicePlan final : public DevicePlanBase {
   // lvl_seq_ = 0, 1, ... (rows of ctmp_)
   static constexpr int kFactorRows = 256;
   static constexpr int kVListSlots = 4096;
+  static constexpr int64_t kVListBytes = int64_t(1) << 31;
   DBuf<int32_t> lvl_seq_;
   // the fp16 Hadamard kernels (FP32): the spectrum bound of each slot of X (or, in the adjoint,
   // of Y) and the scale of each run of tiles
@@ -672,9 +673,13 @@ class DevicePlan final : public DevicePlanBase {
     h_.v_partner = v_partner; h_.v_src_fc = v_src_fc; h_.v_trg_fc = v_trg_fc; h_.offs = offs;
     build_tiles(v_partner, n_vtrg_, n_vsrc_, vt_, &total);
     // A V-list pass takes as many vectors as make about kVListSlots source or target parents (a
-    // parent is one block of a transform), so that a small tree's pass fills the chip; a large
-    // tree's takes one, whose spectra alone may be gigabytes.
+    // parent is one block of a transform), so that a small tree's pass fills the chip, and whose
+    // spectra fit kVListBytes, which many trees may keep side by side; a large tree's takes one,
+    // whose spectra alone may be gigabytes.
+    x_vs_ = (int64_t)n_vsrc_ * M_dim_ * 16 * e0_;
+    y_vs_ = (int64_t)n_vtrg_ * M_dim_ * 16 * e1_;
     vlist_nv_ = std::max(1, std::min(nvb_, kVListSlots / std::max(1, std::max(n_vsrc_, n_vtrg_))));
+    vlist_nv_ = (int)std::max<int64_t>(1, std::min<int64_t>(vlist_nv_, kVListBytes / (int64_t)sizeof(Real) / std::max<int64_t>(1, x_vs_ + y_vs_)));
     if (split_) {
       // per slot and component; the adjoint's sources are the target slots
       bound_vs_ = std::max(1, std::max(n_vsrc_ * e0_, n_vtrg_ * e1_));
@@ -685,8 +690,6 @@ class DevicePlan final : public DevicePlanBase {
     stats.v_tile_partners = vt_.partners;
     stats.v_tile_max_partners = vt_.max_partners;
     stats.v_tile_staged = vt_.staged_delta;
-    x_vs_ = (int64_t)n_vsrc_ * M_dim_ * 16 * e0_;
-    y_vs_ = (int64_t)n_vtrg_ * M_dim_ * 16 * e1_;
     X_.alloc(x_vs_ * vlist_nv_, &total);
     Y_.alloc(y_vs_ * vlist_nv_, &total);
 
