@@ -30,7 +30,7 @@ sys.path.insert(0, ROOT)
 
 MI355X_FP32_MFMA_TFLOPS = 157.3
 MI355X_F16_MFMA_TFLOPS = 2500.0  # dense fp16 (and bf16)
-F16_PRODUCTS_PER_FP32 = 3  # two-way fp16 split of both operands, three partial products kept
+F16_PRODUCTS_PER_FP32 = 4  # two-way fp16 split of both operands
 MI355X_FP32_VALU_TFLOPS = 78.6  # non-packed FP32 FMA (packed FP32 is not used)
 MI355X_FP64_TFLOPS = 78.6
 MI355X_HBM_GBS = 8000.0
@@ -128,8 +128,8 @@ def roofline(ph: dict, st: dict, m: int, real_bytes: int):
 
     V-list Hadamard (scalar kernels): 512*k0*k1 flop per (V1 pair, frequency) (the reference's
     own count, include/fmm_pts.txx:3336) in FP32, which the kernel computes on the fp16 matrix
-    cores as three fp16 products per FP32 product (both operands scaled and split exactly into
-    two fp16 parts).  At the dense fp16 peak those products take less time than the kernel's
+    cores as four fp16 products per FP32 product (both operands scaled and split into two fp16
+    parts).  At the dense fp16 peak those products take less time than the kernel's
     compulsory HBM traffic, every source spectrum read once and every target spectrum written
     once (16*M_dim*k0 reals per source parent, 16*M_dim*k1 per target parent, the 26 V1
     matrices once), so with t_bound = max(bytes / HBM peak, flops / MFMA peak) the bound is

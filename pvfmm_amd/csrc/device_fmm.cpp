@@ -31,7 +31,7 @@ const char* phase_name(int p) {
 
 namespace {
 
-// LDS pool slots of the V-list tiles' staged partners for the bf16 kernel (FP32 scalar
+// LDS pool slots of the V-list tiles' staged partners for the fp16 kernel (FP32 scalar
 // kernels), which keeps one pool of `pool` staged entries across the run of tiles a block
 // handles: a partner of tile k that tile k-1 also lists keeps its slot, and only the others
 // (the delta) are read and staged, into slots that no partner of tile k-1 holds, while tile
@@ -231,10 +231,11 @@ class DevicePlan final : public DevicePlanBase {
   // of Y) and the scale of each run of tiles
   DBuf<float> vbound_, vrscale_;
   bool split_ = false;
-  DBuf<Real> gemm_work_;  // split-K partial tiles of the small coarse-level GEMMs
+  // split-K partial tiles of the small coarse-level GEMMs: room for 4 of the largest output, at most 2^25
+  DBuf<Real> gemm_work_;
   int64_t gemm_work_elems_ = 0;
   int nvb_ = 1;  // density vectors per evaluation pass (buffers hold this many)
-  int64_t eq_vs_ = 0, dn_vs_ = 0, chk_vs_ = 0, ctmp_vs_ = 0;  // per-vector strides  // room for 4 K-split partials of the largest GEMM output, at most 2^25
+  int64_t eq_vs_ = 0, dn_vs_ = 0, chk_vs_ = 0, ctmp_vs_ = 0;  // per-vector strides
   int ru_ = 0, rd_ = 0;
   // The coarsest level whose upward equivalent densities anything reads (V or W list, boundary
   // operator), and whose downward check potentials anything writes: U2U and D2D stop there (in

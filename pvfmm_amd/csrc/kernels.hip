@@ -1523,7 +1523,7 @@ struct DftShape {
   // (m = 10: 138 registers at 4, none at 2; 1.22, 0.95 and 0.82 ms at 4, 3 and 2 on the 1M
   // adaptive tree), the others fit
   static constexpr int WAVES_UP = sizeof(Real) == 8 && M >= 10 ? 2 : 4;
-  // FP64 recomputes the y stage per half (ky, ky+m) instead of holding both in registers
+  // FP64 recomputes the y stage for each of the rows ky and N - ky instead of holding both in registers
   static constexpr bool SPLIT_H = sizeof(Real) == 8;
 };
 
@@ -1547,8 +1547,8 @@ struct DftShape {
 // f = kx + m(ky + N kz).
 // NTS: non-temporal stores of X, which is read back only by the Hadamard, long after its lines
 // would have left the caches (1.20 -> 1.04 ms for the 2M adaptive workload).  Only where each
-// block writes whole lines: with several components (or vectors in one group) the blocks of one
-// parent interleave their stores within a line, which must merge in L2 first.
+// block writes whole lines: with several components the blocks of one parent interleave their
+// stores within a line, which must merge in L2 first.
 template <typename Real, int M, bool NTS>
 __global__ __launch_bounds__((DftShape<Real, M>::NT), (DftShape<Real, M>::WAVES_UP)) void k_fft_up_m(const int32_t* __restrict__ first_child,
                                                                          const Real* __restrict__ up, int K0, int e0,
@@ -3063,7 +3063,7 @@ void DeviceKernels<Real>::fft_up(hipStream_t s, int n_slots, const int32_t* firs
 
 template <typename Real>
 int DeviceKernels<Real>::hadamard_union_max(int e0) {
-  // scalar kernels: FP32 250, FP64 256 partners per tile; Stokes: 160, which fits three FP32
+  // scalar kernels: FP32 250, FP64 240 partners per tile; Stokes: 160, which fits three FP32
   // blocks (one frequency each, fp16 parts) or one FP64 block (2 frequencies) in a CU's 160 KiB
   // of LDS (fuller tiles pay for the per-tile transfer-block loads over more targets)
   if (e0 != 1) return 160;

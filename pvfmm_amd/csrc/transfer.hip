@@ -75,7 +75,9 @@ __global__ __launch_bounds__(256) void k_lattice_kernel(int m, int n, double h, 
 }
 
 // Twiddles exp(-2 pi i k / n) of the block
-constexpr int kMaxN = 1024;  // points per axis
+// points per axis: every m whose spectra fit the card, more than the transforms of an evaluation take
+// (k_fft_up holds m^3 values in LDS)
+constexpr int kMaxN = 1024;
 __device__ __forceinline__ void load_twiddles(double2* tw, int n) {
   for (int k = threadIdx.x; k < n; k += 256) {
     double s, c;
