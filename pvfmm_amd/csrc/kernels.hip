@@ -1530,12 +1530,12 @@ struct DftShape {
 // The grid of the V-list transforms is N = 2m - 1 points per axis, the least that keeps the
 // convolution of the m-point lattices free of wrap-around (displacements -(m-1) .. m-1), so a
 // spectrum has m N^2 values, 18% (m = 10) to 28% (m = 6) fewer than on the usual 2m grid, in
-// every V-list kernel (2M adaptive, m = 10, FP32: Hadamard 3.78 -> 2.84 ms, inverse DFT 1.57 ->
-// 1.37, forward 1.10 -> 1.00; 1M FP64: 5.65 -> 4.61, 1.53 -> 1.42, 0.95 -> 0.82).  The rounding of
+// every V-list kernel (2M adaptive, m = 10, FP32: Hadamard 3.78 -> 2.84 ms with three products, 3.17
+// with four, inverse DFT 1.57 -> 1.41, forward 1.10 -> 1.02; 1M FP64: 5.65 -> 4.61, 1.53 -> 1.42, 0.95 -> 0.82).  The rounding of
 // the spectra spreads over N^3 points of which m^3 are results: on the smaller grid an FP32 result
 // holds 8 to 10% more of it (60,000 points, m = 8: 2.49e-7 -> 2.68e-7 from the FP64 sums).  The sums
 // below make up for that, for less than 1% of the time: the forward stages add even and odd terms apart in
-// FP32 (2.62e-7 -> 2.58e-7 by itself), the inverse adds from the high frequencies, which are small,
+// FP32 (2.68e-7 -> 2.66e-7 by itself), the inverse adds from the high frequencies, which are small,
 // down to 0 (2.62e-7 -> 2.56e-7), and the Hadamard's main products go to two sums (2.68e-7 ->
 // 2.62e-7); with its fourth product 2.41e-7.
 //
