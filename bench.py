@@ -143,7 +143,7 @@ def roofline(ph: dict, st: dict, m: int, real_bytes: int):
     dom = max(ph, key=ph.get)
     t = ph[dom] * 1e-3
     if dom == "V-List:Hadamard":
-        name = "k_hadamard_split<250, 496>"
+        name = "k_hadamard_split<250, 496, false>"
         bytes_model = (16.0 * M_dim * real_bytes * st["v_pairs"] + 16.0 * M_dim * real_bytes * st["v_trg_slots"]
                        + 26.0 * M_dim * 128 * real_bytes)
         bytes_alg = (16.0 * M_dim * real_bytes * (st["v_src_slots"] + st["v_trg_slots"]) + 26.0 * M_dim * 128 * real_bytes)

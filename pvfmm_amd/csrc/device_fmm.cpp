@@ -685,7 +685,7 @@ class DevicePlan final : public DevicePlanBase {
       // per slot and component; the adjoint's sources are the target slots
       bound_vs_ = std::max(1, std::max(n_vsrc_ * e0_, n_vtrg_ * e1_));
       vbound_.alloc(bound_vs_ * vlist_nv_, &total);
-      vrscale_.alloc((int64_t)std::max(1, vt_.n) * vlist_nv_, &total);
+      vrscale_.alloc((int64_t)2 * std::max(1, vt_.n) * vlist_nv_, &total);
     }
     stats.v_tiles = vt_.n;
     stats.v_tile_partners = vt_.partners;
@@ -1033,7 +1033,7 @@ class DevicePlan final : public DevicePlanBase {
       for (int t = 0; t < n_vtrg_; t++) fscal[t] = (Real)std::pow(2.0, ki.src_scal * (h_.vtrg_depth[t] + 1));
       a->n_vt = (int)fc.size();
       build_tiles(partner, a->n_vt, n_vtrg_, a->vt, &total);
-      if (split_) a->vrscale.alloc((int64_t)std::max(1, a->vt.n) * vlist_nv_, &total);
+      if (split_) a->vrscale.alloc((int64_t)2 * std::max(1, a->vt.n) * vlist_nv_, &total);
       a->v_fc.upload(fc, &total);
       a->fft_scal.upload(fscal, &total);
       a->ifft_scal.upload(iscal, &total);

@@ -1468,36 +1468,51 @@ __global__ __launch_bounds__(256) void k_spectrum_bound(int n_slots, const int32
   }
 }
 
-// Scale of each run of tpb consecutive V-list tiles for the fp16 Hadamard: the power of two s
-// with s * b < 2^14 <= 2 s * b, b the largest spectrum bound of the sources the run stages (its
-// first tile's partners and every later tile's new ones, as (slot << 9 | pool slot)); 1 when b
-// is 0 (or not finite).
+// Scale and passes of each run of tpb consecutive V-list tiles for the fp16 Hadamard, from the spectrum
+// bounds of the sources the run stages (its first tile's partners and every later tile's new ones, as
+// (slot << 9 | pool slot)): run_scale[r] the power of two s with s * b < 2^14 <= 2 s * b, b the largest
+// (1 when b is 0 or not finite), and, after the scales of all vectors, the number of passes, one more for
+// every kPassBits by which the smallest bound that is not 0 is below b.
+constexpr int kPassBits = 24;
 __global__ __launch_bounds__(256) void k_run_scale(int n_tiles, int tpb, const int32_t* __restrict__ tile_u0,
                                                    const int32_t* __restrict__ usrc, const int32_t* __restrict__ tile_d0,
                                                    const int32_t* __restrict__ dent, const float* __restrict__ bound,
                                                    float* __restrict__ run_scale, int64_t bound_vs) {
-  __shared__ float red[256];
+  __shared__ float red[256], red_mn[256];
   const int r = blockIdx.x, t = threadIdx.x, k0 = r * tpb, k1 = min(n_tiles, k0 + tpb);
   bound += blockIdx.y * bound_vs;  // density vector
-  float mx = 0.f;
-  for (int u = tile_u0[k0] + t; u < tile_u0[k0 + 1]; u += 256) mx = fmaxf(mx, bound[usrc[u] >> 9]);
+  float mx = 0.f, mn = 3.4e38f;
+  auto take = [&](float b) __attribute__((always_inline)) {
+    mx = fmaxf(mx, b);
+    if (b > 0.f) mn = fminf(mn, b);
+  };
+  for (int u = tile_u0[k0] + t; u < tile_u0[k0 + 1]; u += 256) take(bound[usrc[u] >> 9]);
   if (k0 + 1 < k1)
-    for (int d = tile_d0[k0 + 1] + t; d < tile_d0[k1]; d += 256) mx = fmaxf(mx, bound[dent[d] >> 9]);
+    for (int d = tile_d0[k0 + 1] + t; d < tile_d0[k1]; d += 256) take(bound[dent[d] >> 9]);
   red[t] = mx;
+  red_mn[t] = mn;
   __syncthreads();
   for (int o = 128; o > 0; o >>= 1) {
-    if (t < o) red[t] = fmaxf(red[t], red[t + o]);
+    if (t < o) {
+      red[t] = fmaxf(red[t], red[t + o]);
+      red_mn[t] = fminf(red_mn[t], red_mn[t + o]);
+    }
     __syncthreads();
   }
   if (t == 0) {
     const float b = red[0];
     float sc = 1.f;
+    int passes = 1;
     if (b > 0.f && b <= 3.4e38f) {
-      int e = 0;
+      int e = 0, em = 0;
       (void)frexpf(b, &e);  // b < 2^e
+      (void)frexpf(red_mn[0], &em);
       sc = ldexpf(1.f, min(100, max(-100, 14 - e)));
+      passes = 1 + (e - em) / kPassBits;
     }
-    run_scale[blockIdx.y * gridDim.x + r] = sc;
+    const int at = blockIdx.y * gridDim.x + r;
+    run_scale[at] = sc;
+    run_scale[gridDim.y * gridDim.x + at] = (float)passes;
   }
 }
 
@@ -2324,8 +2339,15 @@ __global__ __launch_bounds__(512, 2) void k_hadamard_run(int M_dim, int n_tiles,
 // divided by s tau_f (exact).  The factor 2^11 puts x1 where x0 was, so values down to 2^-28 of
 // their run's bound keep the 22 bits and smaller ones an error of 2^-50 of that bound.  With x1
 // unscaled that error was 2^-39, and two clusters far apart whose charges differ by 2^20 in size
-// (8 vectors, gradient, m = 10) came out 1.1e-5 off at the weak one, 2.2e-7 with it; the factor
-// costs nothing.  x1 t1 (2^-24 of a product on average) is a third more products: 60,000 points,
+// (8 vectors, gradient, m = 10) came out 1.1e-5 off at the weak one, 2.0e-7 with it; the factor
+// costs nothing.  A run whose sources' bounds differ by more than 2^24 is computed again (MULTI) in
+// several passes over its tiles, each with its own scale: a pass takes the values of the 24 bits below
+// its scale and leaves the smaller ones, and what the parts of its own did not hold, to the next
+// (split_rest).  Small values are left out and not merely repeated, because sums of products with
+// subnormal fp16 operands round at one size, however small they are.  At 2^32 the weak cluster was 4.4e-2
+// off without either, 2.3e-5 with the factor alone, and is 2.0e-7.  The second launch costs 2-4 us where
+// it finds no such run, which is the rule (of 48 trees and densities looked at, only log-normal densities
+// of e^(+-16) had some).  x1 t1 (2^-24 of a product on average) is a third more products: 60,000 points,
 // m = 8: 2.62e-7 -> 2.51e-7 from the FP64 sums; 32 vectors on 1M points 46.7 -> 47.9 ms, the 2M
 // adaptive tree 10.4 -> 10.6 ms.
 // One v_mfma_f32_16x16x32_f16 covers two parent offsets (k = 16 a + real index, a the offset
@@ -2347,7 +2369,15 @@ typedef _Float16 halfx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kSplitPool = 496;
 
-template <int UMAX, int POOL>
+// What a pass leaves of x for the next, times 2^kPassBits (at most 2^14, exact): all of a value below
+// kPassLeast, else what its two fp16 parts do not hold
+constexpr float kPassLeast = 16384.f / (1 << kPassBits);
+__device__ __forceinline__ float split_rest(float x) {
+  const float x0 = (float)(_Float16)x, x1 = (float)(_Float16)((x - x0) * kSplitLow);
+  return (fabsf(x) < kPassLeast ? x : (x - x0) - x1 * (1.f / kSplitLow)) * (float)(1 << kPassBits);
+}
+
+template <int UMAX, int POOL, bool MULTI>
 __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tiles, int tiles_per_block, int n_chunks,
                                                           const int32_t* __restrict__ tile_t0,
                                                           const int32_t* __restrict__ tile_u0, const int32_t* __restrict__ usrc,
@@ -2371,13 +2401,6 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
   __shared__ __align__(16) uint16_t ul[2][UT];
   __shared__ uint32_t m_g[4 * TMAX];  // the run's skip masks, delta starts and target starts
   __shared__ int32_t m_d[TMAX + 1], m_t[TMAX + 1];
-  // blocks b and b + 8 run on one XCD one after the other and take the two frequencies of one
-  // 128-byte line of X and Y (a frequency's 16 reals are 64 bytes) for the same run of tiles,
-  // so the second block's reads hit that XCD's L2
-  const int b = blockIdx.x, xcd = b & 7, local = b >> 3, lp = local >> 1;
-  const int f = ((lp / n_chunks) * 8 + xcd) * 2 + (local & 1), chunk = lp % n_chunks;
-  const int k0 = chunk * tiles_per_block, k1 = min(n_tiles, k0 + tiles_per_block);
-  if (f >= M_dim || k0 >= k1) return;  // whole block
   X += blockIdx.y * x_vs;  // density vector
   Y += blockIdx.y * y_vs;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63;
@@ -2386,155 +2409,188 @@ __global__ __launch_bounds__(256, 2) void k_hadamard_split(int M_dim, int n_tile
   const int lane_off = 4 * (kg & 1);        // word offset of its 8 reals within a part
   const int sr = tid & 3, su = tid >> 2;    // staging: reals 4sr..4sr+3 of entries su + EPP * i
 
-  // transfer-block parts of frequency f (scaled by tau_f): bq[j][p] holds, for lane
-  // (n = l%16, kg), part p of B_{2j + kg/2}[8 (kg%2) + i][n], i < 8
-  halfx8 bq[NPAIR][2];
-#pragma unroll
-  for (int j = 0; j < NPAIR; j++)
-#pragma unroll
-    for (int p = 0; p < 2; p++)
-      bq[j][p] = *reinterpret_cast<const halfx8*>(Vh + ((((int64_t)j * 2 + p) * M_dim + f) * 64 + l) * 8);
-  // the run's scale, and the factor that undoes both scales
-  const float xsc = run_scale[blockIdx.y * n_chunks + chunk], ysc = tinv[f] / xsc;
-  for (int e = tid; e < EST; e += 256) Xl[POOL * EST + e] = 0u;
-  const int nk = k1 - k0;
-  for (int i = tid; i < 4 * nk; i += 256) m_g[i] = gmask[4 * k0 + i];
-  for (int i = tid; i <= nk; i += 256) {
-    m_d[i] = tile_d0[k0 + i];
-    m_t[i] = tile_t0[k0 + i];
+  const float* n_pass = run_scale + (int64_t)(gridDim.y + blockIdx.y) * n_chunks;
+  if constexpr (MULTI) {  // the runs of more than one pass, if any
+    int any = 0;
+    for (int r = tid; r < n_chunks; r += 256) any |= n_pass[r] > 1.f;
+    if (!__syncthreads_or(any)) return;
   }
-
-  int src[NPASS];  // staged entries (source slot << 9 | pool slot)
-  int dst[NPASS];  // their pool slots, kept from the global loads to the LDS stores
-  floatx4 val[NPASS];
-  uint2 uw[UWP];
-  // start and length of tile k's delta list (length 0 past the run's end), from the run's
-  // copy in LDS, the length uniform over the block
-  auto d0_l = [&](int k) __attribute__((always_inline)) { return m_d[min(k, k1 - 1) - k0]; };
-  auto nd_l = [&](int k) __attribute__((always_inline)) {
-    const int kk = min(k, k1 - 1) - k0;
-    const int n = m_d[kk + 1] - m_d[kk];
-    return __builtin_amdgcn_readfirstlane(k < k1 ? n : 0);
-  };
-  auto load_src = [&](int i, const int32_t* list, int at, int n) __attribute__((always_inline)) {
-    src[i] = list[at + min(su + EPP * i, max(n - 1, 0))];
-  };
-  // X row of source slot s at frequency f: xf + s * xstride bytes (M_dim * 64 < 2^32: the
-  // host bounds M_dim)
-  const char* xf = reinterpret_cast<const char*>(X + (int64_t)f * RW + 4 * sr);
-  const uint32_t xstride = (uint32_t)M_dim * RW * sizeof(float);
-  auto load_val = [&](int i, int n) __attribute__((always_inline)) {
-    const int e = su + EPP * i < n ? src[i] : POOL + 1;  // a select on the input keeps it branch-free
-    dst[i] = e & 511;
-    val[i] = *reinterpret_cast<const floatx4*>(xf + (uint64_t)((uint32_t)e >> 9) * xstride);
-  };
-  auto load_uw = [&](int k) __attribute__((always_inline)) {
-    const uint2* ug = reinterpret_cast<const uint2*>(uidx + (int64_t)min(k, k1 - 1) * UT);
+  for (int64_t item = blockIdx.x; !MULTI || item < (int64_t)n_chunks * M_dim; item += gridDim.x) {
+    // blocks b and b + 8 run on one XCD one after the other and take the two frequencies of one
+    // 128-byte line of X and Y (a frequency's 16 reals are 64 bytes) for the same run of tiles,
+    // so the second block's reads hit that XCD's L2
+    const int b = blockIdx.x, xcd = b & 7, local = b >> 3, lp = local >> 1;
+    const int f = MULTI ? (int)(item % M_dim) : ((lp / n_chunks) * 8 + xcd) * 2 + (local & 1);
+    const int chunk = MULTI ? (int)(item / M_dim) : lp % n_chunks;
+    const int passes = MULTI ? (int)n_pass[chunk] : 1;
+    if (MULTI && passes == 1) continue;
+    if (f >= M_dim) return;  // whole block
+    const int k0 = chunk * tiles_per_block, k1 = min(n_tiles, k0 + tiles_per_block);
+    // transfer-block parts of frequency f (scaled by tau_f): bq[j][p] holds, for lane
+    // (n = l%16, kg), part p of B_{2j + kg/2}[8 (kg%2) + i][n], i < 8
+    halfx8 bq[NPAIR][2];
 #pragma unroll
-    for (int i = 0; i < UWP; i++) uw[i] = ug[tid + 256 * i];
-  };
-  // entry layout (words): part p at 8p, reals 2q, 2q+1 in word 8p + q
-  auto store_lds = [&](int buf, int n) __attribute__((always_inline)) {
+    for (int j = 0; j < NPAIR; j++)
 #pragma unroll
-    for (int i = 0; i < NPASS; i++) {
-      if (EPP * i >= n) break;  // uniform
-      halfx4 h0, h1;
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const float x = val[i][q] * xsc;  // exact (power of two)
-        h0[q] = (_Float16)x;
-        h1[q] = (_Float16)((x - (float)h0[q]) * kSplitLow);
-      }
-      uint32_t* d = &Xl[dst[i] * EST + 2 * sr];
-      *reinterpret_cast<halfx4*>(d) = h0;
-      *reinterpret_cast<halfx4*>(d + 8) = h1;
+      for (int p = 0; p < 2; p++)
+        bq[j][p] = *reinterpret_cast<const halfx8*>(Vh + ((((int64_t)j * 2 + p) * M_dim + f) * 64 + l) * 8);
+    // the run's scale, and the factor that undoes both scales
+    const float xsc = run_scale[blockIdx.y * n_chunks + chunk];
+    float ysc = tinv[f] / xsc;
+    int pass = 0;
+    for (int e = tid; e < EST; e += 256) Xl[POOL * EST + e] = 0u;
+    const int nk = k1 - k0;
+    for (int i = tid; i < 4 * nk; i += 256) m_g[i] = gmask[4 * k0 + i];
+    for (int i = tid; i <= nk; i += 256) {
+      m_d[i] = tile_d0[k0 + i];
+      m_t[i] = tile_t0[k0 + i];
     }
-#pragma unroll
-    for (int i = 0; i < UWP; i++) reinterpret_cast<uint2*>(ul[buf])[tid + 256 * i] = uw[i];
-  };
-  {
-    // the run's first tile: its whole union
-    const int u00 = tile_u0[k0], nu0 = __builtin_amdgcn_readfirstlane(tile_u0[k0 + 1] - u00);
-#pragma unroll
-    for (int i = 0; i < NPASS; i++) load_src(i, usrc, u00, nu0);
-#pragma unroll
-    for (int i = 0; i < NPASS; i++) load_val(i, nu0);
-    load_uw(k0);
-    __syncthreads();  // m_d
-    const int nd1 = nd_l(k0 + 1), d01 = d0_l(k0 + 1);
-#pragma unroll
-    for (int i = 0; i < NPASS; i++) load_src(i, dent, d01, nd1);
-    store_lds(0, nu0);
-    // the loop's first use of src[] then waits for nothing: without this wait the compiler
-    // carries the prologue's outstanding loads into the loop's wait counts, where they would
-    // make every tile wait for the previous tile's Y stores
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  }
-#pragma unroll
-  for (int j = 0; j < NPAIR; j++)
-#pragma unroll
-    for (int p = 0; p < 2; p++) asm volatile("" : "+v"(bq[j][p]));
-  __syncthreads();
 
-  for (int k = k0; k < k1; k++) {
-    const int buf = (k - k0) & 1;
-    const int nd1 = nd_l(k + 1), nd2 = nd_l(k + 2), d02 = d0_l(k + 2);
-    // offsets at which a target of the wave's group has a partner
-    const uint32_t wm = __builtin_amdgcn_readfirstlane(m_g[4 * (k - k0) + w]);
-    const uint32_t* xb = Xl;
-    // staged positions of the partners of target (w, row) at offsets 2j + pa, j < 13, read at
-    // once so that the operand reads of a pair wait for no other LDS read; the 16 rows of a
-    // read are consecutive 16-byte words (one per LDS bank group)
-    u32x4 pw[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) pw[h] = *reinterpret_cast<const u32x4*>(&ul[buf][(((w * 2 + h) * 2 + pa) * 16 + row) * 8]);
-    auto pidx = [&](int j) __attribute__((always_inline)) { return (int)((pw[j >> 3][(j >> 1) & 3] >> (16 * (j & 1))) & 0xFFFFu); };
-    auto aop = [&](int pos, int p) __attribute__((always_inline)) {
-      return *reinterpret_cast<const halfx8*>(&xb[pos * EST + 8 * p + lane_off]);
+    int src[NPASS];  // staged entries (source slot << 9 | pool slot)
+    int dst[NPASS];  // their pool slots, kept from the global loads to the LDS stores
+    floatx4 val[NPASS];
+    uint2 uw[UWP];
+    // start and length of tile k's delta list (length 0 past the run's end), from the run's
+    // copy in LDS, the length uniform over the block
+    auto d0_l = [&](int k) __attribute__((always_inline)) { return m_d[min(k, k1 - 1) - k0]; };
+    auto nd_l = [&](int k) __attribute__((always_inline)) {
+      const int kk = min(k, k1 - 1) - k0;
+      const int n = m_d[kk + 1] - m_d[kk];
+      return __builtin_amdgcn_readfirstlane(k < k1 ? n : 0);
     };
-    floatx4 acc0[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // even and odd pairs
-    floatx4 acc1 = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
-    halfx8 an[2];
-    {
-      const int p0 = pidx(0);
+    auto load_src = [&](int i, const int32_t* list, int at, int n) __attribute__((always_inline)) {
+      src[i] = list[at + min(su + EPP * i, max(n - 1, 0))];
+    };
+    // X row of source slot s at frequency f: xf + s * xstride bytes (M_dim * 64 < 2^32: the
+    // host bounds M_dim)
+    const char* xf = reinterpret_cast<const char*>(X + (int64_t)f * RW + 4 * sr);
+    const uint32_t xstride = (uint32_t)M_dim * RW * sizeof(float);
+    auto load_val = [&](int i, int n) __attribute__((always_inline)) {
+      const int e = su + EPP * i < n ? src[i] : POOL + 1;  // a select on the input keeps it branch-free
+      dst[i] = e & 511;
+      val[i] = *reinterpret_cast<const floatx4*>(xf + (uint64_t)((uint32_t)e >> 9) * xstride);
+    };
+    auto load_uw = [&](int k) __attribute__((always_inline)) {
+      const uint2* ug = reinterpret_cast<const uint2*>(uidx + (int64_t)min(k, k1 - 1) * UT);
 #pragma unroll
-      for (int p = 0; p < 2; p++) an[p] = aop(p0, p);
+      for (int i = 0; i < UWP; i++) uw[i] = ug[tid + 256 * i];
+    };
+    // entry layout (words): part p at 8p, reals 2q, 2q+1 in word 8p + q
+    auto store_lds = [&](int buf, int n) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < NPASS; i++) {
+        if (EPP * i >= n) break;  // uniform
+        halfx4 h0, h1;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          float x = val[i][q] * xsc;  // exact (power of two)
+          if constexpr (MULTI) {
+            for (int p = 0; p < pass; p++) x = split_rest(x);
+            if (pass + 1 < passes && fabsf(x) < kPassLeast) x = 0.f;
+          }
+          h0[q] = (_Float16)x;
+          h1[q] = (_Float16)((x - (float)h0[q]) * kSplitLow);
+        }
+        uint32_t* d = &Xl[dst[i] * EST + 2 * sr];
+        *reinterpret_cast<halfx4*>(d) = h0;
+        *reinterpret_cast<halfx4*>(d + 8) = h1;
+      }
+#pragma unroll
+      for (int i = 0; i < UWP; i++) reinterpret_cast<uint2*>(ul[buf])[tid + 256 * i] = uw[i];
+    };
+    for (;;) {
+      {
+        // the run's first tile: its whole union
+        const int u00 = tile_u0[k0], nu0 = __builtin_amdgcn_readfirstlane(tile_u0[k0 + 1] - u00);
+#pragma unroll
+        for (int i = 0; i < NPASS; i++) load_src(i, usrc, u00, nu0);
+#pragma unroll
+        for (int i = 0; i < NPASS; i++) load_val(i, nu0);
+        load_uw(k0);
+        __syncthreads();  // m_d
+        const int nd1 = nd_l(k0 + 1), d01 = d0_l(k0 + 1);
+#pragma unroll
+        for (int i = 0; i < NPASS; i++) load_src(i, dent, d01, nd1);
+        store_lds(0, nu0);
+        // the loop's first use of src[] then waits for nothing: without this wait the compiler
+        // carries the prologue's outstanding loads into the loop's wait counts, where they would
+        // make every tile wait for the previous tile's Y stores
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+      }
+#pragma unroll
+      for (int j = 0; j < NPAIR; j++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) asm volatile("" : "+v"(bq[j][p]));
+      __syncthreads();
+
+      for (int k = k0; k < k1; k++) {
+        const int buf = (k - k0) & 1;
+        const int nd1 = nd_l(k + 1), nd2 = nd_l(k + 2), d02 = d0_l(k + 2);
+        // offsets at which a target of the wave's group has a partner
+        const uint32_t wm = __builtin_amdgcn_readfirstlane(m_g[4 * (k - k0) + w]);
+        const uint32_t* xb = Xl;
+        // staged positions of the partners of target (w, row) at offsets 2j + pa, j < 13, read at
+        // once so that the operand reads of a pair wait for no other LDS read; the 16 rows of a
+        // read are consecutive 16-byte words (one per LDS bank group)
+        u32x4 pw[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) pw[h] = *reinterpret_cast<const u32x4*>(&ul[buf][(((w * 2 + h) * 2 + pa) * 16 + row) * 8]);
+        auto pidx = [&](int j) __attribute__((always_inline)) { return (int)((pw[j >> 3][(j >> 1) & 3] >> (16 * (j & 1))) & 0xFFFFu); };
+        auto aop = [&](int pos, int p) __attribute__((always_inline)) {
+          return *reinterpret_cast<const halfx8*>(&xb[pos * EST + 8 * p + lane_off]);
+        };
+        floatx4 acc0[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // even and odd pairs
+        floatx4 acc1 = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
+        halfx8 an[2];
+        {
+          const int p0 = pidx(0);
+#pragma unroll
+          for (int p = 0; p < 2; p++) an[p] = aop(p0, p);
+        }
+#pragma unroll
+        for (int j = 0; j < NPAIR; j++) {
+          halfx8 ac[2];
+#pragma unroll
+          for (int p = 0; p < 2; p++) ac[p] = an[p];
+          if (j + 1 < NPAIR) {
+            const int pn = pidx(j + 1);
+#pragma unroll
+            for (int p = 0; p < 2; p++) an[p] = aop(pn, p);
+          }
+          if (j < NPASS && EPP * j < nd1) {
+            load_val(j, nd1);  // tile k+1, from the entries read during tile k-1
+          }
+          if (j < NPASS && EPP * j < nd2) {
+            load_src(j, dent, d02, nd2);  // tile k+2
+          }
+          if (j == NPASS) load_uw(k + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          if ((wm >> (2 * j)) & 3u) {
+            acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[1], bq[j][0], acc1, 0, 0, 0);
+            acc0[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][0], acc0[j & 1], 0, 0, 0);
+            acc2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[1], bq[j][1], acc2, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][1], acc1, 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        store_lds(buf ^ 1, nd1);  // tile k+1 (slots that tile k does not read; the other table buffer is free since the last barrier)
+        {
+          const int t0 = m_t[k - k0], nt = m_t[k - k0 + 1] - t0;
+          const floatx4 sum = ((acc0[0] + acc0[1]) + (acc1 + acc2 * (1.f / kSplitLow)) * (1.f / kSplitLow)) * ysc;
+          float* yr = Y + ((int64_t)(t0 + 16 * w + 4 * kg) * M_dim + f) * RW + row;
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            if (16 * w + 4 * kg + r < nt) {
+              float* y = yr + (int64_t)r * M_dim * RW;
+              *y = MULTI && pass > 0 ? *y + sum[r] : sum[r];
+            }
+        }
+        __syncthreads();
+      }
+      if (!MULTI || ++pass == passes) break;
+      ysc *= 1.f / (1 << kPassBits);
     }
-#pragma unroll
-    for (int j = 0; j < NPAIR; j++) {
-      halfx8 ac[2];
-#pragma unroll
-      for (int p = 0; p < 2; p++) ac[p] = an[p];
-      if (j + 1 < NPAIR) {
-        const int pn = pidx(j + 1);
-#pragma unroll
-        for (int p = 0; p < 2; p++) an[p] = aop(pn, p);
-      }
-      if (j < NPASS && EPP * j < nd1) {
-        load_val(j, nd1);  // tile k+1, from the entries read during tile k-1
-      }
-      if (j < NPASS && EPP * j < nd2) {
-        load_src(j, dent, d02, nd2);  // tile k+2
-      }
-      if (j == NPASS) load_uw(k + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      if ((wm >> (2 * j)) & 3u) {
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[1], bq[j][0], acc1, 0, 0, 0);
-        acc0[j & 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][0], acc0[j & 1], 0, 0, 0);
-        acc2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[1], bq[j][1], acc2, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(ac[0], bq[j][1], acc1, 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    store_lds(buf ^ 1, nd1);  // tile k+1 (slots that tile k does not read; the other table buffer is free since the last barrier)
-    {
-      const int t0 = m_t[k - k0], nt = m_t[k - k0 + 1] - t0;
-      const floatx4 sum = ((acc0[0] + acc0[1]) + (acc1 + acc2 * (1.f / kSplitLow)) * (1.f / kSplitLow)) * ysc;
-      float* yr = Y + ((int64_t)(t0 + 16 * w + 4 * kg) * M_dim + f) * RW + row;
-#pragma unroll
-      for (int r = 0; r < 4; r++)
-        if (16 * w + 4 * kg + r < nt) yr[(int64_t)r * M_dim * RW] = sum[r];
-    }
+    if constexpr (!MULTI) return;
     __syncthreads();
   }
 }
@@ -3095,13 +3151,16 @@ void DeviceKernels<Real>::hadamard_tiled(hipStream_t s, int n_tiles, int M_dim, 
       const int TPB = std::min(64, std::max(1, tiles_per_block));
       const int n_chunks = (n_tiles + TPB - 1) / TPB;
       const int64_t nbs = (int64_t)n_chunks * ((M_dim + 15) / 16) * 16;
-      if (nbs >= (1ll << 31) || (int64_t)n_chunks * nv > hp->run_scale_cap) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
+      if (nbs >= (1ll << 31) || (int64_t)2 * n_chunks * nv > hp->run_scale_cap) throw_device_error(hipErrorInvalidValue, __FILE__, __LINE__);
       hipLaunchKernelGGL(k_run_scale, dim3((unsigned)n_chunks, nv), dim3(256), 0, s, n_tiles, TPB, tile_u0, usrc, tile_d0, dent,
                          hp->bound, hp->run_scale, hp->bound_vs);
       HIP_LAUNCH_CHECK();
-      hipLaunchKernelGGL((k_hadamard_split<250, kSplitPool>), dim3((unsigned)nbs, nv), dim3(256), 0, s, M_dim, n_tiles, TPB,
+      hipLaunchKernelGGL((k_hadamard_split<250, kSplitPool, false>), dim3((unsigned)nbs, nv), dim3(256), 0, s, M_dim, n_tiles, TPB,
                          n_chunks, tile_t0, tile_u0, usrc, tile_d0, dent, uidx, gmask, hp->Vh, hp->tinv, hp->run_scale, X, Y, x_vs,
                          y_vs);
+      HIP_LAUNCH_CHECK();
+      hipLaunchKernelGGL((k_hadamard_split<250, kSplitPool, true>), dim3(512, nv), dim3(256), 0, s, M_dim, n_tiles, TPB, n_chunks,
+                         tile_t0, tile_u0, usrc, tile_d0, dent, uidx, gmask, hp->Vh, hp->tinv, hp->run_scale, X, Y, x_vs, y_vs);
     } else {
       const int n_fgt = (M_dim + 1) / 2;
       const int64_t nbt = (int64_t)n_tiles * ((n_fgt + 7) / 8) * 8;

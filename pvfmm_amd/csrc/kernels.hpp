@@ -15,7 +15,7 @@ struct HadamardParts {
   const uint16_t* Vh = nullptr;  // transfer blocks as two fp16 parts, scaled by tau_f
   const float* tinv = nullptr;   // 1 / tau_f per frequency (powers of two)
   const float* bound = nullptr;  // spectrum bound per source slot and component (fft_up's `bound`)
-  float* run_scale = nullptr;    // scratch: one scale per run of tiles (scalar kernels)
+  float* run_scale = nullptr;    // scratch: scale and passes of each run of tiles (scalar kernels)
   int run_scale_cap = 0;         // its length
   int64_t bound_vs = 0;          // stride of bound per density vector
 };
@@ -148,7 +148,7 @@ struct DeviceKernels {
   // [part p][lane 64][8], lane l holding part p of B_{2j + a}[8 b + i][16 nb + l % 16] with
   // q = 4c + l/16, a = q / 6, b = q % 6; hp->tinv 1 / tau_f; hp->bound the spectrum bounds of
   // X's slots and components (fft_up); hp->run_scale (scalar kernels) room for
-  // ceil(n_tiles / tiles_per_block) scales per vector.
+  // 2 ceil(n_tiles / tiles_per_block) values per vector (their scales and passes).
   // They stage into an LDS pool of hadamard_pool_max() entries kept across a block's run of
   // tiles: usrc entries are (source slot << 9 | pool slot), uidx holds pool slots (the pool
   // size for none), and tile k's partners new since tile k-1 are dent[tile_d0[k] ..

@@ -1,12 +1,13 @@
-"""The mixed evaluator on one and on 8 density vectors whose charges differ by 2^16 and 2^20 in size
+"""The mixed evaluator on one and on 8 density vectors whose charges differ by 2^16 to 2^32 in size
 within one run of V-list tiles, against the FP64 evaluator at the FP32 pseudo-inverse cutoff on the
 same tree (the same operators, so that only the rounding differs).
 
 Two clusters of 6,000 points lie far apart; the charges of one are strong, in pairs of opposite sign
 0.4% of the cluster apart, so that at the other cluster its field is below the rounding of the weak
-charges' own.  FP32 spectra keep their 24 bits whatever their size (2.5e-7 and 3.0e-7 at the weak
+charges' own.  FP32 spectra keep their 24 bits whatever their size (2.5e-7 to 3.0e-7 at the weak
 cluster when each was multiplied with its own exponent); fp16 parts of a common scale keep them only
-if the second part has a scale of its own.  The bar is three times those errors."""
+if the second part has a scale of its own, and beyond 2^24 only if weak and strong spectra are
+multiplied apart.  The bar is three times those errors."""
 import numpy as np
 import pytest
 
@@ -19,6 +20,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("kernel,size,ratio,tol", [
     ("laplace_grad", 2.0**-9, 2.0**20, 7.5e-7),
     ("laplace_grad", 2.0**-12, 2.0**16, 7.5e-7),
+    ("laplace_grad", 2.0**-12, 2.0**32, 8e-7),
     ("laplace_poten", 2.0**-12, 2.0**16, 9e-7),
 ])
 def test_weak_cluster_far_from_a_strong_one(gpu, kernel, size, ratio, tol, nv):
